@@ -258,16 +258,6 @@ inline int grid_for(int64_t work, int num_cus) {
   return (int)std::max<int64_t>(1, std::min(g, cap));
 }
 
-template <typename T>
-constexpr int vec_of() {
-  return 16 / (int)sizeof(T);
-}
-
-bool ptr_aligned(const void *p, int64_t off_elems, int elem) {
-  return ((reinterpret_cast<uintptr_t>(p) + (uintptr_t)(off_elems * elem)) &
-          15u) == 0;
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -277,7 +267,6 @@ template <Elem E, typename OutT>
 hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
                          double beta, void *C, int64_t ldc, int64_t cOff,
                          int64_t strideC, void *const *Cptrs, int64_t batch) {
-  using T = typename ElemT<E>::T;
   using Acc = typename ElemT<E>::Acc;
   if (c.M == 0 || c.N == 0 || batch == 0) return HCBLAS_STATUS_SUCCESS;
   if (C == nullptr && Cptrs == nullptr) return HCBLAS_STATUS_INVALID_VALUE;
@@ -318,21 +307,7 @@ hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
   p.cOff = cOff;
   p.alpha = alpha;
   p.beta = beta;
-  // 16-byte global loads need every matrix base, offset and leading dimension
-  // (and batch stride) aligned to one vector. For pointer arrays the host
-  // checks offsets and leading dimensions only; the kernel checks each
-  // problem's bases and takes the element-wise loaders for a misaligned one.
-  constexpr int V = vec_of<T>();
-  // An r-contiguous operand also needs its row count to be a whole number
-  // of vectors, so that a vector is wholly inside or outside the rows.
-  bool vload = c.lda % V == 0 && c.ldb % V == 0 && c.aOff % V == 0 &&
-               c.bOff % V == 0 && (c.a_k || c.M % V == 0) &&
-               (c.b_k || c.N % V == 0);
-  if (!c.Aptrs) vload = vload && ptr_aligned(c.A, c.aOff, sizeof(T)) &&
-                        (batch == 1 || c.strideA % V == 0);
-  if (!c.Bptrs) vload = vload && ptr_aligned(c.B, c.bOff, sizeof(T)) &&
-                        (batch == 1 || c.strideB % V == 0);
-  if (batch == 1 && vload && !c.Aptrs && !c.Bptrs && !Cptrs) {
+  if (batch == 1 && !c.Aptrs && !c.Bptrs && !Cptrs) {
     int ks = 0;
     const int S = splitk_count(c.M, c.N, c.K, h->num_cus,
                                E == Elem::F64 ? 16 : E == Elem::F32 ? 32 : 64,
@@ -346,8 +321,7 @@ hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
                                          static_cast<Acc *>(h->kpart_ws.ptr));
     }
   }
-  return launch_gemm<E, OutT>(h->stream, h->num_cus, p, c.a_k, c.b_k, vload,
-                              batch);
+  return launch_gemm<E, OutT>(h->stream, h->num_cus, p, c.a_k, c.b_k, batch);
 }
 
 // ---------------------------------------------------------------------------

@@ -36,8 +36,7 @@ namespace {
 
 struct ProbDev {
   int dtype;  // 0: fp32, 1: fp16
-  int flags;  // bit 0: A' k-contiguous, bit 1: B' k-contiguous, bit 2: C
-              // allows 16-byte vector accesses
+  int flags;  // bit 0: A' k-contiguous, bit 1: B' k-contiguous
   int M, N, K;
   int tiles_n;
   float alpha, beta;
@@ -64,36 +63,33 @@ struct GroupCfg {
 
 // One tile: the plain kernels' main loop (same K step, so the sums are
 // bit-identical to per-problem launches), then the LDS-staged epilogue.
-template <Elem E, typename OutT, int TM, bool VL, bool A_K, bool B_K>
+template <Elem E, typename OutT, int TM, bool NARROW, bool A_K, bool B_K>
 __device__ __forceinline__ void tile_body(const ProbDev &p, int m0, int n0,
-                                          char *lds) {
+                                          int tid, char *lds) {
   using T = typename ElemT<E>::T;
   constexpr int BK = E == Elem::F32 ? kF32BK : kF16BK;
-  using WT = WaveTile<E, TM, TM, 2, 2, 16>;
-  typename WT::AccV acc[WT::FM][WT::FN];
-  gemm_mainloop<E, A_K, B_K, TM, TM, BK, 2, 2, VL, VL, 16>(
+  gemm_tile<E, OutT, A_K, B_K, TM, TM, BK, 2, 2, 16, GroupCfg<TM>::LDS,
+            NARROW>(
       static_cast<const T *>(p.A), p.lda, static_cast<const T *>(p.B), p.ldb,
-      p.M, p.N, p.K, m0, n0, lds, acc);
-  store_tile_lds<E, OutT, TM, TM, 2, 2, 16, GroupCfg<TM>::LDS>(
-      acc, static_cast<OutT *>(p.C), p.ldc, p.M, p.N, m0, n0, p.alpha,
-      p.beta, lds, (p.flags & 4) != 0);
+      static_cast<OutT *>(p.C), p.ldc, p.M, p.N, p.K, p.alpha, p.beta, m0, n0,
+      tid, lds);
 }
 
-template <Elem E, typename OutT, int TM, bool VL>
+template <Elem E, typename OutT, int TM, bool NARROW>
 __device__ __forceinline__ void run_tile(const ProbDev &p, int m0, int n0,
-                                         char *lds) {
+                                         int tid, char *lds) {
   switch (p.flags & 3) {
     case 0:
-      tile_body<E, OutT, TM, VL, false, false>(p, m0, n0, lds);
+      tile_body<E, OutT, TM, NARROW, false, false>(p, m0, n0, tid, lds);
       break;
     case 1:
-      tile_body<E, OutT, TM, VL, true, false>(p, m0, n0, lds);
+      tile_body<E, OutT, TM, NARROW, true, false>(p, m0, n0, tid, lds);
       break;
     case 2:
-      tile_body<E, OutT, TM, VL, false, true>(p, m0, n0, lds);
+      tile_body<E, OutT, TM, NARROW, false, true>(p, m0, n0, tid, lds);
       break;
     default:
-      tile_body<E, OutT, TM, VL, true, true>(p, m0, n0, lds);
+      tile_body<E, OutT, TM, NARROW, true, true>(p, m0, n0, tid, lds);
       break;
   }
 }
@@ -105,7 +101,7 @@ __device__ __forceinline__ void run_tile(const ProbDev &p, int m0, int n0,
 // workgroups; the last one resets both counters.
 // OCC: workgroups per CU the launch is sized for (the register budget
 // follows from it: 4 waves per workgroup, one per SIMD).
-template <int TM, bool VL, int OCC>
+template <int TM, bool NARROW, int OCC>
 __global__ __launch_bounds__(256, OCC) void grouped_gemm_kernel(
     const ProbDev *__restrict__ probs, const int2 *__restrict__ work,
     int total, unsigned int *counters, int dynamic) {
@@ -128,10 +124,15 @@ __global__ __launch_bounds__(256, OCC) void grouped_gemm_kernel(
     const ProbDev p = probs[__builtin_amdgcn_readfirstlane(it.x)];
     const int t = __builtin_amdgcn_readfirstlane(it.y);
     const int tm = t / p.tiles_n, tn = t - tm * p.tiles_n;
+    // The thread id is made opaque for each tile: the eight tile bodies' lane
+    // constants would otherwise all be computed once and live across the
+    // loop, in scratch memory (36 VGPRs spilled at four workgroups per CU).
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
     if (p.dtype == 0)
-      run_tile<Elem::F32, float, TM, VL>(p, tm * TM, tn * TM, lds);
+      run_tile<Elem::F32, float, TM, NARROW>(p, tm * TM, tn * TM, tid, lds);
     else
-      run_tile<Elem::F16, uint16_t, TM, VL>(p, tm * TM, tn * TM, lds);
+      run_tile<Elem::F16, uint16_t, TM, NARROW>(p, tm * TM, tn * TM, tid, lds);
   }
   if (threadIdx.x == 0) {
     const unsigned int t = __hip_atomic_fetch_add(
@@ -158,7 +159,7 @@ using namespace hcb;
 struct hcblasGroupedPlan {
   int device = 0;
   int count = 0;
-  bool vload = true;
+  bool narrow = false;  // an operand is shorter than one 16-byte vector
   std::vector<ProbDev> probs;  // host copy (canonical)
   ProbDev *d_probs = nullptr;
   int2 *d_work = nullptr;
@@ -183,38 +184,30 @@ void free_graph(hcblasGroupedPlan *p) {
   p->graph = nullptr;
 }
 
-template <int TM, bool VL>
+template <int TM, bool NARROW>
 void launch_occ(hcblasGroupedPlan *p, hipStream_t s) {
   dim3 g(p->grid);
   switch (kOccupancies[p->occ]) {
     case 2:
-      grouped_gemm_kernel<TM, VL, 2><<<g, 256, 0, s>>>(
+      grouped_gemm_kernel<TM, NARROW, 2><<<g, 256, 0, s>>>(
           p->d_probs, p->d_work, p->total, p->d_counters, p->sched == 0);
       break;
     case 3:
-      grouped_gemm_kernel<TM, VL, 3><<<g, 256, 0, s>>>(
+      grouped_gemm_kernel<TM, NARROW, 3><<<g, 256, 0, s>>>(
           p->d_probs, p->d_work, p->total, p->d_counters, p->sched == 0);
       break;
     default:
-      grouped_gemm_kernel<TM, VL, 4><<<g, 256, 0, s>>>(
+      grouped_gemm_kernel<TM, NARROW, 4><<<g, 256, 0, s>>>(
           p->d_probs, p->d_work, p->total, p->d_counters, p->sched == 0);
       break;
   }
 }
 
 void launch_grouped(hcblasGroupedPlan *p, hipStream_t s) {
-  const int tm = kTileShapes[p->shape];
-  if (tm == 64) {
-    if (p->vload)
-      launch_occ<64, true>(p, s);
-    else
-      launch_occ<64, false>(p, s);
-  } else {
-    if (p->vload)
-      launch_occ<32, true>(p, s);
-    else
-      launch_occ<32, false>(p, s);
-  }
+  if (kTileShapes[p->shape] == 64)
+    p->narrow ? launch_occ<64, true>(p, s) : launch_occ<64, false>(p, s);
+  else
+    p->narrow ? launch_occ<32, true>(p, s) : launch_occ<32, false>(p, s);
 }
 
 // Builds the work list for (shape, order, occupancy), uploads it and
@@ -307,7 +300,6 @@ hcblasStatus_t hcblasGroupedPlanCreate(hcblasHandle_t handle,
   p->device = handle->device;
   p->count = count;
   p->probs.resize(count);
-  bool vload = true;
   for (int i = 0; i < count; ++i) {
     const hcblasGemmProblem &u = problems[i];
     ProbDev &q = p->probs[i];
@@ -351,20 +343,9 @@ hcblasStatus_t hcblasGroupedPlanCreate(hcblasHandle_t handle,
     // leaves acc = 0, so C = beta*C).
     if (q.alpha == 0.f) q.K = 0;
     const int vec = q.dtype == 0 ? 4 : 8;
-    const size_t es = q.dtype == 0 ? 4 : 2;
-    auto al = [&](const void *ptr) {
-      return ptr == nullptr ||
-             (reinterpret_cast<uintptr_t>(ptr) % 16 == 0);
-    };
-    // bit 2: 16-byte vector accesses of C in the epilogue
-    if (q.ldc % vec == 0 && al(q.C)) q.flags |= 4;
-    (void)es;
-    if (q.lda % vec || q.ldb % vec || !al(q.A) || !al(q.B)) vload = false;
-    // r-contiguous operands: whole vectors of rows (see TileLoader)
-    if ((!(q.flags & 1) && q.M % vec) || (!(q.flags & 2) && q.N % vec))
-      vload = false;
+    if (((q.flags & 1) ? q.K : q.M) < vec || ((q.flags & 2) ? q.K : q.N) < vec)
+      p->narrow = true;
   }
-  p->vload = vload;
   if (hipMalloc(&p->d_probs, sizeof(ProbDev) * std::max(1, count)) !=
           hipSuccess ||
       hipMalloc(&p->d_counters, 2 * sizeof(unsigned int)) != hipSuccess ||

@@ -102,6 +102,22 @@ typedef int intx16 __attribute__((ext_vector_type(16)));
 // struct defeats scalar replacement of the staging arrays).
 typedef unsigned int vec4u __attribute__((ext_vector_type(4)));
 typedef unsigned int vec2u __attribute__((ext_vector_type(2)));
+// The same 16 bytes of global memory at an address that is only a multiple of
+// the element size: gfx950 serves a global_load / store_dwordx4 at any
+// address, so one kernel takes every base, offset and leading dimension. A
+// wave's 1 KiB run off a cache line boundary touches one more line.
+template <int ESIZE>
+struct GlobalVecOf;
+template <>
+struct GlobalVecOf<1> { typedef vec4u type __attribute__((aligned(1))); };
+template <>
+struct GlobalVecOf<2> { typedef vec4u type __attribute__((aligned(2))); };
+template <>
+struct GlobalVecOf<4> { typedef vec4u type __attribute__((aligned(4))); };
+template <>
+struct GlobalVecOf<8> { typedef vec4u type __attribute__((aligned(8))); };
+template <typename T>
+using GlobalVec = GlobalVecOf<(int)sizeof(T)>;
 
 template <Elem E, int MI>
 struct AccOf;
@@ -179,11 +195,24 @@ __device__ __forceinline__ void mfma_step(const vec4u &a, const vec4u &b,
 // Global -> register -> LDS tile loader for one operand.
 // ROWS = tile extent in m (or n); the LDS tile is [ROWS][BK] k-contiguous.
 // KCONT: the global operand is k-contiguous (element (r,k) at P[k + r*ld]).
-// VLOAD: 16-byte global loads are legal (base, ld aligned to the vector).
+//
+// Every load is 16 bytes wide, whatever the operand's alignment, without
+// branches and inside the operand:
+//   - k-contiguous: a vector that reaches past K is read from k = K - VEC on
+//     and moved down to its place (zeros behind it) before it goes to LDS;
+//   - r-contiguous: of a row count R that is not a whole number of vectors,
+//     the last vector is read from row R - VEC on and stays so: the tile rows
+//     of that vector hold the rows `edge_shift` further down, which the
+//     epilogue undoes (no other tile row is affected). Steps past K read the
+//     last k and are zeroed before they go to LDS.
+// Only an operand shorter than one vector is read by elements (load_narrow).
+// Element-wise loads of unaligned operands cost 1.1-3 times the whole GEMM
+// (529 x 192 x 1152 SGEMM NN 51.6 us, 2051 x 1777 x 1533 DGEMM NT 226 us).
 // ---------------------------------------------------------------------------
-template <typename T, int ROWS, int BK, bool KCONT, bool VLOAD, int NTH = 256>
+template <typename T, int ROWS, int BK, bool KCONT, int NTH = 256>
 struct TileLoader {
   static constexpr int VEC = 16 / (int)sizeof(T);
+  using GV = typename GlobalVec<T>::type;
   static constexpr int NV = ROWS * BK / VEC;  // 16-byte vectors per tile
   static constexpr int PER_THREAD = (NV + NTH - 1) / NTH;
   static constexpr int ROWB = BK * (int)sizeof(T) + 16;  // LDS row stride
@@ -222,7 +251,10 @@ struct TileLoader {
                                  NV == 2 * NTH && ROWS / 4 == NTH / 16;
   static constexpr bool TRANS2H = !KCONT && VEC == 8 && BK == 64 &&
                                   NV == 2 * NTH && (ROWS / 8) * 32 == NTH;
+  const int tid;  // thread of the workgroup
   vec4u reg[PER_THREAD];
+
+  __device__ __forceinline__ explicit TileLoader(int t) : tid(t) {}
 
   // (r, k) of vector v of the tile (r, k are element indices).
   __device__ __forceinline__ static void vec_pos(int v, int &r, int &k) {
@@ -258,82 +290,110 @@ struct TileLoader {
     }
   }
 
-  __device__ __forceinline__ void load(const T *__restrict__ P, int64_t ld,
-                                       int r0, int k0, int R, int K) {
+  // The contiguous dimension holds at least one vector.
+  __device__ __forceinline__ static bool wide(int R, int K) {
+    return (KCONT ? K : R) >= VEC;
+  }
+
+  // Tile rows of the last vector lie this far above the operand's rows.
+  __device__ __forceinline__ static int edge_shift(int R) {
+    return !KCONT && R >= VEC && R % VEC != 0 ? VEC - R % VEC : 0;
+  }
+
+  // A wide operand's step at k0: FULL if it lies entirely inside [0, K),
+  // else mask() has to follow before the LDS store. Rows past R read row r0
+  // (k-contiguous) or the last vector; they only feed outputs that are never
+  // stored. The loaded registers are first consumed by the LDS store after
+  // the MFMAs: the global latency stays hidden behind them.
+  template <bool FULL>
+  __device__ __forceinline__ void load_wide(const T *__restrict__ P,
+                                            int64_t ld, int r0, int k0, int R,
+                                            int K) {
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i) {
-      const int v = threadIdx.x + i * NTH;
+      const int v = tid + i * NTH;
       if (NV % NTH != 0 && v >= NV) continue;
       int r, k;
       vec_pos(v, r, k);
-      const int gr = r0 + r, gk = k0 + k;
-      if (KCONT) {
-        const T *src = P + (int64_t)gr * ld + gk;
-        if (VLOAD && gr < R && gk + VEC <= K) {
-          reg[i] = *reinterpret_cast<const vec4u *>(src);
-        } else {
-          T t[VEC];
+      const int last = KCONT ? K - VEC : K - 1;
+      const int gr = r0 + r, gk = FULL || k0 + k < last ? k0 + k : last;
+      const T *src = KCONT ? P + (int64_t)(gr < R ? gr : r0) * ld + gk
+                           : P + (int64_t)gk * ld +
+                                 (gr < R - VEC ? gr : R - VEC);
+      reg[i] = *reinterpret_cast<const GV *>(src);
+    }
+  }
+
+  // Zeros for k >= K in the registers of the (partial) step at k0.
+  __device__ __forceinline__ void mask(int k0, int K) {
+    // K - VEC of a moved vector lies this far below its place (0: none).
+    const int shift = KCONT && K % VEC ? VEC - K % VEC : 0;
 #pragma unroll
-          for (int e = 0; e < VEC; ++e)
-            t[e] = (gr < R && gk + e < K) ? src[e] : T(0);
-          __builtin_memcpy(&reg[i], t, 16);
-        }
-      } else {
-        const T *src = P + (int64_t)gk * ld + gr;
-        if (VLOAD && gk < K && gr + VEC <= R) {
-          reg[i] = *reinterpret_cast<const vec4u *>(src);
-        } else {
-          T t[VEC];
+    for (int i = 0; i < PER_THREAD; ++i) {
+      int r, k;
+      vec_pos(tid + i * NTH, r, k);
+      const int n = K - (k0 + k);  // k values of this vector inside K
+      if (KCONT && n > 0 && n < VEC) reg[i] = down(reg[i], shift);
+      if (n <= 0) reg[i] = vec4u{};
+    }
+  }
+
+  // The vector moved down by n elements (0 < n < VEC), zeros behind it.
+  __device__ __forceinline__ static vec4u down(vec4u w, int n) {
+    const int b = n * (int)sizeof(T);
+    if (b & 8) w = vec4u{w.z, w.w, 0, 0};
+    if (b & 4) w = vec4u{w.y, w.z, w.w, 0};
+    if (sizeof(T) < 4 && (b & 3)) {
+      const int sh = 8 * (b & 3);
+      w = vec4u{__builtin_amdgcn_alignbit(w.y, w.x, sh),
+                __builtin_amdgcn_alignbit(w.z, w.y, sh),
+                __builtin_amdgcn_alignbit(w.w, w.z, sh), w.w >> sh};
+    }
+    return w;
+  }
+
+  // An operand shorter than one vector, element by element.
+  __device__ __forceinline__ void load_narrow(const T *__restrict__ P,
+                                              int64_t ld, int r0, int k0,
+                                              int R, int K) {
 #pragma unroll
-          for (int e = 0; e < VEC; ++e)
-            t[e] = (gk < K && gr + e < R) ? src[e] : T(0);
-          __builtin_memcpy(&reg[i], t, 16);
-        }
+    for (int i = 0; i < PER_THREAD; ++i) {
+      const int v = tid + i * NTH;
+      if (NV % NTH != 0 && v >= NV) continue;
+      int r, k;
+      vec_pos(v, r, k);
+      T t[VEC];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const int gr = r0 + r + (KCONT ? 0 : e), gk = k0 + k + (KCONT ? e : 0);
+        const int64_t rr = gr < R ? gr : R - 1, kk = gk < K ? gk : K - 1;
+        const T x = KCONT ? P[rr * ld + kk] : P[kk * ld + rr];
+        t[e] = gk < K ? x : T(0);
       }
+      __builtin_memcpy(&reg[i], t, 16);
+      // One vector's addresses at a time: this path must not cost registers.
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 
-  // A K step that lies entirely inside [0, K): no K checks, and rows past R
-  // load row r0 instead (always inside the operand). Those rows only feed
-  // output rows / columns >= M / N, which the epilogue never stores, so they
-  // need no zeroing, and the loaded registers are first consumed by the LDS
-  // store after the MFMAs: the global latency stays hidden behind them.
-  // Requires VLOAD and, for r-contiguous operands, R % VEC == 0 (a vector
-  // is then either wholly inside or wholly outside [0, R)).
-  __device__ __forceinline__ void load_full(const T *__restrict__ P,
-                                            int64_t ld, int r0, int k0,
-                                            int R) {
-    static_assert(VLOAD, "vector loads only");
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
-      const int v = threadIdx.x + i * NTH;
-      if (NV % NTH != 0 && v >= NV) continue;
-      int r, k;
-      vec_pos(v, r, k);
-      const int gr = r0 + r, gk = k0 + k;
-      const int rr = gr < R ? gr : r0;
-      const T *src = KCONT ? P + (int64_t)rr * ld + gk : P + (int64_t)gk * ld + rr;
-      reg[i] = *reinterpret_cast<const vec4u *>(src);
-    }
-  }
-
-  // Full steps take the branch-free path; the K tail the checked one.
+  // Any step of any operand, ready for the LDS store.
   __device__ __forceinline__ void load_step(const T *__restrict__ P,
                                             int64_t ld, int r0, int k0, int R,
                                             int K, bool full) {
-    if constexpr (VLOAD) {
-      if (full) {
-        load_full(P, ld, r0, k0, R);
-        return;
-      }
+    if (full) {
+      load_wide<true>(P, ld, r0, k0, R, K);
+    } else if (wide(R, K)) {
+      load_wide<false>(P, ld, r0, k0, R, K);
+      mask(k0, K);
+    } else {
+      load_narrow(P, ld, r0, k0, R, K);
     }
-    load(P, ld, r0, k0, R, K);
   }
 
   __device__ __forceinline__ void store(char *lds) const {
     if constexpr (TRANS4) {
       int r, k;
-      vec_pos(threadIdx.x, r, k);  // reg[i] holds rows r..r+3 at k + i
+      vec_pos(tid, r, k);  // reg[i] holds rows r..r+3 at k + i
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         *reinterpret_cast<vec4u *>(lds + (r + e) * ROWB + k * 4) =
@@ -342,7 +402,7 @@ struct TileLoader {
     }
     if constexpr (TRANS2) {
       int r, k;
-      vec_pos(threadIdx.x, r, k);  // reg[i] holds rows r..r+3 at k + i
+      vec_pos(tid, r, k);  // reg[i] holds rows r..r+3 at k + i
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         *reinterpret_cast<vec2u *>(lds + (r + e) * ROWB + k * 4) =
@@ -351,7 +411,7 @@ struct TileLoader {
     }
     if constexpr (TRANS2H) {
       int r, k;
-      vec_pos(threadIdx.x, r, k);  // reg[i] holds rows r..r+7 at k + i
+      vec_pos(tid, r, k);  // reg[i] holds rows r..r+7 at k + i
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int d = e >> 1;
@@ -363,7 +423,7 @@ struct TileLoader {
     }
     if constexpr (TRANS4H) {
       int r, k;
-      vec_pos(threadIdx.x, r, k);  // reg[i] holds rows r..r+7 at k + i
+      vec_pos(tid, r, k);  // reg[i] holds rows r..r+7 at k + i
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         // Row r + e is the low (e even) or high half of dword e / 2.
@@ -381,7 +441,7 @@ struct TileLoader {
     }
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i) {
-      const int v = threadIdx.x + i * NTH;
+      const int v = tid + i * NTH;
       if (NV % NTH != 0 && v >= NV) continue;
       int r, k;
       vec_pos(v, r, k);
@@ -493,11 +553,11 @@ struct WaveTile {
 // kernel and the residue kernel, so all of them produce bit-identical sums
 // for the same K step.
 template <Elem E, bool A_K, bool B_K, int BM, int BN, int BK, int WM, int WN,
-          bool VA, bool VB, int MI, bool KFULL = false>
+          int MI, bool NARROW = true>
 __device__ __forceinline__ void gemm_mainloop(
     const typename ElemT<E>::T *__restrict__ A, int64_t lda,
     const typename ElemT<E>::T *__restrict__ B, int64_t ldb, int M, int N,
-    int K, int m0, int n0, char *lds,
+    int K, int m0, int n0, int tid, char *lds,
     typename WaveTile<E, BM, BN, WM, WN, MI>::AccV (
         &acc)[WaveTile<E, BM, BN, WM, WN, MI>::FM]
              [WaveTile<E, BM, BN, WM, WN, MI>::FN]) {
@@ -512,12 +572,12 @@ __device__ __forceinline__ void gemm_mainloop(
   constexpr int NTH = 64 * WM * WN;  // workgroup size
   constexpr int WTM = WT::WTM, WTN = WT::WTN, FM = WT::FM, FN = WT::FN;
 
-  using LA = TileLoader<T, BM, BK, A_K, VA, NTH>;
-  using LB = TileLoader<T, BN, BK, B_K, VB, NTH>;
+  using LA = TileLoader<T, BM, BK, A_K, NTH>;
+  using LB = TileLoader<T, BN, BK, B_K, NTH>;
   constexpr int ROWB = LA::ROWB;
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB;
 
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = tid >> 6, lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;
   const int lrow = lane % MI, lgrp = lane / MI;
 
@@ -526,11 +586,13 @@ __device__ __forceinline__ void gemm_mainloop(
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = AccV{};
 
-  LA la;
-  LB lb;
+  LA la(tid);
+  LB lb(tid);
   const int nk = (K + BK - 1) / BK;
-  // Steps with no K tail (KFULL: the caller guarantees K % BK == 0).
-  const int nfull = KFULL ? nk : K / BK;
+  // (NARROW = false: the caller knows that both operands are wide)
+  const bool wide_a = !NARROW || LA::wide(M, K);
+  const bool wide_b = !NARROW || LB::wide(N, K);
+  const int nfull = wide_a && wide_b ? K / BK : 0;  // steps without a tail
 
   // MFMAs over one LDS buffer. Small wave tiles (the 64 x 64 tiles of 8
   // waves, at most 2 fragments of each operand, and the 4-wave 64 x 64 FP64
@@ -665,17 +727,27 @@ __device__ __forceinline__ void gemm_mainloop(
   // top of step kt they are written to the other LDS buffer (free: every
   // wave passed the previous barrier) and refilled with step kt+2, so the
   // LDS writes overlap this step's MFMAs and one barrier ends the step.
-  auto load = [&](int k, bool full) {
-    la.load_step(A, lda, m0, k * BK, M, K, full);
-    lb.load_step(B, ldb, n0, k * BK, N, K, full);
+  auto load = [&](int k) {
+    if (wide_a)
+      la.template load_wide<false>(A, lda, m0, k * BK, M, K);
+    else
+      la.load_narrow(A, lda, m0, k * BK, M, K);
+    if (wide_b)
+      lb.template load_wide<false>(B, ldb, n0, k * BK, N, K);
+    else
+      lb.load_narrow(B, ldb, n0, k * BK, N, K);
   };
   auto store = [&](int k) {
+    if ((k + 1) * BK > K) {
+      if (wide_a) la.mask(k * BK, K);
+      if (wide_b) lb.mask(k * BK, K);
+    }
     la.store(buf(k));
     lb.store(buf(k) + A_BYTES);
   };
-  load(0, nfull > 0);
+  load(0);
   store(0);
-  if (nk > 1) load(1, 1 < nfull);
+  if (nk > 1) load(1);
   __syncthreads();
   int kt = 0;
   for (; kt + 2 < nfull; ++kt) {
@@ -683,11 +755,15 @@ __device__ __forceinline__ void gemm_mainloop(
       if constexpr (SPREAD) {
         if (c == 0) la.store(buf(kt + 1));
         if (c == 1) lb.store(buf(kt + 1) + A_BYTES);
-        if (c == 2) la.load_step(A, lda, m0, (kt + 2) * BK, M, K, true);
-        if (c == 3) lb.load_step(B, ldb, n0, (kt + 2) * BK, N, K, true);
+        if (c == 2)
+          la.template load_wide<true>(A, lda, m0, (kt + 2) * BK, M, K);
+        if (c == 3)
+          lb.template load_wide<true>(B, ldb, n0, (kt + 2) * BK, N, K);
       } else {
-        store(kt + 1);
-        load(kt + 2, true);
+        la.store(buf(kt + 1));
+        lb.store(buf(kt + 1) + A_BYTES);
+        la.template load_wide<true>(A, lda, m0, (kt + 2) * BK, M, K);
+        lb.template load_wide<true>(B, ldb, n0, (kt + 2) * BK, N, K);
       }
     };
     if constexpr (ILV) {
@@ -701,7 +777,7 @@ __device__ __forceinline__ void gemm_mainloop(
   }
   for (; kt < nk; ++kt) {
     if (kt + 1 < nk) store(kt + 1);
-    if (kt + 2 < nk) load(kt + 2, kt + 2 < nfull);
+    if (kt + 2 < nk) load(kt + 2);
     compute(buf(kt), none);
     __syncthreads();
   }
@@ -721,15 +797,20 @@ __device__ __forceinline__ void gemm_mainloop(
 //   32x32 FP32/INT32: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32;
 //   16x16 FP32: row 4 (l / 16) + r, column l % 16;
 //   16x16 FP64: row l / 16 + 4 r, column l % 16.
-// vec_c: C and ldc allow 16-byte accesses. Expects the LDS free on entry
-// (the main loop ends with a barrier) and ends with a barrier.
+// shift_m / shift_n: the loaders' edge_shift of either operand. Output row m of
+// the last, partial vector of rows then lies in tile row m + shift_m (and
+// columns alike); those few rows leave one by one. C is accessed 16 bytes at
+// a time at any alignment.
+// Expects the LDS free on entry (the main loop ends with a barrier) and ends
+// with a barrier.
 template <Elem E, typename OutT, int BM, int BN, int WM, int WN, int MI,
           int LDS_BYTES, typename AccArr>
 __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
                                                int64_t ldc, int M, int N,
                                                int m0, int n0, double alpha_d,
-                                               double beta_d, char *lds,
-                                               bool vec_c) {
+                                               double beta_d, int tid,
+                                               char *lds, int shift_m,
+                                               int shift_n) {
   using WT = WaveTile<E, BM, BN, WM, WN, MI>;
   using Acc = typename ElemT<E>::Acc;
   constexpr int LROW = BM + 16 / (int)sizeof(Acc);  // elements
@@ -746,10 +827,15 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
   constexpr int TPC = BM / VE;  // threads per column
   static_assert(BM % VE == 0 && NTH % TPC == 0, "epilogue shape");
   Acc *t = reinterpret_cast<Acc *>(lds);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = tid >> 6, lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;
   const int lrow = lane % MI, lgrp = lane / MI;
   const Acc alpha = (Acc)alpha_d, beta = (Acc)beta_d;
+  using GV = typename GlobalVec<OutT>::type;
+  // First row / column of a shifted last vector (M / N when there is none).
+  constexpr int VEC = ElemT<E>::VEC;
+  const int edge_m = shift_m ? M - (VEC - shift_m) : M;
+  const int edge_n = shift_n ? N - (VEC - shift_n) : N;
 #pragma unroll
   for (int c0 = 0; c0 < BN; c0 += NC) {
 #pragma unroll
@@ -782,16 +868,16 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
     __syncthreads();
 #pragma unroll
     for (int cc = 0; cc < NC; cc += NTH / TPC) {
-      const int nl = cc + (int)threadIdx.x / TPC;
-      const int ml = ((int)threadIdx.x % TPC) * VE;
+      const int nl = cc + tid / TPC;
+      const int ml = (tid % TPC) * VE;
       const int n = n0 + c0 + nl, m = m0 + ml;
       if (nl < NC && n < N && m < M) {
         OutT *dst = C + (int64_t)n * ldc + m;
-        const Acc *src = t + nl * LROW + ml;
-        if (vec_c && m + VE <= M) {
+        const Acc *src = t + (n < edge_n ? nl : nl + shift_n) * LROW + ml;
+        if (m + VE <= edge_m) {
           OutT cin[VE], o[VE];
           if (beta != Acc(0)) {
-            const vec4u w = *reinterpret_cast<const vec4u *>(dst);
+            const vec4u w = *reinterpret_cast<const GV *>(dst);
             __builtin_memcpy(cin, &w, 16);
           }
 #pragma unroll
@@ -802,8 +888,9 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
           }
           vec4u w;
           __builtin_memcpy(&w, o, 16);
-          *reinterpret_cast<vec4u *>(dst) = w;
+          *reinterpret_cast<GV *>(dst) = w;
         } else {
+          if (m >= edge_m) src += shift_m;
           const int ne = M - m < VE ? M - m : VE;
           for (int e = 0; e < ne; ++e) {
             Acc v = alpha * src[e];
@@ -818,36 +905,33 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
 }
 
 // One BM x BN output tile at (m0, n0) of C = alpha*A'*B' + beta*C, the whole
-// K range; beta == 0 never reads C.
+// K range; beta == 0 never reads C. LDS_BYTES: the LDS at `lds`.
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
-          int WM, int WN, bool VA, bool VB, int MI = 16>
+          int WM, int WN, int MI, int LDS_BYTES, bool NARROW = true>
 __device__ __forceinline__ void gemm_tile(
     const typename ElemT<E>::T *__restrict__ A, int64_t lda,
     const typename ElemT<E>::T *__restrict__ B, int64_t ldb, OutT *C,
     int64_t ldc, int M, int N, int K, double alpha_d, double beta_d, int m0,
-    int n0, char *lds) {
+    int n0, int tid, char *lds) {
+  using T = typename ElemT<E>::T;
   using WT = WaveTile<E, BM, BN, WM, WN, MI>;
+  constexpr int NTH = 64 * WM * WN;
   typename WT::AccV acc[WT::FM][WT::FN];
-  gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, VA, VB, MI>(
-      A, lda, B, ldb, M, N, K, m0, n0, lds, acc);
-  constexpr int VE = 16 / (int)sizeof(OutT);
-  const bool vec_c = reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc % VE == 0;
-  store_tile_lds<E, OutT, BM, BN, WM, WN, MI, tile_lds_bytes<E, BM, BN, BK>()>(
-      acc, C, ldc, M, N, m0, n0, alpha_d, beta_d, lds, vec_c);
+  gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, MI, NARROW>(
+      A, lda, B, ldb, M, N, K, m0, n0, tid, lds, acc);
+  store_tile_lds<E, OutT, BM, BN, WM, WN, MI, LDS_BYTES>(
+      acc, C, ldc, M, N, m0, n0, alpha_d, beta_d, tid, lds,
+      TileLoader<T, BM, BK, A_K, NTH>::edge_shift(M),
+      TileLoader<T, BN, BK, B_K, NTH>::edge_shift(N));
 }
 
-// CHK (pointer-array batches with 16-byte loads): the matrices of a batch
-// come from a device array of pointers that the host never sees, so each
-// workgroup checks its problem's A and B bases (one problem per blockIdx.z,
-// so the branch is uniform) and runs the element-wise loaders for a base
-// that is not 16-byte aligned. Offsets and leading dimensions were checked
-// on the host.
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
-          int WM, int WN, bool VA, bool VB, int MI = 16, bool CHK = false>
+          int WM, int WN, int MI = 16>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     GemmParams p) {
   using T = typename ElemT<E>::T;
-  __shared__ __attribute__((aligned(16))) char lds[tile_lds_bytes<E, BM, BN, BK>()];
+  constexpr int LDS_BYTES = tile_lds_bytes<E, BM, BN, BK>();
+  __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
   const int z = blockIdx.z;
   const T *A;
   const T *B;
@@ -866,18 +950,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     C = static_cast<OutT *>(p.C) + p.cOff + (int64_t)z * p.strideC;
   int tile_m, tile_n;
   tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-  if constexpr (CHK) {
-    if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) &
-         15u) != 0) {
-      gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, false, false, MI>(
-          A, p.lda, B, p.ldb, C, p.ldc, p.M, p.N, p.K, p.alpha, p.beta,
-          tile_m * BM, tile_n * BN, lds);
-      return;
-    }
-  }
-  gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, VA, VB, MI>(
+  gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES>(
       A, p.lda, B, p.ldb, C, p.ldc, p.M, p.N, p.K, p.alpha, p.beta,
-      tile_m * BM, tile_n * BN, lds);
+      tile_m * BM, tile_n * BN, threadIdx.x, lds);
 }
 
 // Split-K partial tile: the K range [z ks, min(K, (z + 1) ks)) of one
@@ -886,7 +961,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
 // CUs and a long K, splitting K gives every CU several workgroups to switch
 // between; splitk_reduce_kernel then adds the partials in split order.
 template <Elem E, bool A_K, bool B_K, int BM, int BN, int BK, int WM, int WN,
-          bool VA, bool VB, int MI>
+          int MI>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_splitk_kernel(
     GemmParams p, int ks, typename ElemT<E>::Acc *W) {
   using T = typename ElemT<E>::T;
@@ -902,14 +977,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_splitk_kernel(
                (B_K ? (int64_t)k0 : (int64_t)k0 * p.ldb);
   int tile_m, tile_n;
   tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-  using WT = WaveTile<E, BM, BN, WM, WN, MI>;
-  typename WT::AccV acc[WT::FM][WT::FN];
-  gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, VA, VB, MI>(
-      A, p.lda, B, p.ldb, p.M, p.N, kl, tile_m * BM, tile_n * BN, lds, acc);
-  constexpr int VE = 16 / (int)sizeof(Acc);
-  store_tile_lds<E, Acc, BM, BN, WM, WN, MI, LDS_BYTES>(
-      acc, W + (int64_t)z * p.M * p.N, p.M, p.M, p.N, tile_m * BM,
-      tile_n * BN, 1.0, 0.0, lds, p.M % VE == 0);
+  gemm_tile<E, Acc, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES>(
+      A, p.lda, B, p.ldb, W + (int64_t)z * p.M * p.N, p.M, p.M, p.N, kl, 1.0,
+      0.0, tile_m * BM, tile_n * BN, threadIdx.x, lds);
 }
 
 // C = alpha * sum_z W[z] + beta * C, the partials added in split order.

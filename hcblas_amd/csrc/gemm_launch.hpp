@@ -7,14 +7,12 @@
 namespace hcb {
 
 // Launches C = alpha*A'*B' + beta*C for `batch` problems described by p
-// (column-major storage; a_k / b_k give the operand orientations; vload
-// allows 16-byte global loads for both operands).
+// (column-major storage; a_k / b_k give the operand orientations).
 template <Elem E, typename OutT>
 hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
-                           bool a_k, bool b_k, bool vload, int64_t batch);
+                           bool a_k, bool b_k, int64_t batch);
 
-// Split-K form for one problem (no batch, no pointer arrays, vector loads):
-// S partial tiles of K step ks into W (S * M * N accumulators), then the
+// Split-K form for one problem (no batch, no pointer arrays): S partial tiles of K step ks into W (S * M * N accumulators), then the
 // reduction into C.
 template <Elem E, typename OutT>
 hcblasStatus_t launch_gemm_splitk(hipStream_t stream, int num_cus,

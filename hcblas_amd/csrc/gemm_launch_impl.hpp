@@ -28,7 +28,7 @@ struct TileCfg<Elem::BF16> {
 template <Elem E, typename OutT, int BM, int BN, int BK, int WM, int WN,
           int MI = 16>
 hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
-                            bool b_k, bool vload, int64_t batch) {
+                            bool b_k, int64_t batch) {
   p.tiles_m = (int)cdiv(p.M, BM);
   p.tiles_n = (int)cdiv(p.N, BN);
   const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n);
@@ -45,25 +45,14 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
       else q.C = (char *)q.C + b0 * q.strideC * sizeof(OutT);
     }
     dim3 grid(tiles, 1, (unsigned)nb);
-    // Pointer-array batches with 16-byte loads check each problem's bases
-    // on the device (CHK).
-    const bool chk = vload && (q.Aptrs || q.Bptrs);
-#define HCB_GEMM_CASE(AK, BKC, VL, CK)                                    \
-  if (a_k == AK && b_k == BKC && vload == VL && chk == CK)                \
-    gemm_mfma_kernel<E, OutT, AK, BKC, BM, BN, BK, WM, WN, VL, VL, MI, CK> \
+#define HCB_GEMM_CASE(AK, BKC)                                   \
+  if (a_k == AK && b_k == BKC)                                   \
+    gemm_mfma_kernel<E, OutT, AK, BKC, BM, BN, BK, WM, WN, MI>   \
         <<<grid, 64 * WM * WN, 0, stream>>>(q);
-    HCB_GEMM_CASE(false, false, false, false)
-    HCB_GEMM_CASE(false, true, false, false)
-    HCB_GEMM_CASE(true, false, false, false)
-    HCB_GEMM_CASE(true, true, false, false)
-    HCB_GEMM_CASE(false, false, true, false)
-    HCB_GEMM_CASE(false, true, true, false)
-    HCB_GEMM_CASE(true, false, true, false)
-    HCB_GEMM_CASE(true, true, true, false)
-    HCB_GEMM_CASE(false, false, true, true)
-    HCB_GEMM_CASE(false, true, true, true)
-    HCB_GEMM_CASE(true, false, true, true)
-    HCB_GEMM_CASE(true, true, true, true)
+    HCB_GEMM_CASE(false, false)
+    HCB_GEMM_CASE(false, true)
+    HCB_GEMM_CASE(true, false)
+    HCB_GEMM_CASE(true, true)
 #undef HCB_GEMM_CASE
     hcblasStatus_t st = launch_status();
     if (st != HCBLAS_STATUS_SUCCESS) return st;
@@ -79,50 +68,37 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
 //         waves, 64x64;
 //   FP64  256x128x16, 8 waves of 64x64 (71.6 TF/s NN and TN, 91%, with the
 //         same interleave; 66.9 / 64.5 before it; 128x256 2x4 was as fast
-//         on NN, 128x128 and
-//         smaller tiles stay at 75% or below; aligned operands only, the
-//         element-wise loaders spill at this size), then 128x64x16 8 waves
-//         (58.5), then 64x64 8 waves;
+//         on NN, 128x128 and smaller tiles stay at 75% or below), then
+//         128x64x16 8 waves (58.5), then 64x64 8 waves;
 //   F16 / BF16 256x256x64, 8 waves on 32x32 blocks, then 128x128 8 waves,
 //         then 64x64.
 template <Elem E, typename OutT>
 hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
-                           bool a_k, bool b_k, bool vload, int64_t batch) {
+                           bool a_k, bool b_k, int64_t batch) {
   auto tiles = [&](int bm, int bn) {
     return cdiv(p.M, bm) * cdiv(p.N, bn) * batch;
   };
-  // Tiles whose element-wise loaders do not fit the registers take aligned
-  // strided operands only: a pointer-array batch may hold misaligned bases,
-  // which its kernel sends to the element-wise loaders.
-  const bool big_ok = vload && !p.Aptrs && !p.Bptrs;
   if constexpr (E == Elem::F32) {
     if (tiles(256, 256) >= num_cus)
-      return launch_tiles<E, OutT, 256, 256, 32, 2, 4, 32>(stream, p, a_k, b_k,
-                                                           vload, batch);
+      return launch_tiles<E, OutT, 256, 256, 32, 2, 4, 32>(stream, p, a_k, b_k, batch);
     if (tiles(256, 128) >= num_cus)
-      return launch_tiles<E, OutT, 256, 128, 32, 2, 4>(stream, p, a_k, b_k,
-                                                       vload, batch);
+      return launch_tiles<E, OutT, 256, 128, 32, 2, 4>(stream, p, a_k, b_k, batch);
     if (tiles(128, 128) >= num_cus)
-      return launch_tiles<E, OutT, 128, 128, 32, 2, 2>(stream, p, a_k, b_k,
-                                                       vload, batch);
+      return launch_tiles<E, OutT, 128, 128, 32, 2, 2>(stream, p, a_k, b_k, batch);
   } else if constexpr (E == Elem::F64) {
-    if (big_ok && tiles(256, 128) >= num_cus)
-      return launch_tiles<E, OutT, 256, 128, 16, 4, 2>(stream, p, a_k, b_k,
-                                                       vload, batch);
+    if (tiles(256, 128) >= num_cus)
+      return launch_tiles<E, OutT, 256, 128, 16, 4, 2>(stream, p, a_k, b_k, batch);
     if (tiles(128, 64) >= num_cus)
-      return launch_tiles<E, OutT, 128, 64, 16, 2, 4>(stream, p, a_k, b_k,
-                                                      vload, batch);
+      return launch_tiles<E, OutT, 128, 64, 16, 2, 4>(stream, p, a_k, b_k, batch);
   } else {
-    // (the element-wise loaders of unaligned operands do not fit the 256x256
-    // tile's registers: they take the 128x128 tile)
-    if (big_ok && tiles(256, 256) >= num_cus)
+    if (tiles(256, 256) >= num_cus)
       return launch_tiles<E, OutT, 256, 256, TileCfg<E>::BK_BIG, 2, 4, 32>(
-          stream, p, a_k, b_k, vload, batch);
+          stream, p, a_k, b_k, batch);
     // 8 waves of 64 x 32 (fragment read-ahead, two-vector transposed loads):
     // 2048^3 HGEMM NN 38.6 against 44.4 us with 4 waves of 64 x 64.
     if (tiles(128, 128) >= num_cus)
       return launch_tiles<E, OutT, 128, 128, TileCfg<E>::BK_BIG, 2, 4, 32>(
-          stream, p, a_k, b_k, vload, batch);
+          stream, p, a_k, b_k, batch);
   }
   // Small problems: 64x64 tiles, 8 waves of 32x16 for every type (more
   // waves per CU to cover the load latency when there are only about as
@@ -134,11 +110,10 @@ hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
   // 29.5 with 64); shorter K keeps 32 so the last step pads little.
   if constexpr (E == Elem::F32) {
     if (p.K >= 512)
-      return launch_tiles<E, OutT, 64, 64, 128, 2, 4>(stream, p, a_k, b_k,
-                                                      vload, batch);
+      return launch_tiles<E, OutT, 64, 64, 128, 2, 4>(stream, p, a_k, b_k, batch);
   }
   return launch_tiles<E, OutT, 64, 64, TileCfg<E>::BK_SMALL, 2, 4>(
-      stream, p, a_k, b_k, vload, batch);
+      stream, p, a_k, b_k, batch);
 }
 
 template <Elem E, typename OutT>
@@ -155,7 +130,7 @@ hcblasStatus_t launch_gemm_splitk(hipStream_t stream, int num_cus,
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)S);
 #define HCB_SPLITK_CASE(AK, BKC)                                           \
   if (a_k == AK && b_k == BKC)                                             \
-    gemm_splitk_kernel<E, AK, BKC, BM, BN, BK, WM, WN, true, true, 16>     \
+    gemm_splitk_kernel<E, AK, BKC, BM, BN, BK, WM, WN, 16>                 \
         <<<grid, 64 * WM * WN, 0, stream>>>(p, ks, W);
   HCB_SPLITK_CASE(false, false)
   HCB_SPLITK_CASE(false, true)

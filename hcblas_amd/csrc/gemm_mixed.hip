@@ -53,12 +53,13 @@ __device__ __forceinline__ void split3_bf16(float x, uint16_t &h, uint16_t &m,
 // Global -> register loader of an FP32 tile (the plain kernel's loader) whose
 // store writes three BF16 planes [ROWS][BK] (row stride BK*2 + 16 bytes,
 // planes PLANE bytes apart) in the BF16 operand's LDS layout.
-template <int ROWS, int BK, bool VLOAD, int NTH>
+template <int ROWS, int BK, int NTH>
 struct SplitPlaneLoader {
-  using L = TileLoader<float, ROWS, BK, true, VLOAD, NTH>;
+  using L = TileLoader<float, ROWS, BK, true, NTH>;
   static constexpr int ROWB = BK * 2 + 16;
   static constexpr int PLANE = ROWS * ROWB;
   L ld;
+  __device__ __forceinline__ explicit SplitPlaneLoader(int tid) : ld(tid) {}
   __device__ __forceinline__ void load_step(const float *__restrict__ P,
                                             int64_t ld_, int r0, int k0,
                                             int R, int K, bool full) {
@@ -132,10 +133,9 @@ struct MixedParams {
   int tiles_m, tiles_n;
 };
 
-// AF: A' is the FP32 operand (else B' is); both are k-contiguous. VL:
-// 16-byte global loads legal for both. OutT: float or Bf16Out. BM x BN
-// tile over WM x WN waves.
-template <bool AF, bool VL, typename OutT, int BM, int BN, int WM, int WN>
+// AF: A' is the FP32 operand (else B' is); both are k-contiguous. OutT: float
+// or Bf16Out. BM x BN tile over WM x WN waves.
+template <bool AF, typename OutT, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
     MixedParams p) {
   constexpr int NTH = 64 * WM * WN, MI = 32;
@@ -144,10 +144,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
   constexpr int PLANE_A = BM * kMRowB, PLANE_B = BN * kMRowB;
   constexpr int BUF = mixed_buf_bytes<AF, BM, BN>(), LDS = 2 * BUF;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
-  using FL_A = SplitPlaneLoader<BM, kMBK, VL, NTH>;
-  using FL_B = SplitPlaneLoader<BN, kMBK, VL, NTH>;
-  using HL_A = TileLoader<uint16_t, BM, kMBK, true, VL, NTH>;
-  using HL_B = TileLoader<uint16_t, BN, kMBK, true, VL, NTH>;
+  using FL_A = SplitPlaneLoader<BM, kMBK, NTH>;
+  using FL_B = SplitPlaneLoader<BN, kMBK, NTH>;
+  using HL_A = TileLoader<uint16_t, BM, kMBK, true, NTH>;
+  using HL_B = TileLoader<uint16_t, BN, kMBK, true, NTH>;
   using LA = typename std::conditional<AF, FL_A, HL_A>::type;
   using LB = typename std::conditional<AF, HL_B, FL_B>::type;
   using TA = typename std::conditional<AF, float, uint16_t>::type;
@@ -172,8 +172,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = typename WT::AccV{};
 
-  LA la;
-  LB lb;
+  LA la(threadIdx.x);
+  LB lb(threadIdx.x);
   const int K = p.K;
   const int nk = (K + kMBK - 1) / kMBK, nfull = K / kMBK;
   auto buf = [&](int kt) { return lds + (kt & 1) * BUF; };
@@ -228,10 +228,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
       __syncthreads();
     }
   }
-  const bool vec_c = reinterpret_cast<uintptr_t>(C) % 16 == 0 &&
-                     p.ldc % (16 / (int)sizeof(OutT)) == 0;
   store_tile_lds<Elem::BF16, OutT, BM, BN, WM, WN, MI, LDS>(
-      acc, C, p.ldc, p.M, p.N, m0, n0, (double)p.alpha, 0.0, lds, vec_c);
+      acc, C, p.ldc, p.M, p.N, m0, n0, (double)p.alpha, 0.0, threadIdx.x, lds,
+      0, 0);
 }
 
 // Tiles: 256 x 256 over 8 waves of 64 x 128 (FP32 operand along the wave
@@ -239,7 +238,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
 // 8 per 12 for 64 x 64 wave tiles) when both output sides reach 256, else
 // 128 x 128 over 4 waves of 64 x 64.
 template <bool AF, typename OutT, int BM, int BN, int WM, int WN>
-hcblasStatus_t launch_mixed_cfg(hipStream_t s, MixedParams p, bool vl,
+hcblasStatus_t launch_mixed_cfg(hipStream_t s, MixedParams p,
                                 int64_t batch) {
   p.tiles_m = (int)cdiv(p.M, BM);
   p.tiles_n = (int)cdiv(p.N, BN);
@@ -253,27 +252,23 @@ hcblasStatus_t launch_mixed_cfg(hipStream_t s, MixedParams p, bool vl,
           b0 * q.strideB * (AF ? sizeof(uint16_t) : sizeof(float));
     q.C = static_cast<OutT *>(q.C) + b0 * q.strideC;
     dim3 grid(tiles, 1, (unsigned)nb);
-    if (vl)
-      gemm_mixed_kernel<AF, true, OutT, BM, BN, WM, WN>
-          <<<grid, 64 * WM * WN, 0, s>>>(q);
-    else
-      gemm_mixed_kernel<AF, false, OutT, BM, BN, WM, WN>
-          <<<grid, 64 * WM * WN, 0, s>>>(q);
+    gemm_mixed_kernel<AF, OutT, BM, BN, WM, WN>
+        <<<grid, 64 * WM * WN, 0, s>>>(q);
     const hcblasStatus_t st = launch_status();
     if (st != HCBLAS_STATUS_SUCCESS) return st;
   }
   return HCBLAS_STATUS_SUCCESS;
 }
 template <bool AF, typename OutT>
-hcblasStatus_t launch_mixed(hipStream_t s, MixedParams p, bool vl,
+hcblasStatus_t launch_mixed(hipStream_t s, MixedParams p,
                             int64_t batch) {
   if (p.M >= 256 && p.N >= 256) {
     if constexpr (AF)
-      return launch_mixed_cfg<AF, OutT, 256, 256, 4, 2>(s, p, vl, batch);
+      return launch_mixed_cfg<AF, OutT, 256, 256, 4, 2>(s, p, batch);
     else
-      return launch_mixed_cfg<AF, OutT, 256, 256, 2, 4>(s, p, vl, batch);
+      return launch_mixed_cfg<AF, OutT, 256, 256, 2, 4>(s, p, batch);
   }
-  return launch_mixed_cfg<AF, OutT, 128, 128, 2, 2>(s, p, vl, batch);
+  return launch_mixed_cfg<AF, OutT, 128, 128, 2, 2>(s, p, batch);
 }
 
 // out[z][c * ldo + r] = in[z][r * ldi + c] for r < rows, c < cols, z <
@@ -368,11 +363,6 @@ void launch_transpose(hipStream_t s, int rows, int cols, const T *in,
   }
 }
 
-inline bool aligned_ptr(const void *p, size_t esize, int64_t off) {
-  return ((reinterpret_cast<uintptr_t>(p) + (uintptr_t)(off * esize)) & 15u) ==
-         0;
-}
-
 }  // namespace
 
 hcblasStatus_t gemm_mixed_bf16(hcblasHandle_t h, const Canon &c, bool a_f32,
@@ -438,17 +428,11 @@ hcblasStatus_t gemm_mixed_bf16(hcblasHandle_t h, const Canon &c, bool a_f32,
   p.ldc = ldc;
   p.strideC = strideC;
   p.alpha = alpha;
-  // 16-byte loads: every base, leading dimension and batch stride a whole
-  // number of vectors of its type.
-  const int va = 16 / (int)ea, vb = 16 / (int)eb;
-  const bool vl = lda % va == 0 && ldb % vb == 0 && aligned_ptr(A, ea, 0) &&
-                  aligned_ptr(B, eb, 0) &&
-                  (batch == 1 || (sA % va == 0 && sB % vb == 0));
   if (c_bf16)
-    return a_f32 ? launch_mixed<true, Bf16Out>(h->stream, p, vl, batch)
-                 : launch_mixed<false, Bf16Out>(h->stream, p, vl, batch);
-  return a_f32 ? launch_mixed<true, float>(h->stream, p, vl, batch)
-               : launch_mixed<false, float>(h->stream, p, vl, batch);
+    return a_f32 ? launch_mixed<true, Bf16Out>(h->stream, p, batch)
+                 : launch_mixed<false, Bf16Out>(h->stream, p, batch);
+  return a_f32 ? launch_mixed<true, float>(h->stream, p, batch)
+               : launch_mixed<false, float>(h->stream, p, batch);
 }
 
 }  // namespace hcb

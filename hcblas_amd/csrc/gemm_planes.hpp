@@ -55,8 +55,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_planes_kernel(
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int FM = WTM / MI, FN = WTN / MI;
   constexpr int NTH = 64 * WM * WN;
-  using LA = TileLoader<T, BM, BK, true, true, NTH>;
-  using LB = TileLoader<T, BN, BK, true, true, NTH>;
+  using LA = TileLoader<T, BM, BK, true, NTH>;
+  using LB = TileLoader<T, BN, BK, true, NTH>;
   constexpr int ROWB = LA::ROWB;
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB;
   __shared__ __attribute__((aligned(16))) char lds[2 * (A_BYTES + B_BYTES)];
@@ -91,13 +91,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_planes_kernel(
   int total = 0;
   for (int g = 0; g < p.ngroups; ++g) total += p.np[g] * kt_per_plane;
 
-  LA la;
-  LB lb;
+  LA la(threadIdx.x);
+  LB lb(threadIdx.x);
   auto load_tile = [&](int g, int kt) {
     const int64_t ka = (int64_t)p.a0[g] * p.Kp + (int64_t)kt * BK;
     const int64_t kb = (int64_t)p.b0[g] * p.Kp + (int64_t)kt * BK;
-    la.load_full(Ap + ka, ld, m0, 0, p.M);
-    lb.load_full(Bp + kb, ld, n0, 0, p.N);
+    la.template load_wide<true>(Ap + ka, ld, m0, 0, p.M, BK);
+    lb.template load_wide<true>(Bp + kb, ld, n0, 0, p.N, BK);
   };
   auto buf = [&](int t) { return lds + (t & 1) * (A_BYTES + B_BYTES); };
   auto store = [&](int t) {

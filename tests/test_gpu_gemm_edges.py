@@ -1,0 +1,79 @@
+"""GEMM on operands of any alignment: every size modulo the 16-byte vector,
+fewer rows than one vector, tightly packed odd leading dimensions and bases at
+odd element offsets, in every order and transpose form.
+
+The reference is the FP64 product of the stored values. The bound is that of
+tests/gemm_bounds.py, c * sqrt(K) * u * (|alpha| |op(A)| |op(B)| + |beta| |C|)
+plus one rounding of the result, with c = 4 and u the unit of the accumulation
+type. Elements of C's buffer outside the M x N block keep their bits.
+"""
+import numpy as np
+import pytest
+
+from gpu_util import to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+ROW, COL = 0, 1
+DT = {"s": np.float32, "d": np.float64, "h": np.float16}
+
+
+def _stored(rng, dt, rows, cols, order, skew):
+    """rows x cols uniform values, tightly packed in `order` behind `skew`
+    elements and followed by seven more: (buffer, leading dimension, the
+    matrix in FP64)."""
+    v = rng.uniform(-1, 1, (rows, cols)).astype(dt)
+    flat = (v if order == ROW else v.T).ravel()
+    buf = np.full(skew + flat.size + 7, 99, dt)
+    buf[skew:skew + flat.size] = flat
+    return buf, max(1, cols if order == ROW else rows), v.astype(np.float64)
+
+
+def _check(hc, handle, p, order, ta, tb, M, N, K, skew, seed):
+    rng = np.random.default_rng(seed)
+    dt = DT[p]
+    A, lda, Am = _stored(rng, dt, *((K, M) if ta else (M, K)), order, skew)
+    B, ldb, Bm = _stored(rng, dt, *((N, K) if tb else (K, N)), order, skew)
+    C, ldc, Cm = _stored(rng, dt, M, N, order, skew)
+    Am, Bm = Am.T if ta else Am, Bm.T if tb else Bm
+    bits = (lambda a: a.view(np.uint16)) if p == "h" else (lambda a: a)
+    dC = to_dev(bits(C))
+    st = getattr(hc.api, f"hcblas_{p}gemm")(
+        handle, order, ta, tb, M, N, K, 0.75, to_dev(bits(A)), lda,
+        to_dev(bits(B)), ldb, 0.5, dC, ldc, skew, skew, skew)
+    assert st == 0
+    got = to_host(dC).view(dt)
+    what = (p, order, ta, tb, M, N, K, skew)
+    assert np.array_equal(got[:skew], C[:skew]), what
+    assert np.array_equal(got[skew + M * N:], C[skew + M * N:]), what
+    g = got[skew:skew + M * N].astype(np.float64)
+    g = g.reshape(M, N) if order == ROW else g.reshape(N, M).T
+    ref = 0.75 * (Am @ Bm) + 0.5 * Cm
+    u = np.finfo(np.float64 if p == "d" else np.float32).eps
+    bound = 4 * np.sqrt(K) * u * (0.75 * (abs(Am) @ abs(Bm)) + 0.5 * abs(Cm))
+    bound += 2 * np.finfo(dt).eps * abs(ref)
+    if p == "h":
+        bound += np.finfo(dt).smallest_subnormal
+    assert np.all(abs(g - ref) <= bound), (what, (abs(g - ref) / bound).max())
+
+
+@pytest.mark.parametrize("p", ["s", "d", "h"])
+@pytest.mark.parametrize("order", [ROW, COL])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_every_residue_of_the_vector(hc, handle, p, order, ta, tb):
+    # below one vector, every residue of it, and the edge of a 64-row tile
+    for M, N in [(1, 6), (2, 1), (3, 7), (5, 65), (6, 66), (7, 67), (8, 61),
+                 (9, 68), (63, 2), (66, 69), (70, 71), (129, 62)]:
+        for K in (1, 37):
+            for skew in (0, 1):
+                _check(hc, handle, p, order, ta, tb, M, N, K, skew,
+                       M * 1000 + N * 10 + K + skew)
+
+
+# The larger tiles (128 x 64 FP64, 128 x 128 and 256 x 256 FP32 / FP16), with
+# partial last tiles, a shifted last vector in either direction and a K tail.
+@pytest.mark.parametrize("p,M,N,K", [("s", 2051, 2049, 75), ("d", 2051, 1777, 35),
+                                     ("h", 2053, 2051, 139),
+                                     ("s", 4111, 4097, 67), ("h", 4111, 4097, 67)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_large_tiles_at_odd_sizes(hc, handle, p, M, N, K, ta, tb):
+    _check(hc, handle, p, COL, ta, tb, M, N, K, 1, M + N + K)
