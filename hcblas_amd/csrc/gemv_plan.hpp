@@ -12,8 +12,6 @@ namespace hcb {
 
 // Kernel geometry constants of level2.hip.
 constexpr int kGemvThreads = 256;
-constexpr int kBandNRows = 4;     // XR of the band-N kernel
-constexpr int kBandNCols = 8;     // UC: columns in flight
 constexpr int kCPW = 4;           // columns per wave of the column kernel
 constexpr int kColsPerBlock = 4 * kCPW;
 constexpr int kBandCols = 8;      // columns per workgroup of the band kernel
@@ -22,6 +20,8 @@ enum class GemvKernel { kBandN, kPanel, kBand16, kBand8, kColumn };
 
 struct GemvPlan {
   GemvKernel kernel;
+  int xr;           // row steps of a band (band kernels)
+  int waves;        // waves per workgroup (panel kernel)
   int64_t oblocks;  // output blocks (grid x, or grid y for band-N)
   int splits;       // reduction splits (grid y, or grid x for band-N)
   size_t partial_bytes;  // split partials (0 when splits == 1)
@@ -30,58 +30,88 @@ struct GemvPlan {
 inline int64_t plan_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // panel: the reduction runs along the contiguous storage rows' columns
-// (y has R entries); otherwise along the rows (y has Cc entries). vec: the
-// 16-byte path is legal; vn: elements per 16 bytes; esize: element bytes.
+// (y has R entries); otherwise along the rows (y has Cc entries). vec: rows
+// are read 16 bytes at a time (vn elements; R >= vn). esize: element bytes.
+//
+// Every rule aims at a grid that covers the GPU (what a memory-bound kernel
+// lacks on a small or narrow matrix is loads in flight, not their width) but
+// not at a few workgroups more than the GPU holds side by side: 258 bands of
+// a 12000^2 SGEMV-N took 120 us, 255 took 91.
 inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
                           bool vec, int vn, size_t esize, int64_t batch) {
   const int64_t len_y = panel ? R : Cc;
   const int64_t target = (int64_t)num_cus * 4;  // workgroups to aim for
-  GemvPlan p{GemvKernel::kColumn, 1, 1, 0};
-  // Band kernel for the column case when a band of 16 (or 8) row steps
-  // fits and the column blocks alone give the grid enough workgroups.
-  int band_xr = 0;
-  if (!panel && vec) {
-    for (int xr : {16, 8}) {
-      const int64_t bands = plan_cdiv(R, (int64_t)xr * kGemvThreads * vn);
-      if (R >= (int64_t)xr * kGemvThreads * vn && bands <= 65535 &&
-          plan_cdiv(Cc, kBandCols) * bands * batch >= target) {
-        band_xr = xr;
+  GemvPlan p{GemvKernel::kColumn, 0, 4, 1, 1, 0};
+  const int64_t step = (int64_t)kGemvThreads * vn;  // rows of one band step
+  const int64_t steps = plan_cdiv(R, step);
+  // Below three quarters of a step a band would leave a whole wave idle.
+  const bool band = vec && 4 * R >= 3 * step;
+  // Row-contiguous case of at most 512 columns and 32 MB: sixteen waves per 64
+  // vectors of rows, a wave's columns in at most two trips, one launch. (Each
+  // workgroup reads 1 KiB of every column; the split form's second launch
+  // costs more than the CUs that stay idle.)
+  const int64_t pblocks = plan_cdiv(R, 64 * (int64_t)(vec ? vn : 1));
+  const bool short_sums = panel && Cc > 32 && Cc <= 512 &&
+                          pblocks * batch < 2 * (int64_t)num_cus &&
+                          R * Cc * (int64_t)esize * batch <= (32ll << 20);
+  // Column case. A band of up to 16 steps, all bands alike (R = 20011, 20
+  // steps: two bands of 10 instead of 16 and 4), and more, shorter bands
+  // where the column blocks are few: up to one workgroup per CU, bands of at
+  // least 2 steps.
+  int64_t bands = plan_cdiv(steps, 16);
+  if (!panel && band) {
+    const int64_t blocks = plan_cdiv(Cc, kBandCols) * batch;
+    bands = std::max(bands,
+                     std::min((int64_t)num_cus / blocks, (steps + 1) / 2));
+  }
+  if (!panel && band && bands <= 65535) {
+    int64_t xr = plan_cdiv(steps, bands);
+    if (xr > 4) xr = (xr + 1) / 2 * 2;  // instances: 1..4, 6, 8, .. 16
+    p.kernel = xr == 16 ? GemvKernel::kBand16 : GemvKernel::kBand8;
+    p.xr = (int)xr;
+    p.oblocks = plan_cdiv(Cc, kBandCols);
+    p.splits = (int)plan_cdiv(steps, xr);
+  } else if (panel && band && !short_sums && Cc >= 64 && steps <= 65535) {
+    // Row-contiguous case: bands of 4 steps (16 KiB of each column in one
+    // run) where they waste at most an eighth of their lanes and, with at
+    // least 64 columns per block, still give every CU a workgroup; else 2
+    // or 1. Column blocks: about one workgroup per CU (at 16384^2 fp32 256
+    // workgroups took 152 us, 128 178 us, 512 159 us), at least 32 columns.
+    // (4096^2 fp32 used one band of 4 steps in 16 blocks: 16 workgroups,
+    // 75 us.)
+    int xr = 1;
+    for (int x : {4, 2}) {
+      const int64_t b = plan_cdiv(steps, x);
+      if (8 * R >= 7 * b * x * step &&
+          b * batch * plan_cdiv(Cc, 64) >= num_cus) {
+        xr = x;
         break;
       }
     }
-  }
-  // Band-N kernel for the row-contiguous case: whole 16 KiB bands and at
-  // least 64 columns.
-  const int64_t bandn_rows = (int64_t)kBandNRows * kGemvThreads * vn;
-  const bool bandn = panel && vec && R >= bandn_rows && Cc >= 64 &&
-                     plan_cdiv(R, bandn_rows) <= 65535;
-  if (bandn) {
     p.kernel = GemvKernel::kBandN;
-    p.oblocks = plan_cdiv(R, bandn_rows);
-    const int64_t per_batch = std::max<int64_t>(
-        1, plan_cdiv((int64_t)num_cus, p.oblocks * batch));
+    p.xr = xr;
+    p.oblocks = plan_cdiv(steps, xr);
     p.splits = (int)std::max<int64_t>(
-        1, std::min<int64_t>(plan_cdiv(Cc, 256), per_batch));
+        1, std::min(plan_cdiv(Cc, 32), num_cus / (p.oblocks * batch)));
   } else if (panel) {
     p.kernel = GemvKernel::kPanel;
-    p.oblocks = plan_cdiv(R, 64 * (int64_t)(vec ? vn : 1));
-    // at least 32 columns per wave-interleaved split
-    const int64_t max_split = std::max<int64_t>(1, Cc / 128);
-    p.splits = (int)std::min<int64_t>(
-        std::max<int64_t>(1, plan_cdiv(target, p.oblocks * batch)), max_split);
-  } else if (band_xr) {
-    p.kernel = band_xr == 16 ? GemvKernel::kBand16 : GemvKernel::kBand8;
-    p.oblocks = plan_cdiv(Cc, kBandCols);
-    p.splits = (int)plan_cdiv(R, (int64_t)band_xr * kGemvThreads * vn);
+    p.oblocks = pblocks;
+    // Otherwise splits of at least 8 columns for each of four waves.
+    if (short_sums)
+      p.waves = 16;
+    else
+      p.splits = (int)std::min<int64_t>(
+          plan_cdiv(target, p.oblocks * batch),
+          std::min<int64_t>(256, std::max<int64_t>(1, Cc / 32)));
   } else {
     p.kernel = GemvKernel::kColumn;
     p.oblocks = plan_cdiv(Cc, kColsPerBlock);
     const int64_t rsteps = plan_cdiv(R, 64 * (vec ? vn : 1));
     const int64_t max_split = std::max<int64_t>(1, rsteps / 16);
     p.splits = (int)std::min<int64_t>(
-        std::max<int64_t>(1, plan_cdiv(target, p.oblocks * batch)), max_split);
+        std::max<int64_t>(1, plan_cdiv(target, p.oblocks * batch)),
+        std::min<int64_t>(256, max_split));
   }
-  if (!band_xr && !bandn && p.splits > 256) p.splits = 256;
   if (p.splits > 1)
     p.partial_bytes = esize * (size_t)p.splits * (size_t)len_y *
                       (size_t)std::min<int64_t>(batch, 65535);

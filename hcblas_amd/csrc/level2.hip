@@ -21,6 +21,8 @@
 // that indexes storage columns; with v = x, w = y for column-major and
 // v = y, w = x for row-major this is bit-identical to CBLAS (netlib
 // "temp = alpha*y(j); a(i,j) += x(i)*temp", row-major by argument swap).
+#include <type_traits>
+
 #include "common.hpp"
 #include "gemv_plan.hpp"
 
@@ -33,16 +35,22 @@ static_assert(kThreads == kGemvThreads, "plan and kernels agree");
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef double d2v __attribute__((ext_vector_type(2)));
 
+// 16 bytes of T. `type` for registers and the library's own buffers; `any` for
+// the caller's operands, at any multiple of the element size: gfx950 serves a
+// global_load / store_dwordx4 at any address, so an odd leading dimension,
+// offset or row count does not leave the vector path.
 template <typename T>
 struct VecT;
 template <>
 struct VecT<float> {
   using type = f4v;
+  typedef f4v any __attribute__((aligned(4)));
   static constexpr int n = 4;
 };
 template <>
 struct VecT<double> {
   using type = d2v;
+  typedef d2v any __attribute__((aligned(8)));
   static constexpr int n = 2;
 };
 
@@ -52,19 +60,21 @@ __device__ __forceinline__ T vlane(const typename VecT<T>::type &v, int i) {
 }
 
 // 16-byte load, non-temporal when NT (operands far larger than the caches).
-template <bool NT, typename V>
-__device__ __forceinline__ V vld(const V *p) {
+template <bool NT, typename T>
+__device__ __forceinline__ typename VecT<T>::type vld(const T *p) {
+  using A = typename VecT<T>::any;
   if constexpr (NT)
-    return __builtin_nontemporal_load(p);
+    return __builtin_nontemporal_load(reinterpret_cast<const A *>(p));
   else
-    return *p;
+    return *reinterpret_cast<const A *>(p);
 }
-template <bool NT, typename V>
-__device__ __forceinline__ void vst(V *p, V v) {
+template <bool NT, typename T>
+__device__ __forceinline__ void vst(T *p, typename VecT<T>::type v) {
+  using A = typename VecT<T>::any;
   if constexpr (NT)
-    __builtin_nontemporal_store(v, p);
+    __builtin_nontemporal_store(v, reinterpret_cast<A *>(p));
   else
-    *p = v;
+    *reinterpret_cast<A *>(p) = v;
 }
 
 // Operands at least this large (bytes) are streamed non-temporally.
@@ -110,55 +120,68 @@ __device__ __forceinline__ void store_y(T *y, T sum, T alpha, T beta) {
 
 // Split reductions: every workgroup stores its partial sums with plain
 // stores to part[split][output], and gemv_finish_kernel, launched next on the
-// same stream, adds them (sixteen running sums over the splits k = j mod 16,
-// combined as a fixed tree, so sixteen loads per thread are in flight: SGEMV-N
-// 16384^2 6846 GB/s against 6753 with eight) and writes y; the order is
-// fixed, so results are deterministic. (An in-kernel
-// last-arriver reduction needs an agent-scope release per workgroup, which on
-// a multi-XCD MI355X is an L2 write-back each: measured 5.1 against 6.4 TB/s
-// for SGEMV-N 16384^2 with 1024 workgroups.)
+// same stream, adds them and writes y. A workgroup takes 64 outputs and its
+// four waves every fourth split, eight loads in flight per thread; the order
+// is fixed, so results are deterministic. (An in-kernel last-arriver reduction
+// needs an agent-scope release per workgroup, which on a multi-XCD MI355X is
+// an L2 write-back each: measured 5.1 against 6.4 TB/s for SGEMV-N 16384^2
+// with 1024 workgroups.)
 template <typename T>
 __global__ __launch_bounds__(kThreads) void gemv_finish_kernel(
     int64_t len_y, int splits, const T *__restrict__ part, int64_t spart,
     T *y, int64_t incy, int64_t sy, T alpha, T beta) {
+  __shared__ T red[4][64];
   const int64_t z = blockIdx.z;
   part += z * spart;
   y += z * sy;
-  for (int64_t o = (int64_t)blockIdx.x * kThreads + threadIdx.x; o < len_y;
-       o += (int64_t)gridDim.x * kThreads) {
-    T s[16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int64_t o0 = (int64_t)blockIdx.x * 64; o0 < len_y;
+       o0 += (int64_t)gridDim.x * 64) {
+    const int64_t o = o0 + lane < len_y ? o0 + lane : len_y - 1;
+    T s[8];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) s[j] = T(0);
-    int k = 0;
-    for (; k + 16 <= splits; k += 16) {
+    for (int j = 0; j < 8; ++j) s[j] = T(0);
+    int k = wave;
+    for (; k + 28 < splits; k += 32) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) s[j] += part[(int64_t)(k + j) * len_y + o];
+      for (int j = 0; j < 8; ++j)
+        s[j] += part[(int64_t)(k + 4 * j) * len_y + o];
     }
-    for (int j = 0; k < splits; ++k, ++j) s[j] += part[(int64_t)k * len_y + o];
 #pragma unroll
-    for (int w = 8; w >= 1; w >>= 1)
+    for (int j = 0; j < 7; ++j)
+      if (k + 4 * j < splits) s[j] += part[(int64_t)(k + 4 * j) * len_y + o];
+#pragma unroll
+    for (int w = 4; w >= 1; w >>= 1)
 #pragma unroll
       for (int j = 0; j < w; ++j) s[j] = s[j] + s[j + w];
-    store_y(&y[bidx(o, len_y, incy)], s[0], alpha, beta);
+    red[wave][lane] = s[0];
+    __syncthreads();
+    if (wave == 0 && o0 + lane < len_y)
+      store_y(&y[bidx(o, len_y, incy)],
+              (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]),
+              alpha, beta);
+    __syncthreads();
   }
 }
 
 // ---------------------------------------------------------------------------
-// Panel kernel: y[r] = alpha * sum_c S[r,c] x[c] + beta*y[r].
-// Workgroup = 4 waves over the same 64*VN rows (one 16-byte vector per lane);
-// the waves interleave the workgroup's columns (c = c0 + wave + 4u) with U
-// loads in flight per lane, and LDS sums the four waves. blockIdx.y splits the
-// columns across workgroups. (Measured on MI355X: 6.4 TB/s at 16384^2 fp32,
-// against 3.5 TB/s for one wave per row band walking all columns.)
+// Panel kernel: y[r] = alpha * sum_c S[r,c] x[c] + beta*y[r], for fewer rows
+// than a band. Workgroup = NW waves over the same 64*VN rows (one 16-byte
+// vector per lane); the waves interleave the workgroup's columns
+// (c = c0 + wave + NW u) with U loads in flight per lane, and LDS sums the
+// waves. blockIdx.y splits the columns across workgroups. Sixteen waves and no
+// split serve small matrices in one launch. The last vector of a row count
+// that is not a whole number of vectors is read from row R - VN on, and its
+// lane stores only the rows that no other lane has.
 // ---------------------------------------------------------------------------
-template <typename T, bool VEC, bool NT>
-__global__ __launch_bounds__(kThreads) void gemv_panel_kernel(
+template <typename T, bool VEC, bool NT, int NW>
+__global__ __launch_bounds__(64 * NW) void gemv_panel_kernel(
     GemvShape s, const T *__restrict__ A, const T *__restrict__ x, T *y,
     T alpha, T beta, T *part) {
   constexpr int VN = VEC ? VecT<T>::n : 1;
-  constexpr int ROWS = 64 * VN;
-  constexpr int U = 8;
-  __shared__ T red[4][ROWS];
+  constexpr int ROWS = 64 * VN, TH = 64 * NW;
+  constexpr int U = NW == 16 ? 16 : 8;
+  __shared__ T red[NW][ROWS];
   const int64_t z = blockIdx.z;
   A += z * s.sA;
   x += z * s.sx;
@@ -173,80 +196,84 @@ __global__ __launch_bounds__(kThreads) void gemv_panel_kernel(
   const int64_t cper = cdiv_dev(s.Cc, s.splits);
   const int64_t c_begin = split * cper;
   const int64_t c_end = c_begin + cper < s.Cc ? c_begin + cper : s.Cc;
+  // Rows this lane reads: r0 .. or, at the edge, the last VN.
+  const int64_t rr = r0 + VN <= s.R ? r0 : s.R - VN;
 
   T acc[VN];
 #pragma unroll
   for (int e = 0; e < VN; ++e) acc[e] = T(0);
 
-  if (r0 < s.R) {  // on the vector path R % VN == 0
-    const T *col = A + r0;
+  if (r0 < s.R) {
+    const T *col = A + rr;
     int64_t c = c_begin + wave;
     if constexpr (VEC) {
       using V = typename VecT<T>::type;
-      for (; c + 4 * (U - 1) < c_end; c += 4 * U) {
-        V a[U];
-        T xv[U];
+      // N of the wave's columns from c: all loads, then all FMAs. (A last
+      // trip of U with the missing columns masked was slower: 9000 x 300 fp32
+      // 9.3 us against 6.9.)
+      auto columns = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        V a[N];
+        T xv[N];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          a[u] = vld<NT>(reinterpret_cast<const V *>(col + (c + 4 * u) * s.ld));
-          xv[u] = x[bidx(c + 4 * u, s.Cc, s.incx)];
+        for (int u = 0; u < N; ++u) {
+          a[u] = vld<NT>(col + (c + NW * u) * s.ld);
+          xv[u] = x[bidx(c + NW * u, s.Cc, s.incx)];
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < N; ++u)
 #pragma unroll
           for (int e = 0; e < VN; ++e) acc[e] = fma_t(a[u][e], xv[u], acc[e]);
-      }
-      for (; c < c_end; c += 4) {
-        const V a = vld<NT>(reinterpret_cast<const V *>(col + c * s.ld));
-        const T xv = x[bidx(c, s.Cc, s.incx)];
-#pragma unroll
-        for (int e = 0; e < VN; ++e) acc[e] = fma_t(a[e], xv, acc[e]);
-      }
+        c += NW * N;
+      };
+      while (c + NW * (U - 1) < c_end) columns(std::integral_constant<int, U>{});
+      while (c + NW * 3 < c_end) columns(std::integral_constant<int, 4>{});
+      while (c < c_end) columns(std::integral_constant<int, 1>{});
     } else {
-      for (; c < c_end; c += 4)
+      for (; c < c_end; c += NW)
         acc[0] = fma_t(col[c * s.ld], x[bidx(c, s.Cc, s.incx)], acc[0]);
     }
-  }
 #pragma unroll
-  for (int e = 0; e < VN; ++e) red[wave][lane * VN + e] = acc[e];
-  __syncthreads();
-  // Four-wave sum, in wave order, into red[0].
-  for (int i = threadIdx.x; i < ROWS; i += kThreads)
-    red[0][i] = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
-  __syncthreads();
-  if (s.splits == 1) {
-    for (int i = threadIdx.x; i < ROWS; i += kThreads)
-      if (rb + i < s.R)
-        store_y(&y[bidx(rb + i, s.R, s.incy)], red[0][i], alpha, beta);
-    return;
+    for (int e = 0; e < VN; ++e)
+      if (rr + e >= r0) red[wave][rr + e - rb] = acc[e];
   }
+  __syncthreads();
+  // Sum of the waves in wave order.
   T *pp = part + (z * s.splits + split) * s.R;
-  for (int i = threadIdx.x; i < ROWS; i += kThreads)
-    if (rb + i < s.R) pp[rb + i] = red[0][i];
+  for (int i = threadIdx.x; i < ROWS && rb + i < s.R; i += TH) {
+    T v = red[0][i];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += red[w][i];
+    if (s.splits == 1)
+      store_y(&y[bidx(rb + i, s.R, s.incy)], v, alpha, beta);
+    else
+      pp[rb + i] = v;
+  }
 }
 
 // ---------------------------------------------------------------------------
-// Band-N kernel: the panel kernel's job for operands with R >= 1024*VN*4.
-// Workgroup = (one band of XR*256*VN rows, one block of columns): the band's
-// sums stay in registers (XR vectors per thread) while the workgroup walks
-// its columns UC at a time, each column's band being one contiguous run
-// (16 KiB) read by all 256 threads; x[c] is wave-uniform (scalar loads). The
-// loads of UC columns are all issued before their FMAs (a scheduling barrier
-// keeps the compiler from interleaving them one by one). Column blocks are
-// sized so that bands x blocks is about one workgroup per CU with at least
-// 256 columns per block, so the partials cost at most 2/256 of the traffic.
-// Measured on MI355X at 16384^2: 155 us fp32 (6.9 TB/s) and 308 us fp64
-// against 166 / 315 us for the panel kernel. Rows of a partial last band
-// load a clamped row (the band's first) and are never stored.
+// Band-N kernel: the panel kernel's job for operands of at least three
+// quarters of a band of 256*VN rows. Workgroup = (one band of XR*256*VN rows,
+// one block of columns): the band's sums stay in registers (XR vectors per
+// thread) while the workgroup walks its columns UC at a time, each column's
+// band being one contiguous run (XR * 4 KiB) read by all 256 threads; x[c] is
+// wave-uniform (scalar loads). The loads of UC columns (32 per thread) are all
+// issued before their FMAs (a scheduling barrier keeps the compiler from
+// interleaving them one by one). Column blocks are sized so that bands x
+// blocks is about one workgroup per CU with at least 32 columns per block, so
+// the partials cost at most 2/32 of the traffic (XR = 4 bands of a large
+// matrix: 2/256). Measured on MI355X at 16384^2: 155 us fp32 (6.9 TB/s) and
+// 308 us fp64 against 166 / 315 us for the panel kernel. Lanes past the edge
+// read the last VN rows; the rows no other lane has are stored.
 // ---------------------------------------------------------------------------
 
-template <typename T, bool NT>
+template <typename T, int XR, bool NT>
 __global__ __launch_bounds__(kThreads) void gemv_bandn_kernel(
     GemvShape s, const T *__restrict__ A, const T *__restrict__ x, T *y,
     T alpha, T beta, T *part) {
   using V = typename VecT<T>::type;
   constexpr int VN = VecT<T>::n;
-  constexpr int XR = kBandNRows, UC = kBandNCols;
+  constexpr int UC = 32 / XR;
   constexpr int64_t STEP = (int64_t)kThreads * VN;
   const int64_t z = blockIdx.z;
   A += z * s.sA;
@@ -255,13 +282,13 @@ __global__ __launch_bounds__(kThreads) void gemv_bandn_kernel(
   // blockIdx.x walks the column blocks and blockIdx.y the bands: consecutive
   // workgroups (spread over the XCDs in turn) then share a band (measured
   // 155 against 164 us at 16384^2 fp32 with the axes swapped).
-  const int64_t r_begin = (int64_t)blockIdx.y * XR * STEP;
-  const int64_t rt = r_begin + (int64_t)threadIdx.x * VN;
+  const int64_t rt = (int64_t)blockIdx.y * XR * STEP +
+                     (int64_t)threadIdx.x * VN;
   int64_t roff[XR];
 #pragma unroll
   for (int u = 0; u < XR; ++u) {
     const int64_t r = rt + u * STEP;
-    roff[u] = r < s.R ? r : r_begin;  // R % VN == 0: wholly in or out
+    roff[u] = r + VN <= s.R ? r : s.R - VN;
   }
   const int split = blockIdx.x;
   const int64_t cper = cdiv_dev(s.Cc, s.splits);
@@ -273,49 +300,51 @@ __global__ __launch_bounds__(kThreads) void gemv_bandn_kernel(
 #pragma unroll
     for (int e = 0; e < VN; ++e) acc[u][e] = T(0);
   int64_t c = c_begin;
-  for (; c + UC <= c_end; c += UC) {
-    V a[UC][XR];
-    T xv[UC];
+  // N columns from c: all loads, then all FMAs.
+  auto columns = [&](auto n) {
+    constexpr int N = decltype(n)::value;
+    V a[N][XR];
+    T xv[N];
 #pragma unroll
-    for (int j = 0; j < UC; ++j) {
+    for (int j = 0; j < N; ++j) {
       xv[j] = x[bidx(c + j, s.Cc, s.incx)];
       const T *col = A + (c + j) * s.ld;
 #pragma unroll
-      for (int u = 0; u < XR; ++u)
-        a[j][u] = vld<NT>(reinterpret_cast<const V *>(col + roff[u]));
+      for (int u = 0; u < XR; ++u) a[j][u] = vld<NT>(col + roff[u]);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < UC; ++j)
+    for (int j = 0; j < N; ++j)
 #pragma unroll
       for (int u = 0; u < XR; ++u)
 #pragma unroll
         for (int e = 0; e < VN; ++e)
           acc[u][e] = fma_t(vlane<T>(a[j][u], e), xv[j], acc[u][e]);
-  }
-  for (; c < c_end; ++c) {
-    const T xv = x[bidx(c, s.Cc, s.incx)];
-    const T *col = A + c * s.ld;
-#pragma unroll
-    for (int u = 0; u < XR; ++u) {
-      const V a = vld<NT>(reinterpret_cast<const V *>(col + roff[u]));
-#pragma unroll
-      for (int e = 0; e < VN; ++e) acc[u][e] = fma_t(vlane<T>(a, e), xv, acc[u][e]);
-    }
-  }
+    c += N;
+  };
+  while (c + UC <= c_end) columns(std::integral_constant<int, UC>{});
+  while (c + 4 <= c_end) columns(std::integral_constant<int, 4>{});
+  while (c < c_end) columns(std::integral_constant<int, 1>{});
 #pragma unroll
   for (int u = 0; u < XR; ++u) {
     const int64_t r = rt + u * STEP;
     if (r >= s.R) continue;
-    if (s.splits == 1) {
-#pragma unroll
-      for (int e = 0; e < VN; ++e)
-        store_y(&y[bidx(r + e, s.R, s.incy)], acc[u][e], alpha, beta);
-    } else {
+    T *pp = part + (z * s.splits + split) * s.R;
+    if (s.splits > 1 && r + VN <= s.R) {
       V v;
 #pragma unroll
       for (int e = 0; e < VN; ++e) v[e] = acc[u][e];
-      *reinterpret_cast<V *>(part + (z * s.splits + split) * s.R + r) = v;
+      vst<false>(pp + r, v);
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < VN; ++e) {
+      const int64_t re = roff[u] + e;
+      if (re < r) continue;
+      if (s.splits == 1)
+        store_y(&y[bidx(re, s.R, s.incy)], acc[u][e], alpha, beta);
+      else
+        pp[re] = acc[u][e];
     }
   }
 }
@@ -362,20 +391,20 @@ __global__ __launch_bounds__(kThreads) void gemv_column_kernel(
     cols[j] = A + (colok[j] ? (cbase + j) : 0) * s.ld;
   }
 
-  if (VEC) {
+  if constexpr (VEC) {
     using V = typename VecT<T>::type;
     const bool xunit = s.incx == 1;
     int64_t r = r_begin + lane_id * VN;
     if (xunit) {
       // Two row steps per iteration: 2 * kCPW loads of A in flight per lane.
-      for (; r + step < r_end; r += 2 * step) {
-        const V t0 = *reinterpret_cast<const V *>(x + r);
-        const V t1 = *reinterpret_cast<const V *>(x + r + step);
+      for (; r + step + VN <= r_end; r += 2 * step) {
+        const V t0 = vld<false>(x + r);
+        const V t1 = vld<false>(x + r + step);
         V a0[kCPW], a1[kCPW];
 #pragma unroll
         for (int j = 0; j < kCPW; ++j) {
-          a0[j] = vld<NT>(reinterpret_cast<const V *>(cols[j] + r));
-          a1[j] = vld<NT>(reinterpret_cast<const V *>(cols[j] + r + step));
+          a0[j] = vld<NT>(cols[j] + r);
+          a1[j] = vld<NT>(cols[j] + r + step);
         }
 #pragma unroll
         for (int j = 0; j < kCPW; ++j) {
@@ -390,22 +419,21 @@ __global__ __launch_bounds__(kThreads) void gemv_column_kernel(
       }
     }
     for (; r < r_end; r += step) {
-      // On this path R % VN == 0, so a vector never straddles R.
+      // A vector that reaches past R is read from R - VN on; the rows below r
+      // belong to another lane and count as zeros here.
+      const int64_t rr = r + VN <= s.R ? r : s.R - VN;
       T xv[VN];
-      if (xunit) {
-        const V t = *reinterpret_cast<const V *>(x + r);
 #pragma unroll
-        for (int e = 0; e < VN; ++e) xv[e] = vlane<T>(t, e);
-      } else {
-#pragma unroll
-        for (int e = 0; e < VN; ++e) xv[e] = x[bidx(r + e, s.R, s.incx)];
-      }
+      for (int e = 0; e < VN; ++e)
+        xv[e] = rr + e >= r ? x[bidx(rr + e, s.R, s.incx)] : T(0);
 #pragma unroll
       for (int j = 0; j < kCPW; ++j) {
         if (!colok[j]) continue;
-        const V a = vld<NT>(reinterpret_cast<const V *>(cols[j] + r));
+        const V a = vld<NT>(cols[j] + rr);
 #pragma unroll
-        for (int e = 0; e < VN; ++e) acc[j][e] = fma_t(vlane<T>(a, e), xv[e], acc[j][e]);
+        for (int e = 0; e < VN; ++e)
+          acc[j][e] = fma_t(rr + e >= r ? vlane<T>(a, e) : T(0), xv[e],
+                            acc[j][e]);
       }
     }
   } else {
@@ -444,17 +472,16 @@ __global__ __launch_bounds__(kThreads) void gemv_column_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Band kernel: the column kernel's job for tall operands (R >= XR*256*VN).
-// Workgroup = (CPB consecutive columns, one band of XR*256*VN rows). The
-// band's x is loaded once into registers (thread t keeps the vectors at rows
-// t*VN + u*256*VN, u < XR) and each column is then one contiguous run of the
-// band read by all 256 threads, XR 16-byte loads per thread in flight with no
-// x traffic. The CPB per-thread sums are reduced once at the end (wave
-// shuffles, then the four waves in order). Measured on MI355X at 16384^2:
+// Band kernel: the column kernel's job for operands of at least three
+// quarters of a row step of 256*VN. Workgroup = (CPB consecutive columns, one
+// band of XR row steps). The band's x is loaded once into registers (thread t
+// keeps the vectors at rows t*VN + u*256*VN, u < XR) and each column is then
+// one contiguous run of the band read by all 256 threads, with no x traffic
+// and at least 16 loads per thread in flight (short bands read several
+// columns together). A column's sum crosses the wave by shuffles while the next
+// columns load, and the four waves are added at the end in order. Measured on MI355X at 16384^2:
 // 6.9 TB/s fp32 and 7.0 TB/s fp64, against 6.2 / 6.5 for the column kernel,
 // whose four columns per wave and per-step x loads cost bandwidth.
-// Bands past the first full ones (R not a multiple of the band) load from a
-// clamped row (the band's first) with x = 0, so every load stays unpredicated.
 // ---------------------------------------------------------------------------
 
 template <typename T, int XR, bool NT>
@@ -464,6 +491,8 @@ __global__ __launch_bounds__(kThreads) void gemv_band_kernel(
   using V = typename VecT<T>::type;
   constexpr int VN = VecT<T>::n;
   constexpr int CPB = kBandCols;
+  // Columns read together: at least 16 vectors in flight per thread.
+  constexpr int CG = XR >= 12 ? 1 : XR >= 6 ? 2 : XR >= 3 ? 4 : 8;
   constexpr int64_t STEP = (int64_t)kThreads * VN;
   __shared__ T red[4][CPB];
   const int64_t z = blockIdx.z;
@@ -474,39 +503,55 @@ __global__ __launch_bounds__(kThreads) void gemv_band_kernel(
   const int64_t r_begin = (int64_t)split * XR * STEP;
   const int64_t rt = r_begin + (int64_t)threadIdx.x * VN;
   const bool full = r_begin + XR * STEP <= s.R;
+  // Lanes past the edge read the last VN rows; rows that another lane (or
+  // none) has count as zeros, in x and in A.
+  auto row = [&](int u) {
+    const int64_t r = rt + u * STEP;
+    return full || r + VN <= s.R ? r : s.R - VN;
+  };
   V xr[XR];
 #pragma unroll
   for (int u = 0; u < XR; ++u) {
-    const int64_t r = rt + u * STEP;
-    if (r >= s.R) {  // R % VN == 0: a vector is wholly in or out
-      xr[u] = V{};
-    } else if (s.incx == 1) {
-      xr[u] = *reinterpret_cast<const V *>(x + r);
+    const int64_t rr = row(u);
+    if (s.incx == 1) {
+      xr[u] = vld<false>(x + rr);
     } else {
 #pragma unroll
-      for (int e = 0; e < VN; ++e) xr[u][e] = x[bidx(r + e, s.R, s.incx)];
+      for (int e = 0; e < VN; ++e) xr[u][e] = x[bidx(rr + e, s.R, s.incx)];
+    }
+    if (!full) {
+#pragma unroll
+      for (int e = 0; e < VN; ++e)
+        if (rr + e < rt + u * STEP) xr[u][e] = T(0);
     }
   }
   const int64_t c0 = (int64_t)blockIdx.x * CPB;
-  T sums[CPB];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  V a[CG][XR];
+  auto load = [&](int j0) {
 #pragma unroll
-  for (int j = 0; j < CPB; ++j) {
-    const int64_t c = c0 + j;
-    T t = T(0);
-    if (c < s.Cc) {
+    for (int j = 0; j < CG; ++j) {
+      // (columns past the last read the last one; their sums are dropped)
+      const int64_t c = c0 + j0 + j < s.Cc ? c0 + j0 + j : s.Cc - 1;
       const T *col = A + c * s.ld;
-      V a[XR];
-      if (full) {
+#pragma unroll
+      for (int u = 0; u < XR; ++u) a[j][u] = vld<NT>(col + row(u));
+    }
+  };
+  load(0);
+  // A rolled loop: one group's vectors in registers, the next group's loads in
+  // flight while this group's sums cross the wave.
+#pragma unroll 1
+  for (int j0 = 0; j0 < CPB; j0 += CG) {
+    T t[CG];
+#pragma unroll
+    for (int j = 0; j < CG; ++j) {
+      if (!full) {
 #pragma unroll
         for (int u = 0; u < XR; ++u)
-          a[u] = vld<NT>(reinterpret_cast<const V *>(col + rt + u * STEP));
-      } else {
 #pragma unroll
-        for (int u = 0; u < XR; ++u) {
-          const int64_t r = rt + u * STEP;
-          a[u] = vld<NT>(
-              reinterpret_cast<const V *>(col + (r < s.R ? r : r_begin)));
-        }
+          for (int e = 0; e < VN; ++e)
+            if (row(u) + e < rt + u * STEP) a[j][u][e] = T(0);
       }
       T acc[VN];
 #pragma unroll
@@ -515,17 +560,17 @@ __global__ __launch_bounds__(kThreads) void gemv_band_kernel(
       for (int u = 0; u < XR; ++u)
 #pragma unroll
         for (int e = 0; e < VN; ++e)
-          acc[e] = fma_t(vlane<T>(a[u], e), vlane<T>(xr[u], e), acc[e]);
+          acc[e] = fma_t(vlane<T>(a[j][u], e), vlane<T>(xr[u], e), acc[e]);
+      t[j] = T(0);
 #pragma unroll
-      for (int e = 0; e < VN; ++e) t += acc[e];
+      for (int e = 0; e < VN; ++e) t[j] += acc[e];
     }
-    sums[j] = t;
-  }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (j0 + CG < CPB) load(j0 + CG);
 #pragma unroll
-  for (int j = 0; j < CPB; ++j) {
-    const T v = wave_sum(sums[j]);
-    if (lane == 0) red[wave][j] = v;
+    for (int j = 0; j < CG; ++j) {
+      const T v = wave_sum(t[j]);
+      if (lane == 0) red[wave][j0 + j] = v;
+    }
   }
   __syncthreads();
   if (threadIdx.x >= CPB) return;
@@ -577,7 +622,7 @@ __global__ __launch_bounds__(kThreads) void ger_kernel(
   for (int e = 0; e < VN; ++e)
     vr[e] = (r0 + e < R) ? v[bidx(r0 + e, R, incv)] : T(0);
   const int64_t cend = c0 + kGerCols < Cc ? c0 + kGerCols : Cc;
-  if (VEC) {
+  if (VEC && r0 + VN <= R) {
     using V = typename VecT<T>::type;
     if (cend - c0 == kGerCols) {
       // Every load is issued before the first store, so kGerCols loads are
@@ -585,39 +630,31 @@ __global__ __launch_bounds__(kThreads) void ger_kernel(
       // behind them: the compiler cannot prove the columns disjoint).
       V a[kGerCols];
 #pragma unroll
-      for (int j = 0; j < kGerCols; ++j) {
-        const V *p = reinterpret_cast<const V *>(A + r0 + (c0 + j) * ld);
-        if constexpr (NT)
-          a[j] = __builtin_nontemporal_load(p);
-        else
-          a[j] = *p;
-      }
+      for (int j = 0; j < kGerCols; ++j) a[j] = vld<NT>(A + r0 + (c0 + j) * ld);
 #pragma unroll
       for (int j = 0; j < kGerCols; ++j) {
         const T t = alpha * w[bidx(c0 + j, Cc, incw)];
 #pragma unroll
         for (int e = 0; e < VN; ++e) a[j][e] = fma_t(vr[e], t, a[j][e]);
-        V *p = reinterpret_cast<V *>(A + r0 + (c0 + j) * ld);
-        if constexpr (NT)
-          __builtin_nontemporal_store(a[j], p);
-        else
-          *p = a[j];
+        vst<NT>(A + r0 + (c0 + j) * ld, a[j]);
       }
       return;
     }
     for (int64_t c = c0; c < cend; ++c) {
       const T t = alpha * w[bidx(c, Cc, incw)];
-      V *p = reinterpret_cast<V *>(A + r0 + c * ld);
-      V a = *p;
+      V a = vld<false>(A + r0 + c * ld);
 #pragma unroll
       for (int e = 0; e < VN; ++e) a[e] = fma_t(vr[e], t, a[e]);
-      *p = a;
+      vst<false>(A + r0 + c * ld, a);
     }
   } else {
     for (int64_t c = c0; c < cend; ++c) {
       const T t = alpha * w[bidx(c, Cc, incw)];
-      T *p = A + r0 + c * ld;
-      *p = fma_t(vr[0], t, *p);
+#pragma unroll
+      for (int e = 0; e < VN; ++e) {
+        T *p = A + r0 + e + c * ld;
+        if (r0 + e < R) *p = fma_t(vr[e], t, *p);
+      }
     }
   }
 }
@@ -625,6 +662,16 @@ __global__ __launch_bounds__(kThreads) void ger_kernel(
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+template <typename T, int NW>
+void launch_panel(dim3 grid, hipStream_t stream, bool vec, bool nt,
+                  const GemvShape &s, const T *A, const T *x, T *y, T alpha,
+                  T beta, T *part) {
+  (!vec ? gemv_panel_kernel<T, false, false, NW>
+   : nt ? gemv_panel_kernel<T, true, true, NW>
+        : gemv_panel_kernel<T, true, false, NW>)
+      <<<grid, 64 * NW, 0, stream>>>(s, A, x, y, alpha, beta, part);
+}
+
 template <typename T>
 hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
                         T alpha, const T *A, int64_t ld, const T *x,
@@ -643,23 +690,24 @@ hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
     return launch_status();
   }
   constexpr int VN = VecT<T>::n;
-  // 16-byte path: aligned base, leading dimension and rows a multiple of VN,
-  // and batch strides that keep every problem's A (and x, where the column
-  // kernels read it as vectors) 16-byte aligned.
-  const bool xvec = !panel && incx == 1;
-  const bool vec = aligned16(A) && (ld % VN == 0) && (R % VN == 0) &&
-                   (!xvec || aligned16(x)) &&
-                   (batch == 1 || (sA % VN == 0 && (!xvec || sx % VN == 0)));
+  // Rows are read 16 bytes at a time unless there is not even one vector.
+  bool vec = R >= VN;
   const bool nt = (int64_t)sizeof(T) * R * Cc * batch >= kStreamBytes;
   GemvShape s{R, Cc, ld, incx, incy, sA, sx, sy, 1};
-  const GemvPlan plan =
+  GemvPlan plan =
       plan_gemv(h->num_cus, panel, R, Cc, vec, VN, sizeof(T), batch);
+  // Bands of a matrix of more than about 80 GB can need more partials than
+  // the allocation-free entry's scratch holds. Where the operands are not
+  // 16-byte aligned both entries then read by elements, whose splits fit.
+  if (batch == 1 && plan.partial_bytes > kNoAllocScratchBytes &&
+      (!aligned16(A) || ld % VN || R % VN ||
+       (!panel && incx == 1 && !aligned16(x)))) {
+    vec = false;
+    plan = plan_gemv(h->num_cus, panel, R, Cc, vec, VN, sizeof(T), batch);
+  }
   s.splits = plan.splits;
   const int64_t oblocks = plan.oblocks;
   const bool bandn = plan.kernel == GemvKernel::kBandN;
-  const int band_xr = plan.kernel == GemvKernel::kBand16  ? 16
-                      : plan.kernel == GemvKernel::kBand8 ? 8
-                                                          : 0;
   T *part = nullptr;
   if (s.splits > 1) {
     if (fixed_part) {
@@ -680,50 +728,59 @@ hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
     const T *Ab = A + b0 * sA;
     const T *xb = x + b0 * sx;
     T *yb = y + b0 * sy;
-    if (bandn) {
-      if (nt)
-        gemv_bandn_kernel<T, true><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else
-        gemv_bandn_kernel<T, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-    } else if (panel) {
-      if (vec && nt)
-        gemv_panel_kernel<T, true, true><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else if (vec)
-        gemv_panel_kernel<T, true, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else
-        gemv_panel_kernel<T, false, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-    } else if (band_xr == 16) {
-      if (nt)
-        gemv_band_kernel<T, 16, true><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else
-        gemv_band_kernel<T, 16, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-    } else if (band_xr == 8) {
-      if (nt)
-        gemv_band_kernel<T, 8, true><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else
-        gemv_band_kernel<T, 8, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-    } else {
-      if (vec && nt)
-        gemv_column_kernel<T, true, true><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else if (vec)
-        gemv_column_kernel<T, true, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
-      else
-        gemv_column_kernel<T, false, false><<<grid, kThreads, 0, h->stream>>>(
-            s, Ab, xb, yb, alpha, beta, part);
+#define HCB_GEMV(KERNEL, TH, ...)                                          \
+  (nt ? KERNEL<T, __VA_ARGS__, true> : KERNEL<T, __VA_ARGS__, false>)      \
+      <<<grid, TH, 0, h->stream>>>(s, Ab, xb, yb, alpha, beta, part)
+#define HCB_BAND(XR)                                                       \
+  case XR:                                                                 \
+    HCB_GEMV(gemv_band_kernel, kThreads, XR);                              \
+    break
+    switch (plan.kernel) {
+      case GemvKernel::kBandN:
+        if (plan.xr == 4)
+          HCB_GEMV(gemv_bandn_kernel, kThreads, 4);
+        else if (plan.xr == 2)
+          HCB_GEMV(gemv_bandn_kernel, kThreads, 2);
+        else
+          HCB_GEMV(gemv_bandn_kernel, kThreads, 1);
+        break;
+      case GemvKernel::kPanel:
+        if (plan.waves == 16)
+          launch_panel<T, 16>(grid, h->stream, vec, nt, s, Ab, xb, yb, alpha,
+                              beta, part);
+        else
+          launch_panel<T, 4>(grid, h->stream, vec, nt, s, Ab, xb, yb, alpha,
+                             beta, part);
+        break;
+      case GemvKernel::kBand16:
+      case GemvKernel::kBand8:
+        switch (plan.xr) {
+          HCB_BAND(1);
+          HCB_BAND(2);
+          HCB_BAND(3);
+          HCB_BAND(4);
+          HCB_BAND(6);
+          HCB_BAND(8);
+          HCB_BAND(10);
+          HCB_BAND(12);
+          HCB_BAND(14);
+          HCB_BAND(16);
+          default:
+            return HCBLAS_STATUS_INTERNAL_ERROR;
+        }
+        break;
+      case GemvKernel::kColumn:
+        if (!vec)
+          gemv_column_kernel<T, false, false><<<grid, kThreads, 0, h->stream>>>(
+              s, Ab, xb, yb, alpha, beta, part);
+        else
+          HCB_GEMV(gemv_column_kernel, kThreads, true);
+        break;
     }
+#undef HCB_BAND
+#undef HCB_GEMV
     if (s.splits > 1) {
-      dim3 fg((unsigned)std::min<int64_t>(cdiv(len_y, kThreads), 1024), 1,
+      dim3 fg((unsigned)std::min<int64_t>(cdiv(len_y, 64), 4096), 1,
               (unsigned)nb);
       gemv_finish_kernel<T><<<fg, kThreads, 0, h->stream>>>(
           len_y, s.splits, part, (int64_t)s.splits * len_y, yb, incy, sy,
@@ -808,8 +865,7 @@ hcblasStatus_t ger_entry(hcblasHandle_t h, hcblasOrder_t order, int M, int N,
   const int64_t sv = col ? sxv : syv, sw = col ? syv : sxv;
   T *Ab = A + aOffset;
   constexpr int VN = VecT<T>::n;
-  const bool vec = aligned16(Ab) && (lda % VN == 0) && (R % VN == 0) &&
-                   (batch == 1 || sA % VN == 0);
+  const bool vec = R >= VN;
   const int64_t rows_per_block = (int64_t)kThreads * (vec ? VN : 1);
   // A matrix larger than the 256 MB last-level cache (MALL) streams through
   // with non-temporal accesses: caching it cannot keep it for the next call

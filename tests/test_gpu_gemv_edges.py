@@ -1,0 +1,99 @@
+"""GEMV and GER at the sizes where the launch plan changes kernel or band, on
+tightly packed matrices with any row count (the last vector of a column is
+read from row R - VN on), at odd element offsets, and with non-finite rows
+next to the edge.
+
+Bound against the FP64 value: the sum of L products in any order is within
+(L + 2) * eps * (|alpha| |A| |x| + |beta| |y|) componentwise, eps the unit of
+the type; GER is one fused multiply-add per element and bit-exact.
+"""
+import numpy as np
+import pytest
+
+from gpu_util import bitwise_equal, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+COL, ROW = 1, 0
+DT = {"s": np.float32, "d": np.float64}
+
+# Storage rows R and columns: below one vector; the panel kernel (sixteen
+# waves up to 512 columns, splits beyond); three quarters of a band step and
+# its neighbours; bands of 1, 2, 4 and 10 row steps with partial last bands;
+# few columns (short bands) and many.
+SHAPES = [(1, 40), (3, 700), (5, 33), (190, 511), (255, 513), (383, 129),
+          (385, 65), (767, 64), (769, 2050), (1021, 31), (1025, 300),
+          (2047, 1030), (4097, 77), (5003, 600), (8193, 130), (20011, 9),
+          (10007, 259)]
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+@pytest.mark.parametrize("trans", [0, 1])
+def test_plan_edges(hc, handle, p, trans):
+    dt = DT[p]
+    eps = np.finfo(dt).eps
+    for R, Cc in SHAPES:
+        rng = np.random.default_rng(R + Cc)
+        m = rng.uniform(-1, 1, (Cc, R)).astype(dt)  # column-major R x Cc
+        A = np.concatenate([np.full(1, 99, dt), m.ravel(), np.full(9, 99, dt)])
+        op = m if trans else m.T
+        ly, lx = op.shape
+        dA = to_dev(A)
+        for incx in (1, -2):
+            x = rng.uniform(-1, 1, lx).astype(dt)
+            xs = np.zeros(1 + (lx - 1) * abs(incx), dt)
+            xs[::abs(incx)] = x if incx > 0 else x[::-1]
+            y = rng.uniform(-1, 1, ly + 1).astype(dt)
+            dy = to_dev(y)
+            st = getattr(hc.api, f"hcblas_{p}gemv")(
+                handle, COL, trans, R, Cc, 1.5, dA, 1, R, to_dev(xs), 0, incx,
+                -0.5, dy, 1, 1)
+            assert st == 0
+            got = to_host(dy)
+            assert got[0] == y[0]
+            o, x64, y64 = op.astype(np.float64), x.astype(np.float64), y[1:]
+            ref = 1.5 * (o @ x64) - 0.5 * y64
+            bound = (lx + 2) * eps * (1.5 * (abs(o) @ abs(x64)) +
+                                      0.5 * abs(y64)) + eps * abs(ref)
+            assert np.all(abs(got[1:] - ref) <= bound), (R, Cc, incx)
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+def test_edge_rows_do_not_leak(hc, handle, p):
+    """An infinity in the rows that a moved last vector reads twice appears in
+    each sum once: the column sums are infinite, not NaN, and no other row's
+    sum sees it."""
+    dt = DT[p]
+    for R, Cc in [(5, 40), (259, 20), (1027, 24), (20011, 16)]:
+        m = np.ones((Cc, R), dt)
+        m[:, R - 2] = np.inf
+        y = to_dev(np.zeros(Cc, dt))
+        st = getattr(hc.api, f"hcblas{p.upper()}gemv")(
+            handle, 1, R, Cc, 1.0, to_dev(m), R, to_dev(np.ones(R, dt)), 1,
+            0.0, y, 1)
+        assert st == 0
+        assert np.all(to_host(y) == np.inf), (R, Cc)
+        y = to_dev(np.zeros(R, dt))
+        st = getattr(hc.api, f"hcblas{p.upper()}gemv")(
+            handle, 0, R, Cc, 1.0, to_dev(m), R, to_dev(np.ones(Cc, dt)), 1,
+            0.0, y, 1)
+        assert st == 0
+        exp = np.full(R, Cc, dt)
+        exp[R - 2] = np.inf
+        assert np.array_equal(to_host(y), exp), (R, Cc)
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+def test_ger_any_alignment(hc, handle, orc, p):
+    dt = DT[p]
+    for M, N in [(1, 17), (3, 16), (5, 33), (1023, 17), (1025, 40), (2051, 16)]:
+        rng = np.random.default_rng(M + N)
+        A = rng.uniform(-1, 1, M * N + 9).astype(dt)
+        x, y = rng.uniform(-1, 1, M).astype(dt), rng.uniform(-1, 1, N).astype(dt)
+        dA = to_dev(A)
+        st = getattr(hc.api, f"hcblas_{p}ger")(
+            handle, COL, M, N, 1.5, to_dev(x), 0, 1, to_dev(y), 0, 1, dA, 1, M)
+        assert st == 0
+        exp = A.copy()
+        exp[1:1 + M * N] = orc.ger(COL, M, N, 1.5, x, 1, y, 1,
+                                   A[1:1 + M * N].copy(), M)
+        assert bitwise_equal(to_host(dA), exp), (M, N)
