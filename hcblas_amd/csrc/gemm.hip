@@ -308,16 +308,15 @@ hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
   p.alpha = alpha;
   p.beta = beta;
   if (batch == 1 && !c.Aptrs && !c.Bptrs && !Cptrs) {
-    int ks = 0;
-    const int S = splitk_count(c.M, c.N, c.K, h->num_cus,
-                               E == Elem::F64 ? 16 : E == Elem::F32 ? 32 : 64,
-                               ks);
-    if (S > 1) {
-      const size_t bytes = sizeof(Acc) * (size_t)S * c.M * c.N;
+    const SplitK sk =
+        splitk_plan(c.M, c.N, c.K, h->num_cus, E == Elem::F64 ? 64 : 128,
+                    E == Elem::F64 ? 16 : E == Elem::F32 ? 32 : 64);
+    if (sk.splits > 1) {
+      const size_t bytes = sizeof(Acc) * (size_t)sk.splits * c.M * c.N;
       if (ensure_workspace(h->kpart_ws, bytes) != hipSuccess)
         return HCBLAS_STATUS_ALLOC_FAILED;
       return launch_gemm_splitk<E, OutT>(h->stream, h->num_cus, p, c.a_k,
-                                         c.b_k, S, ks,
+                                         c.b_k, sk,
                                          static_cast<Acc *>(h->kpart_ws.ptr));
     }
   }

@@ -22,7 +22,8 @@
 // Each tile runs the plain GEMM's main loop with the same K step and an
 // epilogue with the same arithmetic (staged through LDS so that C is written
 // with 16-byte column runs), so a grouped result is bit-identical to
-// per-problem hcblas_sgemm / hcblas_hgemm launches.
+// per-problem hcblas_sgemm / hcblas_hgemm launches (of K < 2048: beyond, those
+// may split K, which the grouped kernel never does).
 #include <algorithm>
 #include <cstring>
 #include <vector>

@@ -6,6 +6,6 @@ template hcblasStatus_t launch_gemm<Elem::F32, float>(hipStream_t, int,
                                                      GemmParams, bool, bool,
                                                      int64_t);
 template hcblasStatus_t launch_gemm_splitk<Elem::F32, float>(
-    hipStream_t, int, GemmParams, bool, bool, int, int,
+    hipStream_t, int, GemmParams, bool, bool, const SplitK &,
     typename ElemT<Elem::F32>::Acc *);
 }  // namespace hcb

@@ -6,6 +6,6 @@ template hcblasStatus_t launch_gemm<Elem::F64, double>(hipStream_t, int,
                                                      GemmParams, bool, bool,
                                                      int64_t);
 template hcblasStatus_t launch_gemm_splitk<Elem::F64, double>(
-    hipStream_t, int, GemmParams, bool, bool, int, int,
+    hipStream_t, int, GemmParams, bool, bool, const SplitK &,
     typename ElemT<Elem::F64>::Acc *);
 }  // namespace hcb

@@ -991,7 +991,15 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < MN;
        i += (int64_t)gridDim.x * 256) {
     Acc s = W[i];
-    for (int z = 1; z < S; ++z) s += W[(int64_t)z * MN + i];
+    int z = 1;
+    for (; z + 3 < S; z += 4) {  // four loads in flight, added in order
+      Acc w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = W[(int64_t)(z + j) * MN + i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s += w[j];
+    }
+    for (; z < S; ++z) s += W[(int64_t)z * MN + i];
     const int64_t n = i / M, m = i - n * M;
     OutT *dst = C + n * ldc + m;
     Acc v = alpha * s;

@@ -77,3 +77,17 @@ def test_every_residue_of_the_vector(hc, handle, p, order, ta, tb):
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_large_tiles_at_odd_sizes(hc, handle, p, M, N, K, ta, tb):
     _check(hc, handle, p, COL, ta, tb, M, N, K, 1, M + N + K)
+
+
+# Few tiles: 32x32 tiles with a short and a long K step (one of each type's
+# thresholds on either side), split K on 32x32 tiles (fewer of them than CUs)
+# and on 64x64 tiles, with slices that do not divide K.
+@pytest.mark.parametrize("p,M,N,K", [("s", 33, 65, 1023), ("s", 129, 31, 1100),
+                                     ("d", 33, 65, 511), ("d", 129, 31, 530),
+                                     ("h", 33, 65, 1023), ("h", 129, 31, 1100),
+                                     ("s", 35, 66, 2051), ("d", 35, 66, 2051),
+                                     ("h", 35, 66, 2051), ("s", 515, 513, 2057),
+                                     ("d", 515, 513, 2057), ("h", 515, 513, 2057)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_few_tiles(hc, handle, p, M, N, K, ta, tb):
+    _check(hc, handle, p, COL, ta, tb, M, N, K, 1, M + N + K)
