@@ -7,14 +7,16 @@
 //   sdot_HC    lib/src/blas/sdot/sdot_array.cpp:30-159    (host-side final sum)
 //   sasum_HC   lib/src/blas/sasum/sasum_array.cpp:30-143
 //
-// Design: every routine is HBM-bound. Unit-stride, 16-byte-aligned operands
-// take the vector path: one 16-byte vector per thread over a full grid
-// (measured on MI355X to stream faster than grid-stride loops), with
-// non-temporal loads / stores once the operands exceed the caches. Everything
-// else takes a scalar path that honours BLAS increments. dot / asum: each of
-// at most 256 workgroups reduces to an FP64 partial, and a one-workgroup
-// launch on the same stream sums the partials in index order (deterministic)
-// into the handle's pinned host block, whose sequence word the host polls.
+// Design: large calls are HBM-bound, small ones launch-bound. Unit-stride
+// operands, at any alignment, take the vector path in one launch: one 16-byte
+// vector per thread over a full grid (measured on MI355X to stream faster than
+// grid-stride loops), with non-temporal loads / stores once the operands exceed
+// the caches, and one more thread for the last, partial vector. Other
+// increments take a scalar path. dot / asum: each of at most 256 workgroups
+// reduces to an FP64 partial, and a one-workgroup launch on the same stream
+// sums the partials in index order (deterministic) into the handle's pinned
+// host block, whose sequence word the host polls; a short vector's only
+// workgroup publishes its sum itself.
 #include "common.hpp"
 
 namespace hcb {
@@ -31,36 +33,52 @@ constexpr int64_t kStreamBytes = 64ll << 20;
 // 2^28 SDOT (307 against 298 us).
 constexpr int kReduceUnroll = 4;
 constexpr int kReduceGrid = kReducePartials;
+// Trips of one workgroup's loads up to which it does a whole reduction alone:
+// a trip takes about 1 us, the finish launch that it saves 2 us on the GPU and
+// 3 us on the host (SDOT and SASUM of 4099 among three updates: the five calls
+// took 51 us with a finish launch each and a launch per vector tail, now 38).
+constexpr int kAloneTrips = 4;
+constexpr int kMaxGridY = 65535;
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef double d2v __attribute__((ext_vector_type(2)));
 
 template <typename T>
 struct V16;  // native 16-byte vector of T
+// (`any`: at any multiple of the element size; gfx950 serves a global_load /
+// store_dwordx4 at any address)
 template <>
 struct V16<float> {
   using type = f4v;
+  typedef f4v any __attribute__((aligned(4)));
   static constexpr int n = 4;
 };
 template <>
 struct V16<double> {
   using type = d2v;
+  typedef d2v any __attribute__((aligned(8)));
   static constexpr int n = 2;
 };
 
-template <bool NT, typename V>
-__device__ __forceinline__ V vload(const V *p) {
+// The 16 bytes at vector index i of p.
+template <bool NT, typename T>
+__device__ __forceinline__ typename V16<T>::type vload(const T *p, int64_t i) {
+  using A = typename V16<T>::any;
+  const A *v = reinterpret_cast<const A *>(p) + i;
   if constexpr (NT)
-    return __builtin_nontemporal_load(p);
+    return __builtin_nontemporal_load(v);
   else
-    return *p;
+    return *v;
 }
-template <bool NT, typename V>
-__device__ __forceinline__ void vstore(V *p, V v) {
+template <bool NT, typename T>
+__device__ __forceinline__ void vstore(T *p, int64_t i,
+                                       typename V16<T>::type w) {
+  using A = typename V16<T>::any;
+  A *v = reinterpret_cast<A *>(p) + i;
   if constexpr (NT)
-    __builtin_nontemporal_store(v, p);
+    __builtin_nontemporal_store(w, v);
   else
-    *p = v;
+    *v = w;
 }
 
 // BLAS element index for an increment (negative increments walk backwards).
@@ -100,43 +118,45 @@ struct AxpyOp<float> {
   static constexpr bool reads_y = true;
 };
 
-// Vector path: x, y 16-byte aligned, unit stride; one vector per thread
-// (grid-stride only beyond kMaxReduceBlocks workgroups).
+// Vector path: unit stride; one vector per thread (grid-stride only beyond
+// kMaxReduceBlocks workgroups), and one thread for the n % VN last elements.
 template <typename T, typename Op, bool NT>
 __global__ __launch_bounds__(kThreads) void elementwise_vec_kernel(
-    int64_t nvec, const typename V16<T>::type *__restrict__ x,
-    typename V16<T>::type *__restrict__ y, Op op) {
+    int64_t n, const T *__restrict__ x, T *__restrict__ y, Op op) {
   using V = typename V16<T>::type;
   constexpr int VN = V16<T>::n;
+  const int64_t nvec = n / VN;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < nvec;
-       i += stride) {
-    const V xv = vload<NT>(x + i);
+  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  for (; i < nvec; i += stride) {
+    const V xv = vload<NT>(x, i);
     V yv{};
-    if (Op::reads_y) yv = vload<NT>(y + i);
+    if (Op::reads_y) yv = vload<NT>(y, i);
     V r;
 #pragma unroll
     for (int e = 0; e < VN; ++e) r[e] = op(xv[e], yv[e]);
-    vstore<NT>(y + i, r);
+    vstore<NT>(y, i, r);
   }
+  if (i == nvec)
+    for (int64_t j = nvec * VN; j < n; ++j)
+      y[j] = op(x[j], Op::reads_y ? y[j] : T(0));
 }
 
 // Scalar path: any increments. Element (b, i) of the batch lives at
-// base + b*bstride + blas_index(i, n, inc).
+// base + b*bstride + blas_index(i, n, inc); blockIdx.y walks the batch.
 template <typename T, typename Op>
 __global__ __launch_bounds__(kThreads) void elementwise_strided_kernel(
     int64_t n, int64_t batch, const T *__restrict__ x, int64_t incx,
     int64_t bsx, T *__restrict__ y, int64_t incy, int64_t bsy, Op op) {
-  const int64_t total = n * batch;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t f = (int64_t)blockIdx.x * kThreads + threadIdx.x; f < total;
-       f += stride) {
-    int64_t b = f / n, i = f - b * n;
-    int64_t ix = b * bsx + blas_index(i, n, incx);
-    int64_t iy = b * bsy + blas_index(i, n, incy);
-    T yv = Op::reads_y ? y[iy] : T(0);
-    y[iy] = op(x[ix], yv);
-  }
+  for (int64_t b = blockIdx.y; b < batch; b += gridDim.y)
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
+         i += stride) {
+      const int64_t ix = b * bsx + blas_index(i, n, incx);
+      const int64_t iy = b * bsy + blas_index(i, n, incy);
+      const T yv = Op::reads_y ? y[iy] : T(0);
+      y[iy] = op(x[ix], yv);
+    }
 }
 
 // Complex scal. Products are rounded separately (contraction is switched
@@ -236,19 +256,34 @@ __global__ __launch_bounds__(kThreads) void reduce_finish_kernel(
   }
 }
 
+// Where a reduction's sum goes: one partial per workgroup for
+// reduce_finish_kernel, or, from the only workgroup, the result itself.
+template <typename T>
+struct ReduceOut {
+  double *partials;
+  T *result;
+  unsigned long long *done, seq;
+  __device__ __forceinline__ void operator()(double sum) const {
+    if (threadIdx.x != 0) return;
+    if (gridDim.x > 1) {
+      partials[blockIdx.x] = sum;
+      return;
+    }
+    *result = (T)sum;
+    __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+
 // Vector-path reduction: grid-stride over 16-byte vectors of x (and y) with
 // U vectors in flight per thread; the scalar tail (< one vector) is added by
-// block 0. Each workgroup writes one FP64 partial; reduce_finish_kernel sums
-// them.
+// block 0.
 template <typename T, typename Red, bool NT, int U, int TH = kThreads>
 __global__ __launch_bounds__(TH) void reduce_vec_kernel(
     int64_t n, const T *__restrict__ x, const T *__restrict__ y,
-    double *partials, Red red) {
+    ReduceOut<T> out, Red red) {
   using V = typename V16<T>::type;
   constexpr int VN = V16<T>::n;
   __shared__ double lds[TH / 64];
-  const V *xv = reinterpret_cast<const V *>(x);
-  const V *yv = reinterpret_cast<const V *>(y);
   const int64_t nvec = n / VN;
   const int64_t stride = (int64_t)gridDim.x * TH;
   T acc[U][VN];
@@ -261,8 +296,8 @@ __global__ __launch_bounds__(TH) void reduce_vec_kernel(
     V a[U], b[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      a[u] = vload<NT>(xv + i + u * stride);
-      if (Red::two) b[u] = vload<NT>(yv + i + u * stride);
+      a[u] = vload<NT>(x, i + u * stride);
+      if (Red::two) b[u] = vload<NT>(y, i + u * stride);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -270,9 +305,9 @@ __global__ __launch_bounds__(TH) void reduce_vec_kernel(
       for (int e = 0; e < VN; ++e) acc[u][e] += red(a[u][e], b[u][e]);
   }
   for (; i < nvec; i += stride) {
-    const V a = vload<NT>(xv + i);
+    const V a = vload<NT>(x, i);
     V b{};
-    if (Red::two) b = vload<NT>(yv + i);
+    if (Red::two) b = vload<NT>(y, i);
 #pragma unroll
     for (int e = 0; e < VN; ++e) acc[0][e] += red(a[e], b[e]);
   }
@@ -285,8 +320,7 @@ __global__ __launch_bounds__(TH) void reduce_vec_kernel(
     const int64_t t = nvec * VN + threadIdx.x;
     if (t < n) s += (double)red(x[t], Red::two ? y[t] : T(0));
   }
-  const double part = block_sum<TH>(s, lds);
-  if (threadIdx.x == 0) partials[blockIdx.x] = part;
+  out(block_sum<TH>(s, lds));
 }
 
 // Strided / batched reduction: element (b, i) at b*bs + blas_index(i, n, inc).
@@ -294,20 +328,20 @@ template <typename T, typename Red>
 __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(
     int64_t n, int64_t batch, const T *__restrict__ x, int64_t incx,
     int64_t bsx, const T *__restrict__ y, int64_t incy, int64_t bsy,
-    double *partials, Red red) {
+    ReduceOut<T> out, Red red) {
   __shared__ double lds[kThreads / 64];
   const int64_t total = n * batch;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   T acc = T(0);
   for (int64_t f = (int64_t)blockIdx.x * kThreads + threadIdx.x; f < total;
        f += stride) {
-    int64_t b = f / n, i = f - b * n;
+    // (no 64-bit division for a single vector)
+    const int64_t b = batch == 1 ? 0 : f / n, i = f - b * n;
     T xv = x[b * bsx + blas_index(i, n, incx)];
     T yv = Red::two ? y[b * bsy + blas_index(i, n, incy)] : T(0);
     acc += red(xv, yv);
   }
-  const double part = block_sum((double)acc, lds);
-  if (threadIdx.x == 0) partials[blockIdx.x] = part;
+  out(block_sum((double)acc, lds));
 }
 
 // ---------------------------------------------------------------------------
@@ -324,48 +358,31 @@ hcblasStatus_t run_elementwise(hcblasHandle_t h, int64_t n, int64_t batch,
                                const T *x, int64_t incx, int64_t bsx, T *y,
                                int64_t incy, int64_t bsy, Op op) {
   constexpr int VN = V16<T>::n;
-  using V = typename V16<T>::type;
   if (n <= 0 || batch <= 0) return HCBLAS_STATUS_SUCCESS;
   // A unit-stride batch with batch stride n is one contiguous vector of
   // n*batch.
   const bool contiguous =
       incx == 1 && incy == 1 && (batch == 1 || (bsx == n && bsy == n));
   const int64_t flat = n * batch;
-  if (contiguous && aligned16(x) && aligned16(y)) {
-    const int64_t nvec = flat / VN;
-    if (nvec > 0) {
-      const bool nt = flat * (int64_t)sizeof(T) >= kStreamBytes;
-      if (nt)
-        elementwise_vec_kernel<T, Op, true>
-            <<<full_grid(nvec), kThreads, 0, h->stream>>>(
-                nvec, reinterpret_cast<const V *>(x), reinterpret_cast<V *>(y),
-                op);
-      else
-        elementwise_vec_kernel<T, Op, false>
-            <<<full_grid(nvec), kThreads, 0, h->stream>>>(
-                nvec, reinterpret_cast<const V *>(x), reinterpret_cast<V *>(y),
-                op);
-    }
-    const int64_t tail = flat - nvec * VN;
-    if (tail > 0)
-      elementwise_strided_kernel<T, Op><<<1, kThreads, 0, h->stream>>>(
-          tail, 1, x + nvec * VN, 1, 0, y + nvec * VN, 1, 0, op);
-    return launch_status();
-  }
   if (contiguous) {
-    elementwise_strided_kernel<T, Op>
-        <<<full_grid(flat), kThreads, 0, h->stream>>>(flat, 1, x, 1, 0, y, 1,
-                                                      0, op);
+    const int grid = full_grid(cdiv(flat, VN));
+    if (flat * (int64_t)sizeof(T) >= kStreamBytes)
+      elementwise_vec_kernel<T, Op, true>
+          <<<grid, kThreads, 0, h->stream>>>(flat, x, y, op);
+    else
+      elementwise_vec_kernel<T, Op, false>
+          <<<grid, kThreads, 0, h->stream>>>(flat, x, y, op);
     return launch_status();
   }
-  elementwise_strided_kernel<T, Op>
-      <<<full_grid(flat), kThreads, 0, h->stream>>>(n, batch, x, incx, bsx, y,
-                                                    incy, bsy, op);
+  dim3 grid((unsigned)full_grid(n),
+            (unsigned)std::min<int64_t>(batch, kMaxGridY));
+  elementwise_strided_kernel<T, Op><<<grid, kThreads, 0, h->stream>>>(
+      n, batch, x, incx, bsx, y, incy, bsy, op);
   return launch_status();
 }
 
 // Waits until the reduction of call `seq` has published its result in the
-// handle's pinned block (see tree_finish).
+// handle's pinned block (ReduceOut, reduce_finish_kernel).
 hcblasStatus_t wait_result(hcblasHandle_t h, unsigned long long seq) {
   const unsigned long long *w =
       reinterpret_cast<const unsigned long long *>(h->h_result + 1);
@@ -397,8 +414,9 @@ hcblasStatus_t run_reduce(hcblasHandle_t h, int64_t n, int64_t batch,
   const bool contiguous = incx == 1 && (!Red::two || incy == 1) &&
                           (batch == 1 || (bsx == n && (!Red::two || bsy == n)));
   const T *yy = Red::two ? y : x;
+  const ReduceOut<T> out{h->d_partials, dres, done, seq};
   int nparts = 1;
-  if (contiguous && aligned16(x) && (!Red::two || aligned16(y))) {
+  if (contiguous) {
     // FP32 asum keeps 16 vectors in flight per lane (SASUM 2^28: 6.05
     // against 5.86 TB/s with 8).
     // FP64 asum runs 512-thread workgroups with 4 vectors in flight (DASUM
@@ -410,27 +428,26 @@ hcblasStatus_t run_reduce(hcblasHandle_t h, int64_t n, int64_t batch,
                       : wide   ? kReduceUnroll
                                : 4 * kReduceUnroll;
     const int64_t nvec = flat / VN;
-    const int grid = (int)std::max<int64_t>(
-        1, std::min<int64_t>(cdiv(nvec, TH * U), kReduceGrid));
+    const int64_t trips = cdiv(nvec, TH * U);
+    nparts = trips <= kAloneTrips
+                 ? 1
+                 : (int)std::min<int64_t>(trips, kReduceGrid);
     const int64_t bytes = flat * (int64_t)sizeof(T) * (Red::two ? 2 : 1);
     if (bytes >= kStreamBytes)
       reduce_vec_kernel<T, Red, true, U, TH>
-          <<<grid, TH, 0, h->stream>>>(flat, x, yy, h->d_partials, red);
+          <<<nparts, TH, 0, h->stream>>>(flat, x, yy, out, red);
     else
       reduce_vec_kernel<T, Red, false, U, TH>
-          <<<grid, TH, 0, h->stream>>>(flat, x, yy, h->d_partials, red);
-    nparts = grid;
-  } else if (contiguous) {
-    nparts = (int)std::min<int64_t>(full_grid(flat), kReduceGrid);
-    reduce_strided_kernel<T, Red><<<nparts, kThreads, 0, h->stream>>>(
-        flat, 1, x, 1, 0, yy, 1, 0, h->d_partials, red);
+          <<<nparts, TH, 0, h->stream>>>(flat, x, yy, out, red);
   } else {
-    nparts = (int)std::min<int64_t>(full_grid(flat), kReduceGrid);
+    if (flat > kAloneTrips * kThreads)
+      nparts = (int)std::min<int64_t>(full_grid(flat), kReduceGrid);
     reduce_strided_kernel<T, Red><<<nparts, kThreads, 0, h->stream>>>(
-        n, batch, x, incx, bsx, yy, incy, bsy, h->d_partials, red);
+        n, batch, x, incx, bsx, yy, incy, bsy, out, red);
   }
-  reduce_finish_kernel<T><<<1, kThreads, 0, h->stream>>>(
-      nparts, h->d_partials, dres, done, seq);
+  if (nparts > 1)
+    reduce_finish_kernel<T><<<1, kThreads, 0, h->stream>>>(
+        nparts, h->d_partials, dres, done, seq);
   hcblasStatus_t st = launch_status();
   if (st != HCBLAS_STATUS_SUCCESS) return st;
   // The API returns a host scalar, so the call waits for its result (same
