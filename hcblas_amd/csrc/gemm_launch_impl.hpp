@@ -65,78 +65,116 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
   return HCBLAS_STATUS_SUCCESS;
 }
 
-// Macro-tile choice (measured at 8192^3 on MI355X, the largest tile whose
-// grid still covers every CU is taken):
-//   FP32  256x256x32, 8 waves of 128x64 on 32x32 MFMA blocks (146-148
-//         TF/s, 93-94% of peak, with the step's LDS writes and loads issued
-//         among the first chunk's MFMAs), then 256x128 8 waves, 128x128 4
-//         waves, 64x64;
-//   FP64  256x128x16, 8 waves of 64x64 (71.6 TF/s NN and TN, 91%, with the
-//         same interleave; 66.9 / 64.5 before it; 128x256 2x4 was as fast
-//         on NN, 128x128 and smaller tiles stay at 75% or below), then
-//         128x64x16 8 waves (58.5), then 64x64 8 waves;
-//   F16 / BF16 256x256x64, 8 waves on 32x32 blocks, then 128x128 8 waves,
-//         then 64x64.
+// Macro tiles, largest first, and the rate of each in TF/s over a grid of many
+// tiles (8192 x 8192 x 1024 on MI355X), with 0, 1 or 2 operands r-contiguous
+// (transposed on their way into LDS):
+//   FP32  256x256x32, 8 waves of 128x64 on 32x32 MFMA blocks (146-148 TF/s at
+//         8192^3, 93-94% of peak), 256x128 8 waves, 128x128 4 waves, 64x64 8
+//         waves, 32x32 4 waves;
+//   FP64  256x128x16, 8 waves of 64x64 (71.6 TF/s at 8192^3, 91%), 128x64, 64x64
+//         8 waves, 32x32 4 waves;
+//   F16 / BF16 256x256x64, 8 waves on 32x32 blocks, 128x128 8 waves of 64x32,
+//         64x64 8 waves, 32x32 4 waves.
+struct MacroTile {
+  int bm, bn;
+  int rate[3];
+};
+template <Elem E>
+inline constexpr MacroTile kTiles[] = {{256, 256, {1180, 1110, 916}},
+                                       {128, 128, {1017, 820, 589}},
+                                       {64, 64, {495, 205, 130}},
+                                       {32, 32, {333, 180, 122}}};
+template <>
+inline constexpr MacroTile kTiles<Elem::F32>[] = {{256, 256, {140, 140, 133}},
+                                                  {256, 128, {128, 128, 129}},
+                                                  {128, 128, {133, 129, 127}},
+                                                  {64, 64, {115, 108, 101}},
+                                                  {32, 32, {104, 93, 75}}};
+template <>
+inline constexpr MacroTile kTiles<Elem::F64>[] = {{256, 128, {68, 68, 68}},
+                                                  {128, 64, {68, 68, 67}},
+                                                  {64, 64, {66, 65, 65}},
+                                                  {32, 32, {58, 55, 52}}};
+
+// The tile with the least time on the CU that gets the most tiles,
+// ceil(tiles / CUs) * area / rate: tiles past the edge of C and a last round
+// that leaves most CUs idle count in full. (Taking the largest tile whose grid
+// covers every CU instead: 3072 x 3072 x 1024 SGEMM NN 267 us on 288 tiles of
+// 256x128, 180 on 2304 of 64x64; 5512 x 6720 x 1024 738 on 256x256, 658 on
+// 128x128; a batch of 212 512 x 37 x 32 DGEMMs 36 us on 256x128, 21 on 64x64;
+// 529 x 192 x 1152 28.8 on 27 tiles of 64x64, 12.1 on 32x32.)
+template <Elem E>
+const MacroTile &pick_tile(int64_t M, int64_t N, int64_t batch, int num_cus,
+                           int r_contiguous) {
+  const MacroTile *best = nullptr;
+  double least = 0;
+  for (const MacroTile &t : kTiles<E>) {
+    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
+    const double time = (double)cdiv(tiles, num_cus) * t.bm * t.bn /
+                        t.rate[r_contiguous];
+    if (best == nullptr || time < least) {
+      best = &t;
+      least = time;
+    }
+  }
+  return *best;
+}
+
 template <Elem E, typename OutT>
 hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
                            bool a_k, bool b_k, int64_t batch) {
-  auto tiles = [&](int bm, int bn) {
-    return cdiv(p.M, bm) * cdiv(p.N, bn) * batch;
-  };
-  if constexpr (E == Elem::F32) {
-    if (tiles(256, 256) >= num_cus)
-      return launch_tiles<E, OutT, 256, 256, 32, 2, 4, 32>(stream, p, a_k, b_k, batch);
-    if (tiles(256, 128) >= num_cus)
-      return launch_tiles<E, OutT, 256, 128, 32, 2, 4>(stream, p, a_k, b_k, batch);
-    if (tiles(128, 128) >= num_cus)
-      return launch_tiles<E, OutT, 128, 128, 32, 2, 2>(stream, p, a_k, b_k, batch);
-  } else if constexpr (E == Elem::F64) {
-    if (tiles(256, 128) >= num_cus)
-      return launch_tiles<E, OutT, 256, 128, 16, 4, 2>(stream, p, a_k, b_k, batch);
-    if (tiles(128, 64) >= num_cus)
-      return launch_tiles<E, OutT, 128, 64, 16, 2, 4>(stream, p, a_k, b_k, batch);
+  using C = TileCfg<E>;
+  const MacroTile &t =
+      pick_tile<E>(p.M, p.N, batch, num_cus, (a_k ? 0 : 1) + (b_k ? 0 : 1));
+  const int64_t tiles = cdiv(p.M, t.bm) * cdiv(p.N, t.bn) * batch;
+  if constexpr (E == Elem::F64) {
+    if (t.bm == 256)
+      return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 4, 2>(stream, p, a_k,
+                                                              b_k, batch);
+    if (t.bm == 128)
+      return launch_tiles<E, OutT, 128, 64, C::BK_BIG, 2, 4>(stream, p, a_k,
+                                                             b_k, batch);
   } else {
-    if (tiles(256, 256) >= num_cus)
-      return launch_tiles<E, OutT, 256, 256, TileCfg<E>::BK_BIG, 2, 4, 32>(
+    if (t.bn == 256)
+      return launch_tiles<E, OutT, 256, 256, C::BK_BIG, 2, 4, 32>(
           stream, p, a_k, b_k, batch);
-    // 8 waves of 64 x 32 (fragment read-ahead, two-vector transposed loads):
-    // 2048^3 HGEMM NN 38.6 against 44.4 us with 4 waves of 64 x 64.
-    if (tiles(128, 128) >= num_cus)
-      return launch_tiles<E, OutT, 128, 128, TileCfg<E>::BK_BIG, 2, 4, 32>(
-          stream, p, a_k, b_k, batch);
+    if constexpr (E == Elem::F32) {
+      if (t.bm == 256)
+        return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 2, 4>(stream, p, a_k,
+                                                                b_k, batch);
+      if (t.bm == 128)
+        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 2>(stream, p, a_k,
+                                                                b_k, batch);
+    } else {
+      // 8 waves of 64 x 32 (fragment read-ahead, two-vector transposed loads):
+      // 2048^3 HGEMM NN 38.6 against 44.4 us with 4 waves of 64 x 64.
+      if (t.bm == 128)
+        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 4, 32>(
+            stream, p, a_k, b_k, batch);
+    }
   }
-  // Fewer 64x64 tiles than CUs: 32x32 tiles of 4 waves on four times as many
-  // CUs (a tile's K loop is a serial chain, so its MFMAs bound the call:
-  // 529 x 192 x 1152 SGEMM NN 12.1 us against 28.8 on 27 tiles of 64x64,
-  // 700^3 13.3 against 19.6, 1024 x 512 x 1024 16.0 against 25.8 on 128).
-  // Beyond three quarters of the CUs some CU gets four 32x32 tiles, which take
-  // longer than one of 64x64 (210 tiles, 900 x 880 x 1000: SGEMM NT 31.6 against
-  // 24.8, DGEMM NN 53.6 against 45.6); FP32 with two r-contiguous operands, whose
-  // LDS writes weigh most, from five eighths on (182 tiles, 880 x 800 x 1000 NT
-  // 25.3 against 24.4, NN 22.7 against 24.3). The sums are the same bit for bit.
-  const int eighths = E == Elem::F32 && !a_k && !b_k ? 5 : 6;
-  if (8 * tiles(64, 64) <= eighths * num_cus) {
-    using C = TileCfg<E>;
-    if (p.K >= C::LONG_K)
+  if (t.bm == 32) {
+    if (p.K >= C::LONG_K && tiles <= num_cus)
       return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2>(
           stream, p, a_k, b_k, batch);
     return launch_tiles<E, OutT, 32, 32, C::BK_32, 2, 2>(stream, p, a_k, b_k,
                                                          batch);
   }
-  // Small problems: 64x64 tiles, 8 waves of 32x16 for every type (more
-  // waves per CU to cover the load latency when there are only about as
-  // many tiles as CUs: 1024^3 SGEMM 0.0376 ms against 0.0382 with 4 waves,
-  // the conv-net shape set 24.6 TF/s against 23.8; 1024^3 DGEMM 58.8 us
-  // against 71.6). FP32 with K >= 512 takes 128-wide K steps:
-  // a 32-wide step is 16 MFMAs per wave, too short to cover the global loads
+  // 64x64 tiles, 8 waves of 32x16 for every type (more waves per CU to cover
+  // the load latency when there are only about as many tiles as CUs: 1024^3
+  // SGEMM 0.0376 ms against 0.0382 with 4 waves; 1024^3 DGEMM 58.8 us against
+  // 71.6). FP32 with one tile per CU and K >= 512 takes 128-wide K steps: a
+  // 32-wide step is 16 MFMAs per wave, too short to cover the global loads
   // issued one step ahead (1024^3 kernel 27.5 us against 31.6 with BK = 32,
-  // 29.5 with 64); shorter K keeps 32 so the last step pads little.
+  // 29.5 with 64); with more tiles the CU's other workgroups cover them (3072 x
+  // 3072 x 1024 NN 180 us with 32, 192 with 128).
   if constexpr (E == Elem::F32) {
-    if (p.K >= 512)
-      return launch_tiles<E, OutT, 64, 64, 128, 2, 4>(stream, p, a_k, b_k, batch);
+    if (p.K >= 512 && tiles <= num_cus)
+      return launch_tiles<E, OutT, 64, 64, 128, 2, 4>(stream, p, a_k, b_k,
+                                                      batch);
   }
-  return launch_tiles<E, OutT, 64, 64, TileCfg<E>::BK_SMALL, 2, 4>(
-      stream, p, a_k, b_k, batch);
+  return launch_tiles<E, OutT, 64, 64, C::BK_SMALL, 2, 4>(stream, p, a_k, b_k,
+                                                          batch);
 }
 
 template <Elem E, int T, int BK, int WM, int WN>
