@@ -95,32 +95,45 @@ __device__ __forceinline__ void run_tile(const ProbDev &p, int m0, int n0,
   }
 }
 
-// Dynamic schedule: counters[0] is the next work entry, taken with one
-// atomic per tile. Static schedule: workgroup g takes entries g, g + G,
-// g + 2G, ... (G = grid size); over a longest-first list that balances like
-// the queue without its atomic per tile. counters[1] counts finished
-// workgroups; the last one resets both counters.
+// The work list is cut into one part per XCD (kXcd, parts[x] .. parts[x + 1]),
+// each holding whole problems: workgroup g belongs to part g % 8, the XCD that
+// the dispatcher gives it, so a problem's tiles read its A and B through one
+// L2. Static schedule: a workgroup takes every (grid / 8)-th entry of its part,
+// longest first. Dynamic schedule: it takes its part's next entry with one atomic
+// on counters[part], and entries of the following parts when its own is empty.
+// counters[8] counts finished workgroups; the last one resets all counters.
 // OCC: workgroups per CU the launch is sized for (the register budget
 // follows from it: 4 waves per workgroup, one per SIMD).
+constexpr int kXcd = 8;
+
 template <int TM, bool NARROW, int OCC>
 __global__ __launch_bounds__(256, OCC) void grouped_gemm_kernel(
     const ProbDev *__restrict__ probs, const int2 *__restrict__ work,
-    int total, unsigned int *counters, int dynamic) {
+    const int *__restrict__ parts, unsigned int *counters, int dynamic) {
   __shared__ __attribute__((aligned(16))) char lds[GroupCfg<TM>::LDS];
   __shared__ int next;
-  for (int s = blockIdx.x;; s += gridDim.x) {
-    int w = s;
+  int part = blockIdx.x % kXcd, left = kXcd;
+  int begin = parts[part], end = parts[part + 1];
+  int w = begin + blockIdx.x / kXcd;
+  while (true) {
     if (dynamic) {
       if (threadIdx.x == 0)
-        next = (int)__hip_atomic_fetch_add(&counters[0], 1u, __ATOMIC_RELAXED,
+        next = (int)__hip_atomic_fetch_add(&counters[part], 1u,
+                                           __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
-      w = next;
+      w = begin + next;
       __syncthreads();
     }
     // uniform across the workgroup: the descriptor comes through scalar loads
     w = __builtin_amdgcn_readfirstlane(w);
-    if (w >= total) break;
+    if (w >= end) {
+      if (!dynamic || --left == 0) break;
+      part = (part + 1) % kXcd;
+      begin = parts[part];
+      end = parts[part + 1];
+      continue;
+    }
     const int2 it = work[w];
     const ProbDev p = probs[__builtin_amdgcn_readfirstlane(it.x)];
     const int t = __builtin_amdgcn_readfirstlane(it.y);
@@ -134,16 +147,15 @@ __global__ __launch_bounds__(256, OCC) void grouped_gemm_kernel(
       run_tile<Elem::F32, float, TM, NARROW>(p, tm * TM, tn * TM, tid, lds);
     else
       run_tile<Elem::F16, uint16_t, TM, NARROW>(p, tm * TM, tn * TM, tid, lds);
+    w += gridDim.x / kXcd;
   }
   if (threadIdx.x == 0) {
     const unsigned int t = __hip_atomic_fetch_add(
-        &counters[1], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    if (t == gridDim.x - 1) {
-      __hip_atomic_store(&counters[0], 0u, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&counters[1], 0u, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    }
+        &counters[kXcd], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (t == gridDim.x - 1)
+      for (int x = 0; x <= kXcd; ++x)
+        __hip_atomic_store(&counters[x], 0u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -165,7 +177,8 @@ struct hcblasGroupedPlan {
   ProbDev *d_probs = nullptr;
   int2 *d_work = nullptr;
   size_t work_cap = 0;
-  unsigned int *d_counters = nullptr;
+  int *d_parts = nullptr;              // kXcd + 1 offsets into d_work
+  unsigned int *d_counters = nullptr;  // kXcd queues, finished workgroups
   int total = 0;
   int grid = 0;
   int shape = 0;   // index into kTileShapes
@@ -191,15 +204,15 @@ void launch_occ(hcblasGroupedPlan *p, hipStream_t s) {
   switch (kOccupancies[p->occ]) {
     case 2:
       grouped_gemm_kernel<TM, NARROW, 2><<<g, 256, 0, s>>>(
-          p->d_probs, p->d_work, p->total, p->d_counters, p->sched == 0);
+          p->d_probs, p->d_work, p->d_parts, p->d_counters, p->sched == 0);
       break;
     case 3:
       grouped_gemm_kernel<TM, NARROW, 3><<<g, 256, 0, s>>>(
-          p->d_probs, p->d_work, p->total, p->d_counters, p->sched == 0);
+          p->d_probs, p->d_work, p->d_parts, p->d_counters, p->sched == 0);
       break;
     default:
       grouped_gemm_kernel<TM, NARROW, 4><<<g, 256, 0, s>>>(
-          p->d_probs, p->d_work, p->total, p->d_counters, p->sched == 0);
+          p->d_probs, p->d_work, p->d_parts, p->d_counters, p->sched == 0);
       break;
   }
 }
@@ -216,27 +229,33 @@ void launch_grouped(hcblasGroupedPlan *p, hipStream_t s) {
 hcblasStatus_t build(hcblasHandle_t h, hcblasGroupedPlan *p, int shape,
                      int order, int occ, int sched) {
   const int tm = kTileShapes[shape];
-  std::vector<int2> work;
-  std::vector<int64_t> cost;
+  // Problems in the order asked for, each to the XCD with the least cost so far.
+  std::vector<int64_t> cost(p->count, 0);
+  std::vector<int> idx;
   for (int i = 0; i < p->count; ++i) {
     ProbDev &q = p->probs[i];
     if (q.M == 0 || q.N == 0) continue;
-    const int tmi = (q.M + tm - 1) / tm;
     q.tiles_n = (q.N + tm - 1) / tm;
-    const int64_t c = (int64_t)(q.K + 64) * (q.dtype == 0 ? 8 : 1);
-    for (int t = 0; t < tmi * q.tiles_n; ++t) {
-      work.push_back(make_int2(i, t));
-      cost.push_back(c);
-    }
+    cost[i] = (int64_t)(q.K + 64) * (q.dtype == 0 ? 8 : 1);
+    idx.push_back(i);
   }
-  if (order == 0) {
-    std::vector<int> idx(work.size());
-    for (size_t i = 0; i < idx.size(); ++i) idx[i] = (int)i;
+  if (order == 0)
     std::stable_sort(idx.begin(), idx.end(),
                      [&](int a, int b) { return cost[a] > cost[b]; });
-    std::vector<int2> w2(work.size());
-    for (size_t i = 0; i < idx.size(); ++i) w2[i] = work[idx[i]];
-    work.swap(w2);
+  std::vector<int2> list[kXcd];
+  int64_t load[kXcd] = {};
+  for (int i : idx) {
+    const ProbDev &q = p->probs[i];
+    const int nt = (q.M + tm - 1) / tm * q.tiles_n;
+    const int x = (int)(std::min_element(load, load + kXcd) - load);
+    for (int t = 0; t < nt; ++t) list[x].push_back(make_int2(i, t));
+    load[x] += cost[i] * nt;
+  }
+  std::vector<int2> work;
+  int parts[kXcd + 1] = {};
+  for (int x = 0; x < kXcd; ++x) {
+    work.insert(work.end(), list[x].begin(), list[x].end());
+    parts[x + 1] = (int)work.size();
   }
   p->total = (int)work.size();
   if (work.size() > p->work_cap) {
@@ -252,14 +271,19 @@ hcblasStatus_t build(hcblasHandle_t h, hcblasGroupedPlan *p, int shape,
                 hipMemcpyHostToDevice) != hipSuccess)
     return HCBLAS_STATUS_EXECUTION_FAILED;
   if (hipMemcpy(p->d_probs, p->probs.data(), sizeof(ProbDev) * p->count,
-                hipMemcpyHostToDevice) != hipSuccess)
+                hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(p->d_parts, parts, sizeof(parts), hipMemcpyHostToDevice) !=
+          hipSuccess)
     return HCBLAS_STATUS_EXECUTION_FAILED;
   p->shape = shape;
   p->order = order;
   p->occ = occ;
   p->sched = sched;
-  p->grid =
-      std::max(1, std::min(p->total, h->num_cus * kOccupancies[occ]));
+  // (a whole number of workgroups for each part)
+  p->grid = (int)cdiv(std::max(1, std::min(p->total, h->num_cus *
+                                                          kOccupancies[occ])),
+                      kXcd) *
+            kXcd;
   free_graph(p);
   if (p->total == 0) return HCBLAS_STATUS_SUCCESS;
   hipStream_t cs;
@@ -349,8 +373,11 @@ hcblasStatus_t hcblasGroupedPlanCreate(hcblasHandle_t handle,
   }
   if (hipMalloc(&p->d_probs, sizeof(ProbDev) * std::max(1, count)) !=
           hipSuccess ||
-      hipMalloc(&p->d_counters, 2 * sizeof(unsigned int)) != hipSuccess ||
-      hipMemset(p->d_counters, 0, 2 * sizeof(unsigned int)) != hipSuccess ||
+      hipMalloc(&p->d_parts, (kXcd + 1) * sizeof(int)) != hipSuccess ||
+      hipMalloc(&p->d_counters, (kXcd + 1) * sizeof(unsigned int)) !=
+          hipSuccess ||
+      hipMemset(p->d_counters, 0, (kXcd + 1) * sizeof(unsigned int)) !=
+          hipSuccess ||
       hipDeviceSynchronize() != hipSuccess) {
     hcblasGroupedPlanDestroy(p);
     return HCBLAS_STATUS_ALLOC_FAILED;
@@ -436,6 +463,7 @@ hcblasStatus_t hcblasGroupedPlanDestroy(hcblasGroupedPlan_t plan) {
   free_graph(plan);
   if (plan->d_probs) (void)hipFree(plan->d_probs);
   if (plan->d_work) (void)hipFree(plan->d_work);
+  if (plan->d_parts) (void)hipFree(plan->d_parts);
   if (plan->d_counters) (void)hipFree(plan->d_counters);
   delete plan;
   return HCBLAS_STATUS_SUCCESS;
