@@ -233,24 +233,26 @@ struct TileLoader {
   static constexpr bool TRANS4 =
       !KCONT && VEC == 4 && NV == 4 * NTH && ROWS % 16 == 0 && BK % 16 == 0 &&
       (ROWS / 16) * (BK / 16) * 16 == NTH;
-  // 16-bit transposing tiles with four vectors per thread and 64-deep K
-  // steps: each thread loads the four k-lines of one 8-row vector and writes
-  // its 8 rows x 4 k with eight 8-byte LDS stores along k (16-bit selects
-  // pair the k values) instead of thirty-two 2-byte ones. The 32 lanes of a
-  // half-wave take 2 consecutive r-vectors x the 16 k-quads, whose slots
-  // (8 jr + e) x 144 + 8 kq are 32 distinct 8-byte slots of 256 bytes.
-  static constexpr bool TRANS4H = !KCONT && VEC == 8 && BK == 64 &&
-                                  NV == 4 * NTH && (ROWS / 8) * 16 == NTH;
-  // The same with two vectors per thread (64-row tiles of 4 waves): a
-  // thread loads two k-lines of one r-vector and writes its rows with
-  // 8-byte (FP32, 32-deep steps) or 4-byte (16-bit, 64-deep steps) stores
-  // along k. FP32: wave w takes r-vectors 4w..4w+3, its half-waves r-vectors
-  // {0, 2} and {1, 3} of those x the 16 k-pairs (row offsets 0 / 128 and
-  // 64 / 192 of 256 bytes); 16-bit: 2 r-vectors x 32 k-pairs per wave.
-  static constexpr bool TRANS2 = !KCONT && VEC == 4 && BK == 32 &&
-                                 NV == 2 * NTH && ROWS / 4 == NTH / 16;
-  static constexpr bool TRANS2H = !KCONT && VEC == 8 && BK == 64 &&
-                                  NV == 2 * NTH && (ROWS / 8) * 32 == NTH;
+  // 16-bit transposing tiles with four vectors per thread: each thread loads
+  // the four k-lines of one 8-row vector and writes its 8 rows x 4 k with
+  // eight 8-byte LDS stores along k (16-bit selects pair the k values) instead
+  // of thirty-two 2-byte ones. Groups of 16 lanes take 16 k-quads of one
+  // r-vector, neighbouring groups neighbouring r-vectors; the slots of a
+  // half-wave, (8 jr + e) x ROWB + 8 kq, are 32 distinct 8-byte slots of 256
+  // bytes, since 8 ROWB is 128 modulo 256 for every K step.
+  static constexpr bool TRANS4H = !KCONT && VEC == 8 && NV == 4 * NTH &&
+                                  BK % 64 == 0 && ROWS % 32 == 0;
+  // The same with two vectors per thread: a thread loads two k-lines of one
+  // r-vector and writes its rows with 8-byte (FP32) or 4-byte (16-bit) stores
+  // along k. FP32: groups of 16 lanes take 16 k-pairs, and of four neighbouring
+  // r-vectors the half-waves take {0, 2} and {1, 3} (row offsets 0 / 128 and
+  // 64 / 192 of 256 bytes). 16-bit: half-waves take 32 k-pairs, so that a
+  // wave's 4-byte slots of two r-vectors are all distinct (16 k-pairs of four
+  // r-vectors collide in pairs).
+  static constexpr bool TRANS2 = !KCONT && VEC == 4 && NV == 2 * NTH &&
+                                 BK % 32 == 0 && ROWS % 16 == 0;
+  static constexpr bool TRANS2H = !KCONT && VEC == 8 && NV == 2 * NTH &&
+                                  BK % 32 == 0 && ROWS % 32 == 0;
   const int tid;  // thread of the workgroup
   vec4u reg[PER_THREAD];
 
@@ -267,18 +269,16 @@ struct TileLoader {
       constexpr int GJ = ROWS / 16;  // groups of 4 r-vectors along r
       r = (4 * (g % GJ) + jj) * 4;
       k = (4 * (g / GJ) + kk) * 4 + i;
-    } else if (TRANS2) {
-      const int t = v % NTH, i = v / NTH, l = t & 63;
-      r = (4 * (t >> 6) + ((l >> 4) & 1) * 2 + (l >> 5)) * 4;
-      k = (l & 15) * 2 + i;
-    } else if (TRANS2H) {
-      const int t = v % NTH, i = v / NTH;
-      r = (t >> 5) * 8;
-      k = (t & 31) * 2 + i;
-    } else if (TRANS4H) {
-      const int t = v % NTH, i = v / NTH;
-      r = (t >> 4) * 8;
-      k = (t & 15) * 4 + i;
+    } else if (TRANS2 || TRANS2H || TRANS4H) {
+      constexpr int NR = ROWS / VEC;       // r-vectors
+      constexpr int KL = TRANS4H ? 4 : 2;  // k-lines per thread
+      constexpr int GL = TRANS2H && BK % 64 == 0 ? 32 : 16;  // lanes per group
+      // (unsigned: a group index that is always 0 costs no registers)
+      const unsigned t = (unsigned)v % NTH, i = (unsigned)v / NTH, g = t / GL;
+      unsigned j = g % NR;
+      if (TRANS2) j = (j & ~3u) | ((j & 1) << 1) | ((j >> 1) & 1);
+      r = j * VEC;
+      k = ((g / NR) * GL + t % GL) * KL + i;
     } else if (BLOCKED) {
       constexpr int NRB = ROWS / VEC / 8;
       const int w = v >> 6, l = v & 63;

@@ -6,25 +6,25 @@
 
 namespace hcb {
 
-// K steps: of the large tiles (BK_BIG), of 64x64 tiles (BK_SMALL), and of 32x32
-// tiles for a short and, from K = LONG_K on, a long K (few steps hide little of
-// the load latency; a long step pads a short K): 529 x 192 x 1152 FP64 NN 20.6
-// us with 64 against 24.7 with 16, 529 x 1152 x 192 12.3 against 11.0.
+// K steps: of the large tiles (BK_BIG); of 64x64 and 32x32 tiles; and of 32x32
+// tiles that leave CUs idle, from K = LONG_K on (few steps hide little of the
+// load latency; a long step pads a short K): 529 x 192 x 1152 FP64 NN 20.6 us
+// with 64 against 24.7 with 16, 529 x 1152 x 192 12.3 against 11.0.
 template <Elem E>
 struct TileCfg;
 template <>
 struct TileCfg<Elem::F32> {
-  static constexpr int BK_BIG = 32, BK_SMALL = 32;
+  static constexpr int BK_BIG = 32, BK_64 = 32;
   static constexpr int BK_32 = 64, BK_32_LONG = 128, LONG_K = 1024;
 };
 template <>
 struct TileCfg<Elem::F64> {
-  static constexpr int BK_BIG = 16, BK_SMALL = 16;
-  static constexpr int BK_32 = 16, BK_32_LONG = 64, LONG_K = 512;
+  static constexpr int BK_BIG = 16, BK_64 = 16;
+  static constexpr int BK_32 = 32, BK_32_LONG = 64, LONG_K = 512;
 };
 template <>
 struct TileCfg<Elem::F16> {
-  static constexpr int BK_BIG = 64, BK_SMALL = 64;
+  static constexpr int BK_BIG = 64, BK_64 = 64;
   static constexpr int BK_32 = 64, BK_32_LONG = 128, LONG_K = 1024;
 };
 template <>
@@ -69,12 +69,13 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
 // tiles (8192 x 8192 x 1024 on MI355X), with 0, 1 or 2 operands r-contiguous
 // (transposed on their way into LDS):
 //   FP32  256x256x32, 8 waves of 128x64 on 32x32 MFMA blocks (146-148 TF/s at
-//         8192^3, 93-94% of peak), 256x128 8 waves, 128x128 4 waves, 64x64 8
-//         waves, 32x32 4 waves;
+//         8192^3, 93-94% of peak), 256x128 8 waves, 128x128, 64x64 and 32x32 4
+//         waves;
 //   FP64  256x128x16, 8 waves of 64x64 (71.6 TF/s at 8192^3, 91%), 128x64, 64x64
 //         8 waves, 32x32 4 waves;
 //   F16 / BF16 256x256x64, 8 waves on 32x32 blocks, 128x128 8 waves of 64x32,
-//         64x64 8 waves, 32x32 4 waves.
+//         64x64 4 waves (8192 x 8192 x 1024 HGEMM NN 292 us against 655 with 8,
+//         whose r-contiguous tiles go to LDS by elements), 32x32 4 waves.
 struct MacroTile {
   int bm, bn;
   int rate[3];
@@ -82,19 +83,19 @@ struct MacroTile {
 template <Elem E>
 inline constexpr MacroTile kTiles[] = {{256, 256, {1180, 1110, 916}},
                                        {128, 128, {1017, 820, 589}},
-                                       {64, 64, {495, 205, 130}},
-                                       {32, 32, {333, 180, 122}}};
+                                       {64, 64, {610, 465, 304}},
+                                       {32, 32, {330, 238, 152}}};
 template <>
 inline constexpr MacroTile kTiles<Elem::F32>[] = {{256, 256, {140, 140, 133}},
                                                   {256, 128, {128, 128, 129}},
                                                   {128, 128, {133, 129, 127}},
-                                                  {64, 64, {115, 108, 101}},
-                                                  {32, 32, {104, 93, 75}}};
+                                                  {64, 64, {120, 117, 114}},
+                                                  {32, 32, {105, 97, 80}}};
 template <>
 inline constexpr MacroTile kTiles<Elem::F64>[] = {{256, 128, {68, 68, 68}},
                                                   {128, 64, {68, 68, 67}},
                                                   {64, 64, {66, 65, 65}},
-                                                  {32, 32, {58, 55, 52}}};
+                                                  {32, 32, {57, 54, 52}}};
 
 // The tile with the least time on the CU that gets the most tiles,
 // ceil(tiles / CUs) * area / rate: tiles past the edge of C and a last round
@@ -157,24 +158,38 @@ hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
     if (p.K >= C::LONG_K && tiles <= num_cus)
       return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2>(
           stream, p, a_k, b_k, batch);
+    // (16-bit r-contiguous tiles of 128-deep steps are transposed in
+    // registers: 8192 x 8192 x 1024 HGEMM NN 564 us against 743)
+    if (sizeof(typename ElemT<E>::T) == 2 && !(a_k && b_k))
+      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2>(
+          stream, p, a_k, b_k, batch);
     return launch_tiles<E, OutT, 32, 32, C::BK_32, 2, 2>(stream, p, a_k, b_k,
                                                          batch);
   }
-  // 64x64 tiles, 8 waves of 32x16 for every type (more waves per CU to cover
-  // the load latency when there are only about as many tiles as CUs: 1024^3
-  // SGEMM 0.0376 ms against 0.0382 with 4 waves; 1024^3 DGEMM 58.8 us against
-  // 71.6). FP32 with one tile per CU and K >= 512 takes 128-wide K steps: a
-  // 32-wide step is 16 MFMAs per wave, too short to cover the global loads
-  // issued one step ahead (1024^3 kernel 27.5 us against 31.6 with BK = 32,
-  // 29.5 with 64); with more tiles the CU's other workgroups cover them (3072 x
-  // 3072 x 1024 NN 180 us with 32, 192 with 128).
+  // 64x64 tiles. At most one tile per CU leaves nothing else to cover a tile's
+  // load latency: FP32 then runs 8 waves and long K steps (1024^3 NN 22.8 us
+  // with 128, 23.7 with 64, 27.5 with 4 waves and 32), FP64 32-deep ones
+  // (1024^3 42.3 against 44.1). With more tiles than CUs, 4 waves and short
+  // steps are ahead for FP32 (4096 x 4096 x 256 NN 84 us against 89 with 8
+  // waves and 92 with 64-deep steps).
   if constexpr (E == Elem::F32) {
     if (p.K >= 512 && tiles <= num_cus)
       return launch_tiles<E, OutT, 64, 64, 128, 2, 4>(stream, p, a_k, b_k,
                                                       batch);
+    if (tiles <= num_cus)
+      return launch_tiles<E, OutT, 64, 64, 64, 2, 4>(stream, p, a_k, b_k,
+                                                     batch);
   }
-  return launch_tiles<E, OutT, 64, 64, C::BK_SMALL, 2, 4>(stream, p, a_k, b_k,
-                                                          batch);
+  if constexpr (E == Elem::F64) {
+    if (tiles <= num_cus)
+      return launch_tiles<E, OutT, 64, 64, 32, 2, 4>(stream, p, a_k, b_k,
+                                                     batch);
+    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 4>(stream, p, a_k, b_k,
+                                                         batch);
+  } else {
+    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 2>(stream, p, a_k, b_k,
+                                                         batch);
+  }
 }
 
 template <Elem E, int T, int BK, int WM, int WN>
@@ -200,14 +215,15 @@ hcblasStatus_t launch_gemm_splitk(hipStream_t stream, int num_cus,
                                   const SplitK &sk,
                                   typename ElemT<E>::Acc *W) {
   using Acc = typename ElemT<E>::Acc;
-  // 64x64 tiles run 8 waves of 32 x 16 for every type (FP64 256 x 128 x 16384
-  // 96 us against 123 with 4 waves of 32 x 32).
+  // (64x64 FP64 256 x 128 x 16384 96 us with 8 waves of 32 x 16 against 123 with
+  // 4 of 32 x 32)
   if (sk.tile == 32)
     launch_splitk_tiles<E, 32, TileCfg<E>::BK_32_LONG, 2, 2>(stream, p, a_k,
                                                              b_k, sk, W);
   else
-    launch_splitk_tiles<E, 64, TileCfg<E>::BK_SMALL, 2, 4>(stream, p, a_k,
-                                                           b_k, sk, W);
+    launch_splitk_tiles<E, 64, TileCfg<E>::BK_64, 2,
+                        sizeof(typename ElemT<E>::T) == 2 ? 2 : 4>(
+        stream, p, a_k, b_k, sk, W);
   hcblasStatus_t st = launch_status();
   if (st != HCBLAS_STATUS_SUCCESS) return st;
   const int64_t MN = (int64_t)p.M * p.N;
