@@ -73,8 +73,6 @@ struct hcblasContext {
   // apart from gemm_ws: a split complex GEMM reads the embedding while it
   // writes the planes).
   hcb::Workspace split_ws;
-  // FP32 copies of BF16 operands for the adjoint GEMMs.
-  hcb::Workspace adj_ws;
   // Split-K partial tiles of the plain GEMM.
   hcb::Workspace kpart_ws;
   // This device's address of the fixed scratch of hcblas_gemv_noalloc.

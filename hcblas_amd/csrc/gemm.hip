@@ -601,7 +601,7 @@ hcblasStatus_t mixed_gemm(hcblasHandle_t h, hcblasOrder_t order,
     return HCBLAS_STATUS_INVALID_VALUE;
   // the row-major form swaps the operands
   const bool a_f32 = order == HCBLAS_COL_MAJOR ? p_f32 : !p_f32;
-  return gemm_mixed_bf16(h, c, a_f32, alpha, C, true, ldc, sC, batch);
+  return gemm_mixed_bf16(h, c, a_f32, alpha, C, ldc, sC, batch);
 }
 
 }  // namespace

@@ -300,6 +300,11 @@ struct TileLoader {
     return !KCONT && R >= VEC && R % VEC != 0 ? VEC - R % VEC : 0;
   }
 
+  // First row of that vector (R if there is none).
+  __device__ __forceinline__ static int edge_row(int R) {
+    return edge_shift(R) ? R - R % VEC : R;
+  }
+
   // A wide operand's step at k0: FULL if it lies entirely inside [0, K),
   // else mask() has to follow before the LDS store. Rows past R read row r0
   // (k-contiguous) or the last vector; they only feed outputs that are never
@@ -460,7 +465,7 @@ struct TileLoader {
   }
 };
 
-// Tile id -> (tile_m, tile_n): XCD-contiguous slices of a GROUP_M-grouped order.
+// Tile id -> (tile_m, tile_n): XCD-contiguous slices of a GROUP_M-grouped order
 __device__ __forceinline__ void tile_coords(int pid, int tm, int tn,
                                             int &tile_m, int &tile_n) {
   constexpr int kXcd = 8;
@@ -797,8 +802,8 @@ __device__ __forceinline__ void gemm_mainloop(
 //   32x32 FP32/INT32: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32;
 //   16x16 FP32: row 4 (l / 16) + r, column l % 16;
 //   16x16 FP64: row l / 16 + 4 r, column l % 16.
-// shift_m / shift_n: the loaders' edge_shift of either operand. Output row m of
-// the last, partial vector of rows then lies in tile row m + shift_m (and
+// edge_m / shift_m, edge_n / shift_n: the loaders' edge_row and edge_shift of
+// either operand. Output row m >= edge_m lies in tile row m + shift_m (and
 // columns alike); those few rows leave one by one. C is accessed 16 bytes at
 // a time at any alignment.
 // Expects the LDS free on entry (the main loop ends with a barrier) and ends
@@ -809,7 +814,8 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
                                                int64_t ldc, int M, int N,
                                                int m0, int n0, double alpha_d,
                                                double beta_d, int tid,
-                                               char *lds, int shift_m,
+                                               char *lds, int edge_m,
+                                               int shift_m, int edge_n,
                                                int shift_n) {
   using WT = WaveTile<E, BM, BN, WM, WN, MI>;
   using Acc = typename ElemT<E>::Acc;
@@ -832,10 +838,6 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
   const int lrow = lane % MI, lgrp = lane / MI;
   const Acc alpha = (Acc)alpha_d, beta = (Acc)beta_d;
   using GV = typename GlobalVec<OutT>::type;
-  // First row / column of a shifted last vector (M / N when there is none).
-  constexpr int VEC = ElemT<E>::VEC;
-  const int edge_m = shift_m ? M - (VEC - shift_m) : M;
-  const int edge_n = shift_n ? N - (VEC - shift_n) : N;
 #pragma unroll
   for (int c0 = 0; c0 < BN; c0 += NC) {
 #pragma unroll
@@ -890,10 +892,9 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
           __builtin_memcpy(&w, o, 16);
           *reinterpret_cast<GV *>(dst) = w;
         } else {
-          if (m >= edge_m) src += shift_m;
           const int ne = M - m < VE ? M - m : VE;
           for (int e = 0; e < ne; ++e) {
-            Acc v = alpha * src[e];
+            Acc v = alpha * src[m + e < edge_m ? e : e + shift_m];
             if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(dst[e]), v);
             dst[e] = to_out<OutT>(v);
           }
@@ -915,14 +916,14 @@ __device__ __forceinline__ void gemm_tile(
     int n0, int tid, char *lds) {
   using T = typename ElemT<E>::T;
   using WT = WaveTile<E, BM, BN, WM, WN, MI>;
-  constexpr int NTH = 64 * WM * WN;
+  using LA = TileLoader<T, BM, BK, A_K, 64 * WM * WN>;
+  using LB = TileLoader<T, BN, BK, B_K, 64 * WM * WN>;
   typename WT::AccV acc[WT::FM][WT::FN];
   gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, MI, NARROW>(
       A, lda, B, ldb, M, N, K, m0, n0, tid, lds, acc);
   store_tile_lds<E, OutT, BM, BN, WM, WN, MI, LDS_BYTES>(
       acc, C, ldc, M, N, m0, n0, alpha_d, beta_d, tid, lds,
-      TileLoader<T, BM, BK, A_K, NTH>::edge_shift(M),
-      TileLoader<T, BN, BK, B_K, NTH>::edge_shift(N));
+      LA::edge_row(M), LA::edge_shift(M), LB::edge_row(N), LB::edge_shift(N));
 }
 
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
