@@ -465,13 +465,30 @@ struct TileLoader {
   }
 };
 
+// Batch member and tile of a workgroup of a (tiles, 1, batch) grid. Workgroups
+// go to the 8 XCDs in turn, so in whole groups of 8 members each takes all its
+// tiles on one XCD, whose L2 then holds the member's A and B once.
+__device__ __forceinline__ void batch_tile(int tiles, int &z, int &pid) {
+  constexpr int kXcd = 8;
+  z = blockIdx.z;
+  pid = blockIdx.x;
+  if (z < (int)gridDim.z / kXcd * kXcd && tiles < 32768) {  // l < 2^31
+    const unsigned l = (unsigned)z * tiles + pid, i = l / kXcd;
+    z = i / tiles * kXcd + l % kXcd;
+    pid = i % tiles;
+  }
+}
+
 // Tile id -> (tile_m, tile_n): XCD-contiguous slices of a GROUP_M-grouped order
+// (`spread`: consecutive ids are on different XCDs).
 __device__ __forceinline__ void tile_coords(int pid, int tm, int tn,
-                                            int &tile_m, int &tile_n) {
+                                            int &tile_m, int &tile_n,
+                                            bool spread = true) {
   constexpr int kXcd = 8;
   constexpr int GROUP_M = 8;
   const int nt = tm * tn;
-  if (nt % kXcd == 0) pid = (pid % kXcd) * (nt / kXcd) + pid / kXcd;
+  if (spread && nt % kXcd == 0)
+    pid = (pid % kXcd) * (nt / kXcd) + pid / kXcd;
   const int width = GROUP_M * tn;
   const int group = pid / width;
   const int first_m = group * GROUP_M;
@@ -933,7 +950,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
   using T = typename ElemT<E>::T;
   constexpr int LDS_BYTES = tile_lds_bytes<E, BM, BN, BK>();
   __shared__ __attribute__((aligned(16))) char lds[LDS_BYTES];
-  const int z = blockIdx.z;
+  int z, pid;
+  batch_tile(p.tiles_m * p.tiles_n, z, pid);
   const T *A;
   const T *B;
   OutT *C;
@@ -950,7 +968,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
   else
     C = static_cast<OutT *>(p.C) + p.cOff + (int64_t)z * p.strideC;
   int tile_m, tile_n;
-  tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+  tile_coords(pid, p.tiles_m, p.tiles_n, tile_m, tile_n, gridDim.z < 8);
   gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES>(
       A, p.lda, B, p.ldb, C, p.ldc, p.M, p.N, p.K, p.alpha, p.beta,
       tile_m * BM, tile_n * BN, threadIdx.x, lds);

@@ -155,12 +155,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
   // LDS buffer: A region (3 planes if FP32, else 1) then B region
   constexpr int A_BYTES = (AF ? 3 : 1) * PLANE_A;
 
-  const int z = blockIdx.z;
+  int z, pid;
+  batch_tile(p.tiles_m * p.tiles_n, z, pid);
   const TA *A = static_cast<const TA *>(p.A) + (int64_t)z * p.strideA;
   const TB *B = static_cast<const TB *>(p.B) + (int64_t)z * p.strideB;
   Bf16Out *C = static_cast<Bf16Out *>(p.C) + (int64_t)z * p.strideC;
   int tile_m, tile_n;
-  tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+  tile_coords(pid, p.tiles_m, p.tiles_n, tile_m, tile_n, gridDim.z < 8);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
