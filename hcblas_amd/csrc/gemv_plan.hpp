@@ -118,4 +118,45 @@ inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
   return p;
 }
 
+// Launch plan of the GEMV pair kernel (both products of one matrix in one
+// pass): bands of `xr` row steps x blocks of columns; xr == 0 where the two
+// GEMVs are to run instead.
+struct PairPlan {
+  int xr;
+  int64_t bands, blocks;
+  size_t partial_bytes;
+};
+
+// Matrices of 4 MB on whose rows fill a band step to three quarters: below, a
+// GEMV is a launch and little else. Bands as in plan_gemv's row-contiguous case,
+// blocks of 32 to 512 columns for about one workgroup per CU (fp32 4500 x 1000
+// 11.8 us with at least 32 columns, 13.0 with 16, 18.3 with 8 and four
+// workgroups per CU; 4096^2 21.0, 21.0 and 27.5). Against the two GEMVs, both
+// finish launches included: fp32 4096^2 28.2 -> 21.0 us, 1100 x 1000 12.8 -> 9.1,
+// 2500^2 18.4 -> 15.2; fp64 4096^2 48.1 -> 30.4, 700 x 3000 19.0 -> 14.2.
+inline PairPlan plan_gemv_pair(int num_cus, int64_t R, int64_t Cc, int vn,
+                               size_t esize) {
+  PairPlan p{0, 0, 0, 0};
+  const int64_t step = (int64_t)kGemvThreads * vn;
+  const int64_t steps = plan_cdiv(R, step);
+  if (4 * R < 3 * step || Cc < 64 || steps > 65535 ||
+      R * Cc * (int64_t)esize < (4ll << 20))
+    return p;
+  p.xr = 1;
+  for (int x : {4, 2}) {
+    const int64_t b = plan_cdiv(steps, x);
+    if (8 * R >= 7 * b * x * step && b * plan_cdiv(Cc, 32) >= num_cus) {
+      p.xr = x;
+      break;
+    }
+  }
+  p.bands = plan_cdiv(steps, p.xr);
+  p.blocks = std::max<int64_t>(
+      2, std::min(plan_cdiv(Cc, 32), num_cus / p.bands));
+  p.blocks = std::max(p.blocks, plan_cdiv(Cc, 512));
+  p.partial_bytes =
+      esize * (size_t)(p.blocks * R + (p.bands > 1 ? p.bands * Cc : 0));
+  return p;
+}
+
 }  // namespace hcb

@@ -598,29 +598,35 @@ __global__ __launch_bounds__(kThreads) void gemv_scale_y_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// GER: S[r,c] = fma(v[r], alpha*w[c], S[r,c]).
-// Each thread owns VN consecutive rows (one 16-byte vector) and walks kGerCols
+// GER: D[r,c] = fma(v[r], alpha*w[c], S[r,c]), in place (D = S) or into another
+// matrix; alpha == 0 copies. HBM bound: one read of S, one write of D. Each
+// thread owns VN consecutive rows (one 16-byte vector) and walks kGerCols
 // columns, so v stays in registers and every store is a full 16-byte store.
+// (The differentiable update copied S first and updated the copy in place, two
+// reads and two writes: 4096^2 fp32 copy 26 us and update 22; now one launch of
+// 22, 5.9 TB/s.)
 // ---------------------------------------------------------------------------
 constexpr int kGerCols = 16;
 
 template <typename T, bool VEC, bool NT>
 __global__ __launch_bounds__(kThreads) void ger_kernel(
-    int64_t R, int64_t Cc, T *A, int64_t ld, int64_t sA,
-    const T *__restrict__ v, int64_t incv, int64_t sv,
+    int64_t R, int64_t Cc, const T *S, int64_t lds, T *D, int64_t ldd,
+    int64_t sA, const T *__restrict__ v, int64_t incv, int64_t sv,
     const T *__restrict__ w, int64_t incw, int64_t sw, T alpha) {
   constexpr int VN = VEC ? VecT<T>::n : 1;
   const int64_t z = blockIdx.z;
-  A += z * sA;
+  S += z * sA;
+  D += z * sA;
   v += z * sv;
   w += z * sw;
+  const bool add = alpha != T(0);
   const int64_t r0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * VN;
   if (r0 >= R) return;
   const int64_t c0 = (int64_t)blockIdx.y * kGerCols;
   T vr[VN];
 #pragma unroll
   for (int e = 0; e < VN; ++e)
-    vr[e] = (r0 + e < R) ? v[bidx(r0 + e, R, incv)] : T(0);
+    vr[e] = (add && r0 + e < R) ? v[bidx(r0 + e, R, incv)] : T(0);
   const int64_t cend = c0 + kGerCols < Cc ? c0 + kGerCols : Cc;
   if (VEC && r0 + VN <= R) {
     using V = typename VecT<T>::type;
@@ -630,32 +636,157 @@ __global__ __launch_bounds__(kThreads) void ger_kernel(
       // behind them: the compiler cannot prove the columns disjoint).
       V a[kGerCols];
 #pragma unroll
-      for (int j = 0; j < kGerCols; ++j) a[j] = vld<NT>(A + r0 + (c0 + j) * ld);
+      for (int j = 0; j < kGerCols; ++j)
+        a[j] = vld<NT>(S + r0 + (c0 + j) * lds);
 #pragma unroll
       for (int j = 0; j < kGerCols; ++j) {
-        const T t = alpha * w[bidx(c0 + j, Cc, incw)];
+        if (add) {
+          const T t = alpha * w[bidx(c0 + j, Cc, incw)];
 #pragma unroll
-        for (int e = 0; e < VN; ++e) a[j][e] = fma_t(vr[e], t, a[j][e]);
-        vst<NT>(A + r0 + (c0 + j) * ld, a[j]);
+          for (int e = 0; e < VN; ++e) a[j][e] = fma_t(vr[e], t, a[j][e]);
+        }
+        vst<NT>(D + r0 + (c0 + j) * ldd, a[j]);
       }
       return;
     }
     for (int64_t c = c0; c < cend; ++c) {
-      const T t = alpha * w[bidx(c, Cc, incw)];
-      V a = vld<false>(A + r0 + c * ld);
+      V a = vld<false>(S + r0 + c * lds);
+      if (add) {
+        const T t = alpha * w[bidx(c, Cc, incw)];
 #pragma unroll
-      for (int e = 0; e < VN; ++e) a[e] = fma_t(vr[e], t, a[e]);
-      vst<false>(A + r0 + c * ld, a);
+        for (int e = 0; e < VN; ++e) a[e] = fma_t(vr[e], t, a[e]);
+      }
+      vst<false>(D + r0 + c * ldd, a);
     }
   } else {
     for (int64_t c = c0; c < cend; ++c) {
-      const T t = alpha * w[bidx(c, Cc, incw)];
+      const T t = add ? alpha * w[bidx(c, Cc, incw)] : T(0);
 #pragma unroll
-      for (int e = 0; e < VN; ++e) {
-        T *p = A + r0 + e + c * ld;
-        if (r0 + e < R) *p = fma_t(vr[e], t, *p);
-      }
+      for (int e = 0; e < VN; ++e)
+        if (r0 + e < R) {
+          const T a = S[r0 + e + c * lds];
+          D[r0 + e + c * ldd] = add ? fma_t(vr[e], t, a) : a;
+        }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// GEMV pair: both products of one matrix in one pass over it,
+//   yr[r] = alpha * sum_c S[r,c] q[c]   and   yc[c] = alpha * sum_r S[r,c] p[r]
+// (the adjoint of GER). HBM bound, and S is read once instead of twice. A
+// workgroup owns a band of XR row steps and a block of columns, as in the
+// band-N kernel: the band's p and its row sums stay in registers; 32 vectors
+// per thread are in flight, all issued before their FMAs. A column's sum over
+// the band crosses the wave by shuffles into LDS. Both results leave as
+// partials (rows: one per column block, columns: one per band), except the
+// column sums of a single band.
+// ---------------------------------------------------------------------------
+constexpr int kPairCols = 512;  // columns of a block at most
+
+template <typename T, int XR, bool NT>
+__global__ __launch_bounds__(kThreads) void gemv_pair_kernel(
+    int64_t R, int64_t Cc, int64_t ld, const T *__restrict__ S,
+    const T *__restrict__ p, int64_t incp, const T *__restrict__ q,
+    int64_t incq, T alpha, T *yc, T *row_part, T *col_part) {
+  using V = typename VecT<T>::type;
+  constexpr int VN = VecT<T>::n;
+  constexpr int UC = 32 / XR;
+  constexpr int64_t STEP = (int64_t)kThreads * VN;
+  __shared__ T red[4][kPairCols];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t rt = (int64_t)blockIdx.y * XR * STEP +
+                     (int64_t)threadIdx.x * VN;
+  const bool full = ((int64_t)blockIdx.y + 1) * XR * STEP <= R;
+  // Lanes past the edge read the last VN rows; rows below their own belong to
+  // another lane: they count as zeros in the column sums (in p and in S), and
+  // their row sums are not stored.
+  int64_t roff[XR];
+  V pv[XR];
+#pragma unroll
+  for (int u = 0; u < XR; ++u) {
+    const int64_t r = rt + u * STEP;
+    roff[u] = r + VN <= R ? r : R - VN;
+#pragma unroll
+    for (int e = 0; e < VN; ++e)
+      pv[u][e] = roff[u] + e >= r ? p[bidx(roff[u] + e, R, incp)] : T(0);
+  }
+  const int64_t cper = cdiv_dev(Cc, (int64_t)gridDim.x);
+  const int64_t c_begin = (int64_t)blockIdx.x * cper;
+  const int64_t c_end = c_begin + cper < Cc ? c_begin + cper : Cc;
+  T acc[XR][VN];
+#pragma unroll
+  for (int u = 0; u < XR; ++u)
+#pragma unroll
+    for (int e = 0; e < VN; ++e) acc[u][e] = T(0);
+  int64_t c = c_begin;
+  // N columns from c: all loads, then all FMAs.
+  auto columns = [&](auto n) {
+    constexpr int N = decltype(n)::value;
+    V a[N][XR];
+    T qv[N], sum[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      qv[j] = q[bidx(c + j, Cc, incq)];
+      const T *col = S + (c + j) * ld;
+#pragma unroll
+      for (int u = 0; u < XR; ++u) a[j][u] = vld<NT>(col + roff[u]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      T t[VN];
+#pragma unroll
+      for (int e = 0; e < VN; ++e) t[e] = T(0);
+#pragma unroll
+      for (int u = 0; u < XR; ++u)
+#pragma unroll
+        for (int e = 0; e < VN; ++e) {
+          const T x = vlane<T>(a[j][u], e);
+          acc[u][e] = fma_t(x, qv[j], acc[u][e]);
+          const bool own = full || roff[u] + e >= rt + u * STEP;
+          t[e] = fma_t(own ? x : T(0), vlane<T>(pv[u], e), t[e]);
+        }
+      sum[j] = t[0];
+#pragma unroll
+      for (int e = 1; e < VN; ++e) sum[j] += t[e];
+    }
+    // The N column sums cross the wave together: each halving of the lanes
+    // also halves the columns a lane holds (N = 16: 17 shuffles, not 96).
+    int width = 32;
+#pragma unroll
+    for (int h = N / 2; h >= 1; h /= 2, width /= 2)
+#pragma unroll
+      for (int i = 0; i < h; ++i) {
+        const bool up = lane & width;
+        const T give = up ? sum[i] : sum[i + h];
+        sum[i] = (up ? sum[i + h] : sum[i]) + __shfl_xor(give, width, 64);
+      }
+#pragma unroll
+    for (; width >= 1; width /= 2) sum[0] += __shfl_xor(sum[0], width, 64);
+    constexpr int LPC = 64 / N;  // lanes that hold a column's sum
+    if (lane % LPC == 0) red[wave][c - c_begin + lane / LPC] = sum[0];
+    c += N;
+  };
+  while (c + UC <= c_end) columns(std::integral_constant<int, UC>{});
+  while (c + 4 <= c_end) columns(std::integral_constant<int, 4>{});
+  while (c < c_end) columns(std::integral_constant<int, 1>{});
+  T *rp = row_part + (int64_t)blockIdx.x * R;
+#pragma unroll
+  for (int u = 0; u < XR; ++u) {
+    const int64_t r = rt + u * STEP;
+    if (r >= R) continue;
+#pragma unroll
+    for (int e = 0; e < VN; ++e)
+      if (roff[u] + e >= r) rp[roff[u] + e] = acc[u][e];
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < (int)(c_end - c_begin); j += kThreads) {
+    const T v = ((red[0][j] + red[1][j]) + red[2][j]) + red[3][j];
+    if (gridDim.y == 1)
+      yc[c_begin + j] = alpha * v;
+    else
+      col_part[(int64_t)blockIdx.y * Cc + c_begin + j] = v;
   }
 }
 
@@ -840,7 +971,8 @@ hcblasStatus_t ger_entry(hcblasHandle_t h, hcblasOrder_t order, int M, int N,
                          int64_t incy, T *A, int64_t aOffset, int64_t lda,
                          int64_t batch, bool ref_batch_strides = true,
                          int64_t sA_in = 0, int64_t sx_in = 0,
-                         int64_t sy_in = 0) {
+                         int64_t sy_in = 0, const T *src = nullptr,
+                         int64_t lds = 0) {
   if (!handle_ok(h)) return HCBLAS_STATUS_NOT_INITIALIZED;
   if (M < 0 || N < 0 || incx == 0 || incy == 0 || batch < 0)
     return HCBLAS_STATUS_INVALID_VALUE;
@@ -852,7 +984,11 @@ hcblasStatus_t ger_entry(hcblasHandle_t h, hcblasOrder_t order, int M, int N,
   if (M == 0 || N == 0 || batch == 0) return HCBLAS_STATUS_SUCCESS;
   if (alpha == nullptr || x == nullptr || y == nullptr || A == nullptr)
     return HCBLAS_STATUS_INVALID_VALUE;
-  if (*alpha == T(0)) return HCBLAS_STATUS_SUCCESS;  // netlib quick return
+  if (src == nullptr) {
+    if (*alpha == T(0)) return HCBLAS_STATUS_SUCCESS;  // netlib quick return
+    src = A + aOffset;
+    lds = lda;
+  }
   // Batch strides as in hcblas.cpp:1160-1167 (x by M, y by N, A by M*N), or
   // the caller's explicit batch offsets.
   const bool multi = batch > 1;
@@ -872,35 +1008,68 @@ hcblasStatus_t ger_entry(hcblasHandle_t h, hcblasOrder_t order, int M, int N,
   // and only adds write-back traffic (DGER 8192^2: 6.09 against 5.6 TB/s).
   // One that fits keeps the cached path, which the next call re-reads from
   // the MALL (SGER 8192^2: 6.87 cached against 6.10 non-temporal).
-  const bool nt =
-      (int64_t)lda * Cc * batch * (int64_t)sizeof(T) > (256ll << 20);
+  // (Into another matrix both count.)
+  const int64_t footprint = src == A + aOffset ? lda : lda + lds;
+  const bool nt = footprint * Cc * batch * (int64_t)sizeof(T) > (256ll << 20);
   for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
     int64_t nb = std::min<int64_t>(65535, batch - b0);
     dim3 grid((unsigned)cdiv(R, rows_per_block),
               (unsigned)cdiv(Cc, kGerCols), (unsigned)nb);
     if (vec && nt)
       ger_kernel<T, true, true><<<grid, kThreads, 0, h->stream>>>(
-          R, Cc, Ab + b0 * sA, lda, sA, v + b0 * sv, incv, sv, w + b0 * sw,
-          incw, sw, *alpha);
+          R, Cc, src + b0 * sA, lds, Ab + b0 * sA, lda, sA, v + b0 * sv, incv,
+          sv, w + b0 * sw, incw, sw, *alpha);
     else if (vec)
       ger_kernel<T, true, false><<<grid, kThreads, 0, h->stream>>>(
-          R, Cc, Ab + b0 * sA, lda, sA, v + b0 * sv, incv, sv, w + b0 * sw,
-          incw, sw, *alpha);
+          R, Cc, src + b0 * sA, lds, Ab + b0 * sA, lda, sA, v + b0 * sv, incv,
+          sv, w + b0 * sw, incw, sw, *alpha);
     else
       ger_kernel<T, false, false><<<grid, kThreads, 0, h->stream>>>(
-          R, Cc, Ab + b0 * sA, lda, sA, v + b0 * sv, incv, sv, w + b0 * sw,
-          incw, sw, *alpha);
+          R, Cc, src + b0 * sA, lds, Ab + b0 * sA, lda, sA, v + b0 * sv, incv,
+          sv, w + b0 * sw, incw, sw, *alpha);
     hcblasStatus_t st = launch_status();
     if (st != HCBLAS_STATUS_SUCCESS) return st;
   }
   return HCBLAS_STATUS_SUCCESS;
 }
 
+// Workspace of the pair kernel. False where it would have to grow while the
+// stream is being captured, or cannot: the two GEMVs then run instead.
+bool pair_workspace(hcblasHandle_t h, size_t bytes) {
+  if (h->gemv_partials.bytes >= bytes) return true;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(h->stream, &cs) != hipSuccess ||
+      cs != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (ensure_workspace(h->gemv_partials, bytes) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+// GER from one matrix into another, D = alpha * x * y^T + A.
+template <typename T>
+hcblasStatus_t ger_out_entry(hcblasHandle_t h, hcblasOrder_t order, int M,
+                             int N, const T *alpha, const T *x, int64_t incx,
+                             const T *y, int64_t incy, const T *A, int64_t lda,
+                             T *D, int64_t ldd) {
+  if (!handle_ok(h)) return HCBLAS_STATUS_NOT_INITIALIZED;
+  if (order != HCBLAS_ROW_MAJOR && order != HCBLAS_COL_MAJOR)
+    return HCBLAS_STATUS_INVALID_VALUE;
+  if (lda < std::max(1, order == HCBLAS_COL_MAJOR ? M : N))
+    return HCBLAS_STATUS_INVALID_VALUE;
+  if (M > 0 && N > 0 && A == nullptr) return HCBLAS_STATUS_INVALID_VALUE;
+  return ger_entry<T>(h, order, M, N, alpha, x, 0, incx, y, 0, incy, D, 0, ldd,
+                      1, true, 0, 0, 0, A, lda);
+}
+
 // Adjoint of A_out = alpha * x * y^T + A_in (no reference counterpart): for
 // a cotangent dA (M x N in the given order) the GEMV pair
 //   dx = alpha * dA * y,   dy = alpha * dA^T * x
 // (dA_in = dA is the identity and needs no work). dx / dy are written with
-// unit stride; either may be NULL.
+// unit stride; either may be NULL. With both wanted of a matrix that the pair
+// kernel covers, dA is read once.
 template <typename T>
 hcblasStatus_t ger_backward_entry(hcblasHandle_t h, hcblasOrder_t order,
                                          int M, int N, const T *alpha,
@@ -910,6 +1079,43 @@ hcblasStatus_t ger_backward_entry(hcblasHandle_t h, hcblasOrder_t order,
   if (!handle_ok(h)) return HCBLAS_STATUS_NOT_INITIALIZED;
   const T zero = T(0);
   hcblasStatus_t st = HCBLAS_STATUS_SUCCESS;
+  const bool col = order == HCBLAS_COL_MAJOR;
+  const int64_t R = col ? M : N, Cc = col ? N : M;
+  if (dx && dy && x && y && dA && alpha && *alpha != zero && M > 0 && N > 0 &&
+      incx != 0 && incy != 0 && ldda >= R &&
+      (col || order == HCBLAS_ROW_MAJOR)) {
+    const PairPlan plan =
+        plan_gemv_pair(h->num_cus, R, Cc, VecT<T>::n, sizeof(T));
+    if (plan.xr && pair_workspace(h, plan.partial_bytes)) {
+      const T *p = col ? x : y, *q = col ? y : x;
+      const int64_t incp = col ? incx : incy, incq = col ? incy : incx;
+      T *yr = col ? dx : dy, *yc = col ? dy : dx;
+      T *row_part = static_cast<T *>(h->gemv_partials.ptr);
+      T *col_part = row_part + plan.blocks * R;
+      const dim3 grid((unsigned)plan.blocks, (unsigned)plan.bands);
+      const bool nt = (int64_t)sizeof(T) * R * Cc >= kStreamBytes;
+#define HCB_PAIR(XR)                                                         \
+  (nt ? gemv_pair_kernel<T, XR, true> : gemv_pair_kernel<T, XR, false>)      \
+      <<<grid, kThreads, 0, h->stream>>>(R, Cc, ldda, dA, p, incp, q, incq,  \
+                                         *alpha, yc, row_part, col_part)
+      if (plan.xr == 4)
+        HCB_PAIR(4);
+      else if (plan.xr == 2)
+        HCB_PAIR(2);
+      else
+        HCB_PAIR(1);
+#undef HCB_PAIR
+      if ((st = launch_status()) != HCBLAS_STATUS_SUCCESS) return st;
+      auto finish = [&](int64_t len, int64_t splits, const T *part, T *out) {
+        gemv_finish_kernel<T>
+            <<<(unsigned)std::min<int64_t>(cdiv(len, 64), 4096), kThreads, 0,
+               h->stream>>>(len, (int)splits, part, 0, out, 1, 0, *alpha, zero);
+      };
+      finish(R, plan.blocks, row_part, yr);
+      if (plan.bands > 1) finish(Cc, plan.bands, col_part, yc);
+      return launch_status();
+    }
+  }
   if (dx) {
     st = gemv_entry<T>(h, order, HCBLAS_OP_N, M, N, alpha, dA, 0, ldda, y, 0,
                        incy, &zero, dx, 0, 1, 1, false);
@@ -1088,6 +1294,23 @@ hcblasStatus_t hcblas_gemv_noalloc(hcblasHandle_t handle,
         static_cast<const double *>(beta), static_cast<double *>(Y), yOffset,
         incY, 1, false, 0, 0, 0, true);
   return HCBLAS_STATUS_INVALID_VALUE;
+}
+
+hcblasStatus_t hcblas_sger_out(hcblasHandle_t handle, hcblasOrder_t order,
+                               int M, int N, const float *alpha,
+                               const float *X, int64_t incX, const float *Y,
+                               int64_t incY, const float *A, int64_t lda,
+                               float *D, int64_t ldd) {
+  return ger_out_entry<float>(handle, order, M, N, alpha, X, incX, Y, incY, A,
+                              lda, D, ldd);
+}
+hcblasStatus_t hcblas_dger_out(hcblasHandle_t handle, hcblasOrder_t order,
+                               int M, int N, const double *alpha,
+                               const double *X, int64_t incX, const double *Y,
+                               int64_t incY, const double *A, int64_t lda,
+                               double *D, int64_t ldd) {
+  return ger_out_entry<double>(handle, order, M, N, alpha, X, incX, Y, incY, A,
+                               lda, D, ldd);
 }
 
 hcblasStatus_t hcblas_sger_backward(hcblasHandle_t handle,

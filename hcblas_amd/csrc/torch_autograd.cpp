@@ -197,20 +197,22 @@ class GerFn : public torch::autograd::Function<GerFn> {
                 "hcblas.ger: types differ");
     x = x.contiguous();
     y = y.contiguous();
-    Tensor out = A.contiguous().clone();
+    const Tensor in = A.resolve_neg().contiguous();
+    Tensor out = torch::empty_like(in);
     const int M = (int)A.size(0), N = (int)A.size(1);
     hcblasHandle_t h = handle_for(A);
     if (A.scalar_type() == torch::kFloat32) {
       const float a = (float)alpha;
-      check(hcblas_sger(h, HCBLAS_ROW_MAJOR, M, N, &a, x.data_ptr<float>(), 0, 1,
-                        y.data_ptr<float>(), 0, 1, out.data_ptr<float>(), 0, N),
-            "hcblas_sger");
+      check(hcblas_sger_out(h, HCBLAS_ROW_MAJOR, M, N, &a, x.data_ptr<float>(), 1,
+                            y.data_ptr<float>(), 1, in.data_ptr<float>(), N,
+                            out.data_ptr<float>(), N),
+            "hcblas_sger_out");
     } else {
       TORCH_CHECK(A.scalar_type() == torch::kFloat64, "hcblas.ger: float32 or float64 only");
-      check(hcblas_dger(h, HCBLAS_ROW_MAJOR, M, N, &alpha, x.data_ptr<double>(), 0,
-                        1, y.data_ptr<double>(), 0, 1, out.data_ptr<double>(), 0,
-                        N),
-            "hcblas_dger");
+      check(hcblas_dger_out(h, HCBLAS_ROW_MAJOR, M, N, &alpha, x.data_ptr<double>(),
+                            1, y.data_ptr<double>(), 1, in.data_ptr<double>(), N,
+                            out.data_ptr<double>(), N),
+            "hcblas_dger_out");
     }
     ctx->save_for_backward({x, y});
     ctx->saved_data["alpha"] = alpha;

@@ -737,6 +737,20 @@ hcblasStatus_t hcblas_gemm_strided_batched_backward(
     int64_t strideDA, void *dB, int64_t lddb, int64_t strideDB, void *dCin,
     int64_t lddcin, int64_t strideDCin, int batchCount);
 
+/* hcblas_sger / hcblas_dger from one matrix into another:
+ * D = alpha * x * y^T + A (M x N in the given order; alpha == 0 copies A). D is
+ * A itself or does not overlap it. */
+hcblasStatus_t hcblas_sger_out(hcblasHandle_t handle, hcblasOrder_t order,
+                               int M, int N, const float *alpha,
+                               const float *X, int64_t incX, const float *Y,
+                               int64_t incY, const float *A, int64_t lda,
+                               float *D, int64_t ldd);
+hcblasStatus_t hcblas_dger_out(hcblasHandle_t handle, hcblasOrder_t order,
+                               int M, int N, const double *alpha,
+                               const double *X, int64_t incX, const double *Y,
+                               int64_t incY, const double *A, int64_t lda,
+                               double *D, int64_t ldd);
+
 /* Adjoint of hcblas_sger / hcblas_dger, A_out = alpha * x * y^T + A_in, for a
  * cotangent dA (M x N in the given order): dx = alpha * dA * y and
  * dy = alpha * dA^T * x, written with unit stride (either may be NULL);

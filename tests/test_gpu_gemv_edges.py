@@ -97,3 +97,91 @@ def test_ger_any_alignment(hc, handle, orc, p):
         exp[1:1 + M * N] = orc.ger(COL, M, N, 1.5, x, 1, y, 1,
                                    A[1:1 + M * N].copy(), M)
         assert bitwise_equal(to_host(dA), exp), (M, N)
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+def test_ger_out(hc, handle, orc, p):
+    """D = alpha x y^T + A: bit-exact as GER in place, other leading dimensions
+    for A and D, A left alone; alpha == 0 copies A, also beside an infinity."""
+    dt = DT[p]
+    for M, N in [(1, 17), (3, 16), (5, 33), (1025, 40), (2051, 16)]:
+        for order in (COL, ROW):
+            rng = np.random.default_rng(M + N)
+            R, Cc = (M, N) if order == COL else (N, M)
+            lda, ldd = R + 3, R + 1
+            A = rng.uniform(-1, 1, lda * Cc + 1).astype(dt)
+            D = rng.uniform(-1, 1, ldd * Cc + 1).astype(dt)
+            x = rng.uniform(-1, 1, M).astype(dt)
+            y = rng.uniform(-1, 1, 2 * N).astype(dt)
+            for alpha in (1.5, 0.0):
+                if alpha == 0.0:
+                    x[0] = np.inf
+                dA, dD = to_dev(A), to_dev(D)
+                st = getattr(hc.api, f"hcblas_{p}ger_out")(
+                    handle, order, M, N, alpha, to_dev(x), 1, to_dev(y), -2,
+                    dA[1:], lda, dD[1:], ldd)
+                assert st == 0
+                exp = D.copy()
+                e = exp[1:].reshape(Cc, ldd)
+                e[:, :R] = A[1:].reshape(Cc, lda)[:, :R]
+                if alpha:
+                    t = orc.ger(order, M, N, alpha, x, 1, y, -2,
+                                np.ascontiguousarray(e[:, :R]).ravel(), R)
+                    e[:, :R] = t.reshape(Cc, R)
+                assert bitwise_equal(to_host(dD), exp), (M, N, order, alpha)
+                assert bitwise_equal(to_host(dA), A)
+
+
+# Storage rows R and columns of the pair kernel: 4 MB and just below; bands of
+# 1, 2 and 4 row steps with partial last vectors, steps and bands; several
+# bands and one; blocks of fewer columns than a trip, and one of 512.
+PAIR = [(767, 1400), (769, 1401), (1023, 1021), (1027, 1030), (4096, 259),
+        (4099, 300), (5003, 257), (8193, 130), (16389, 64), (30001, 77),
+        (1025, 9001)]
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+def test_ger_backward_pair(hc, handle, p):
+    dt = DT[p]
+    eps = np.finfo(dt).eps
+    for R, Cc in PAIR:
+        rng = np.random.default_rng(R + Cc)
+        m = rng.uniform(-1, 1, (Cc, R + 1)).astype(dt)  # ld = R + 1
+        S = m[:, :R].T.astype(np.float64)
+        dS = to_dev(np.concatenate([np.zeros(1, dt), m.ravel()]))
+        a = rng.uniform(-1, 1, R).astype(dt)
+        b = rng.uniform(-1, 1, Cc).astype(dt)
+        for order in (COL, ROW):
+            M, N = (R, Cc) if order == COL else (Cc, R)
+            x, y = (a, b) if order == COL else (b, a)
+            ys = np.zeros(2 * N - 1, dt)
+            ys[::2] = y[::-1]
+            dx, dy = to_dev(np.full(M, 7, dt)), to_dev(np.full(N, 7, dt))
+            st = getattr(hc.api, f"hcblas_{p}ger_backward")(
+                handle, order, M, N, 1.5, to_dev(x), 1, to_dev(ys), -2,
+                dS[1:], R + 1, dx, dy)
+            assert st == 0
+            G = S if order == COL else S.T
+            for got, op, v in ((dx, G, y), (dy, G.T, x)):
+                v = v.astype(np.float64)
+                bound = (len(v) + 2) * eps * 1.5 * (abs(op) @ abs(v))
+                assert np.all(abs(to_host(got) - 1.5 * (op @ v)) <= bound), \
+                    (R, Cc, order)
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+def test_pair_edge_rows_do_not_leak(hc, handle, p):
+    """As test_edge_rows_do_not_leak, through the adjoint of GER."""
+    dt = DT[p]
+    for R, Cc in [(1027, 1100), (20011, 80)]:
+        m = np.ones((Cc, R), dt)
+        m[:, R - 2] = np.inf
+        dx, dy = to_dev(np.zeros(R, dt)), to_dev(np.zeros(Cc, dt))
+        st = getattr(hc.api, f"hcblas_{p}ger_backward")(
+            handle, COL, R, Cc, 1.0, to_dev(np.ones(R, dt)), 1,
+            to_dev(np.ones(Cc, dt)), 1, to_dev(m), R, dx, dy)
+        assert st == 0
+        assert np.all(to_host(dy) == np.inf), (R, Cc)
+        exp = np.full(R, Cc, dt)
+        exp[R - 2] = np.inf
+        assert np.array_equal(to_host(dx), exp), (R, Cc)
