@@ -20,7 +20,9 @@
 // times the 2K x N real view of op(B) (rows alternate re/im) gives the 2M x N
 // real view of the interleaved complex product, i.e. C itself with
 // ldc_real = 2*ldc. This is the 4-real-product method (8MNK flops); alpha is
-// folded into the A embedding (netlib folds it into B: temp = alpha*B(l,j)).
+// folded into the A embedding (netlib folds it into B: temp = alpha*B(l,j)). The
+// tile loaders form both real matrices on their way into LDS; the split
+// precision modes, which read them several times, write them to a workspace.
 #include <cstring>
 
 #include "gemm_common.hpp"
@@ -261,12 +263,15 @@ inline int grid_for(int64_t work, int num_cus) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// Real / half GEMM driver.
+// Real / half GEMM driver. CX: the real form of a complex product (sizes,
+// offsets and strides are the real form's, leading dimensions the complex
+// operands'), whose operands the tile loaders embed with cx.
 // ---------------------------------------------------------------------------
-template <Elem E, typename OutT>
-hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
-                         double beta, void *C, int64_t ldc, int64_t cOff,
-                         int64_t strideC, void *const *Cptrs, int64_t batch) {
+template <Elem E, typename OutT, bool CX>
+hcblasStatus_t run_gemm(hcblasHandle_t h, const Canon &c, double alpha,
+                        double beta, void *C, int64_t ldc, int64_t cOff,
+                        int64_t strideC, void *const *Cptrs, int64_t batch,
+                        const ComplexArgs &cx) {
   using Acc = typename ElemT<E>::Acc;
   if (c.M == 0 || c.N == 0 || batch == 0) return HCBLAS_STATUS_SUCCESS;
   if (C == nullptr && Cptrs == nullptr) return HCBLAS_STATUS_INVALID_VALUE;
@@ -307,6 +312,10 @@ hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
   p.cOff = cOff;
   p.alpha = alpha;
   p.beta = beta;
+  p.cx_ar = cx.ar;
+  p.cx_ai = cx.ai;
+  p.conj_a = cx.conj_a;
+  p.conj_b = cx.conj_b;
   if (batch == 1 && !c.Aptrs && !c.Bptrs && !Cptrs) {
     const SplitK sk =
         splitk_plan(c.M, c.N, c.K, h->num_cus, E == Elem::F64 ? 64 : 128,
@@ -315,12 +324,21 @@ hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
       const size_t bytes = sizeof(Acc) * (size_t)sk.splits * c.M * c.N;
       if (ensure_workspace(h->kpart_ws, bytes) != hipSuccess)
         return HCBLAS_STATUS_ALLOC_FAILED;
-      return launch_gemm_splitk<E, OutT>(h->stream, h->num_cus, p, c.a_k,
-                                         c.b_k, sk,
-                                         static_cast<Acc *>(h->kpart_ws.ptr));
+      return launch_gemm_splitk<E, OutT, CX>(
+          h->stream, h->num_cus, p, c.a_k, c.b_k, sk,
+          static_cast<Acc *>(h->kpart_ws.ptr));
     }
   }
-  return launch_gemm<E, OutT>(h->stream, h->num_cus, p, c.a_k, c.b_k, batch);
+  return launch_gemm<E, OutT, CX>(h->stream, h->num_cus, p, c.a_k, c.b_k,
+                                  batch);
+}
+
+template <Elem E, typename OutT>
+hcblasStatus_t gemm_real(hcblasHandle_t h, const Canon &c, double alpha,
+                         double beta, void *C, int64_t ldc, int64_t cOff,
+                         int64_t strideC, void *const *Cptrs, int64_t batch) {
+  return run_gemm<E, OutT, false>(h, c, alpha, beta, C, ldc, cOff, strideC,
+                                  Cptrs, batch, ComplexArgs{});
 }
 
 // ---------------------------------------------------------------------------
@@ -357,6 +375,23 @@ hcblasStatus_t gemm_complex(hcblasHandle_t h, const Canon &c, T ar, T ai,
   if ((c.A == nullptr && c.Aptrs == nullptr) ||
       (c.B == nullptr && c.Bptrs == nullptr))
     return HCBLAS_STATUS_INVALID_VALUE;
+
+  // The plain math mode embeds the operands in the tile loaders.
+  const int split_modes = E == Elem::F32
+                              ? HCBLAS_OZAKI_CRT_F32_MATH | HCBLAS_SPLIT_BF16_MATH
+                              : HCBLAS_OZAKI_CRT_MATH | HCBLAS_OZAKI_INT8_MATH;
+  if (!(h->math_mode & split_modes)) {
+    Canon r = c;
+    r.M = 2 * c.M;
+    r.K = 2 * c.K;
+    r.aOff = 2 * c.aOff;
+    r.strideA = 2 * c.strideA;
+    r.bOff = 2 * c.bOff;
+    r.strideB = 2 * c.strideB;
+    return run_gemm<E, T, true>(
+        h, r, 1.0, (double)br, C, 2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch,
+        ComplexArgs{(double)ar, (double)ai, c.conj_a, c.conj_b});
+  }
 
   // Workspace: Ar (2M x ldr per batch), Br (N x ldr per batch) if packed.
   const int64_t ldr = (2 * (int64_t)c.K + 15) / 16 * 16;
@@ -424,19 +459,15 @@ hcblasStatus_t gemm_complex(hcblasHandle_t h, const Canon &c, T ar, T ai,
     if (h->math_mode & HCBLAS_OZAKI_CRT_F32_MATH)
       return gemm_ozaki_crt_f32(h, r, 1.f, (float)br, static_cast<float *>(C),
                                 2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch);
-    if (h->math_mode & HCBLAS_SPLIT_BF16_MATH)
-      return gemm_split_bf16(h, r, 1.f, (float)br, static_cast<float *>(C),
-                             2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch);
+    return gemm_split_bf16(h, r, 1.f, (float)br, static_cast<float *>(C),
+                           2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch);
   } else {
     if (h->math_mode & HCBLAS_OZAKI_CRT_MATH)
       return gemm_ozaki_crt(h, r, 1.0, (double)br, static_cast<double *>(C),
                             2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch);
-    if (h->math_mode & HCBLAS_OZAKI_INT8_MATH)
-      return gemm_ozaki_int8(h, r, 1.0, (double)br, static_cast<double *>(C),
-                             2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch);
+    return gemm_ozaki_int8(h, r, 1.0, (double)br, static_cast<double *>(C),
+                           2 * ldc, 2 * cOff, 2 * strideC, Cptrs, batch);
   }
-  return gemm_real<E, T>(h, r, 1.0, (double)br, C, 2 * ldc, 2 * cOff,
-                         2 * strideC, Cptrs, batch);
 }
 
 template hcblasStatus_t gemm_real<Elem::F32, float>(hcblasHandle_t,

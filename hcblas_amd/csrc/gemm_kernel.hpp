@@ -31,6 +31,8 @@
 #pragma once
 
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace hcb {
@@ -116,6 +118,8 @@ template <>
 struct GlobalVecOf<4> { typedef vec4u type __attribute__((aligned(4))); };
 template <>
 struct GlobalVecOf<8> { typedef vec4u type __attribute__((aligned(8))); };
+template <>
+struct GlobalVecOf<16> { typedef vec4u type __attribute__((aligned(8))); };
 template <typename T>
 using GlobalVec = GlobalVecOf<(int)sizeof(T)>;
 
@@ -465,6 +469,139 @@ struct TileLoader {
   }
 };
 
+// Loader of a complex operand for the real embedding of a complex product. Its
+// rows, k and step are those of the real operands,
+//   EMBED (A'):  rows 2m, 2m + 1 of columns 2k, 2k + 1 hold (x, -y; y, x) with
+//                x + iy = (ar + i ai) * a(m, k), the products rounded
+//                separately;
+//   else (B'):   row n of columns 2k, 2k + 1 holds re b(k, n), im b(k, n);
+// a and b conjugated if asked. The operand is read in complex elements (the
+// loader above, on 8- or 16-byte elements) and takes this form on its way into
+// LDS. (Written to memory by a pass of its own, four reals for each complex
+// element of A', it cost two launches and 6 MK + 4 KN complex elements of
+// traffic: sixty-four 96^3 CGEMMs 22.9 us, now 10.9; 1024^3 NT 102 -> 95; 300^3
+// ZGEMM NN 32 -> 13.)
+typedef double doublex2 __attribute__((ext_vector_type(2)));
+template <typename T>
+using ComplexElem =
+    typename std::conditional<sizeof(T) == 4, double, doublex2>::type;
+template <typename T, int ROWS, int BK, bool KCONT, int NTH, bool EMBED>
+struct ComplexLoader
+    : TileLoader<ComplexElem<T>, EMBED ? ROWS / 2 : ROWS, BK / 2, KCONT, NTH> {
+  using L =
+      TileLoader<ComplexElem<T>, EMBED ? ROWS / 2 : ROWS, BK / 2, KCONT, NTH>;
+  using CT = ComplexElem<T>;
+  static constexpr int RD = EMBED ? 2 : 1;  // real rows per complex row
+  static constexpr int ROWB = BK * (int)sizeof(T) + 16;
+  const uint32_t flip;  // sign bit where the operand is conjugated
+  const T ar, ai;
+  int kv;  // k of the held step inside K (complex)
+
+  __device__ __forceinline__ ComplexLoader(int t, bool conj, T r, T i)
+      : L(t), flip(conj ? 0x80000000u : 0u), ar(r), ai(i) {}
+
+  __device__ __forceinline__ static bool wide(int R, int K) {
+    return L::wide(R / RD, K / 2);
+  }
+  __device__ __forceinline__ static int edge_shift(int R) {
+    return RD * L::edge_shift(R / RD);
+  }
+  __device__ __forceinline__ static int edge_row(int R) {
+    return RD * L::edge_row(R / RD);
+  }
+  template <bool FULL>
+  __device__ __forceinline__ void load_wide(const T *P, int64_t ld, int r0,
+                                            int k0, int R, int K) {
+    kv = FULL ? BK / 2 : (K - k0) / 2;
+    L::template load_wide<FULL>(reinterpret_cast<const CT *>(P), ld, r0 / RD,
+                                k0 / 2, R / RD, K / 2);
+  }
+  __device__ __forceinline__ void load_narrow(const T *P, int64_t ld, int r0,
+                                              int k0, int R, int K) {
+    kv = (K - k0) / 2;
+    L::load_narrow(reinterpret_cast<const CT *>(P), ld, r0 / RD, k0 / 2,
+                   R / RD, K / 2);
+  }
+  __device__ __forceinline__ void mask(int k0, int K) { L::mask(k0 / 2, K / 2); }
+
+  __device__ __forceinline__ void store(char *lds) const {
+#pragma clang fp contract(off)
+    constexpr int VC = L::VEC;  // complex elements per vector
+#pragma unroll
+    for (int i = 0; i < L::PER_THREAD; ++i) {
+      const int v = this->tid + i * NTH;
+      if (L::NV % NTH != 0 && v >= L::NV) continue;
+      int r, k;
+      L::vec_pos(v, r, k);
+      char *p = lds + RD * r * ROWB + 2 * k * (int)sizeof(T);
+      vec4u w = this->reg[i];
+      if constexpr (VC == 2) w.y ^= flip;
+      w.w ^= flip;
+      if constexpr (EMBED) {
+        T x[VC], y[VC], c[2 * VC];
+        __builtin_memcpy(c, &w, 16);
+#pragma unroll
+        for (int e = 0; e < VC; ++e) {
+          // (steps past K stay zero whatever alpha is)
+          const bool in = k + (KCONT ? e : 0) < kv;
+          const T sr = in ? ar : T(0), si = in ? ai : T(0);
+          x[e] = sr * c[2 * e] - si * c[2 * e + 1];
+          y[e] = sr * c[2 * e + 1] + si * c[2 * e];
+        }
+        if constexpr (VC == 2 && KCONT) {
+          const T t0[4] = {x[0], -y[0], x[1], -y[1]};
+          const T t1[4] = {y[0], x[0], y[1], x[1]};
+          *reinterpret_cast<vec4u *>(p) = bitcast<vec4u>(t0);
+          *reinterpret_cast<vec4u *>(p + ROWB) = bitcast<vec4u>(t1);
+        } else {
+          using W = typename std::conditional<VC == 2, vec2u, vec4u>::type;
+#pragma unroll
+          for (int e = 0; e < VC; ++e) {
+            const T t0[2] = {x[e], -y[e]}, t1[2] = {y[e], x[e]};
+            *reinterpret_cast<W *>(p + 2 * e * ROWB) = bitcast<W>(t0);
+            *reinterpret_cast<W *>(p + (2 * e + 1) * ROWB) = bitcast<W>(t1);
+          }
+        }
+      } else if constexpr (VC == 2 && !KCONT) {
+        *reinterpret_cast<vec2u *>(p) = vec2u{w.x, w.y};
+        *reinterpret_cast<vec2u *>(p + ROWB) = vec2u{w.z, w.w};
+      } else {
+        *reinterpret_cast<vec4u *>(p) = w;
+      }
+    }
+  }
+};
+
+// alpha and the conjugations of a complex product.
+struct ComplexArgs {
+  double ar, ai;
+  int conj_a, conj_b;
+};
+
+// The loader pair of a product: real operands, or (CX) a complex product's.
+template <typename T, bool CX, bool A_K, bool B_K, int BM, int BN, int BK,
+          int NTH>
+struct Loaders {
+  using A = typename std::conditional<
+      CX, ComplexLoader<T, BM, BK, A_K, NTH, true>,
+      TileLoader<T, BM, BK, A_K, NTH>>::type;
+  using B = typename std::conditional<
+      CX, ComplexLoader<T, BN, BK, B_K, NTH, false>,
+      TileLoader<T, BN, BK, B_K, NTH>>::type;
+  __device__ __forceinline__ static A a(int tid, const ComplexArgs &cx) {
+    if constexpr (CX)
+      return A(tid, cx.conj_a, (T)cx.ar, (T)cx.ai);
+    else
+      return A(tid);
+  }
+  __device__ __forceinline__ static B b(int tid, const ComplexArgs &cx) {
+    if constexpr (CX)
+      return B(tid, cx.conj_b, (T)cx.ar, (T)cx.ai);
+    else
+      return B(tid);
+  }
+};
+
 // Batch member and tile of a workgroup of a (tiles, 1, batch) grid. Workgroups
 // go to the 8 XCDs in turn, so in whole groups of 8 members each takes all its
 // tiles on one XCD, whose L2 then holds the member's A and B once.
@@ -552,6 +689,13 @@ struct GemmParams {
   int64_t aOff, bOff, cOff;
   double alpha, beta;
   int tiles_m, tiles_n;
+  // A complex product's real embedding: M, N, K, offsets and strides are the
+  // real form's, lda and ldb the complex operands'.
+  // (Plain fields, read in the kernel only where needed: as a nested struct
+  // they kept the compiler from seeing that the pointers are global ones, and
+  // flat loads cost 3-5% of a GEMM.)
+  double cx_ar, cx_ai;
+  int conj_a, conj_b;
 };
 
 // LDS bytes used by one macro tile (two buffers of A and B).
@@ -573,13 +717,13 @@ struct WaveTile {
 // Main loop of one BM x BN tile at (m0, n0): acc = A'(m0.., :) * B'(:, n0..)
 // over the whole K range. Shared by the plain / batched kernel, the grouped
 // kernel and the residue kernel, so all of them produce bit-identical sums
-// for the same K step.
+// for the same K step. CX: a complex product's operands (cx).
 template <Elem E, bool A_K, bool B_K, int BM, int BN, int BK, int WM, int WN,
-          int MI, bool NARROW = true>
+          int MI, bool NARROW, bool CX>
 __device__ __forceinline__ void gemm_mainloop(
     const typename ElemT<E>::T *__restrict__ A, int64_t lda,
     const typename ElemT<E>::T *__restrict__ B, int64_t ldb, int M, int N,
-    int K, int m0, int n0, int tid, char *lds,
+    int K, int m0, int n0, int tid, char *lds, ComplexArgs cx,
     typename WaveTile<E, BM, BN, WM, WN, MI>::AccV (
         &acc)[WaveTile<E, BM, BN, WM, WN, MI>::FM]
              [WaveTile<E, BM, BN, WM, WN, MI>::FN]) {
@@ -594,8 +738,9 @@ __device__ __forceinline__ void gemm_mainloop(
   constexpr int NTH = 64 * WM * WN;  // workgroup size
   constexpr int WTM = WT::WTM, WTN = WT::WTN, FM = WT::FM, FN = WT::FN;
 
-  using LA = TileLoader<T, BM, BK, A_K, NTH>;
-  using LB = TileLoader<T, BN, BK, B_K, NTH>;
+  using LP = Loaders<T, CX, A_K, B_K, BM, BN, BK, NTH>;
+  using LA = typename LP::A;
+  using LB = typename LP::B;
   constexpr int ROWB = LA::ROWB;
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB;
 
@@ -608,8 +753,8 @@ __device__ __forceinline__ void gemm_mainloop(
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = AccV{};
 
-  LA la(tid);
-  LB lb(tid);
+  LA la = LP::a(tid, cx);
+  LB lb = LP::b(tid, cx);
   const int nk = (K + BK - 1) / BK;
   // (NARROW = false: the caller knows that both operands are wide)
   const bool wide_a = !NARROW || LA::wide(M, K);
@@ -925,26 +1070,28 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
 // One BM x BN output tile at (m0, n0) of C = alpha*A'*B' + beta*C, the whole
 // K range; beta == 0 never reads C. LDS_BYTES: the LDS at `lds`.
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
-          int WM, int WN, int MI, int LDS_BYTES, bool NARROW = true>
+          int WM, int WN, int MI, int LDS_BYTES, bool NARROW = true,
+          bool CX = false>
 __device__ __forceinline__ void gemm_tile(
     const typename ElemT<E>::T *__restrict__ A, int64_t lda,
     const typename ElemT<E>::T *__restrict__ B, int64_t ldb, OutT *C,
     int64_t ldc, int M, int N, int K, double alpha_d, double beta_d, int m0,
-    int n0, int tid, char *lds) {
+    int n0, int tid, char *lds, ComplexArgs cx = {}) {
   using T = typename ElemT<E>::T;
   using WT = WaveTile<E, BM, BN, WM, WN, MI>;
-  using LA = TileLoader<T, BM, BK, A_K, 64 * WM * WN>;
-  using LB = TileLoader<T, BN, BK, B_K, 64 * WM * WN>;
+  using LP = Loaders<T, CX, A_K, B_K, BM, BN, BK, 64 * WM * WN>;
+  using LA = typename LP::A;
+  using LB = typename LP::B;
   typename WT::AccV acc[WT::FM][WT::FN];
-  gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, MI, NARROW>(
-      A, lda, B, ldb, M, N, K, m0, n0, tid, lds, acc);
+  gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, MI, NARROW, CX>(
+      A, lda, B, ldb, M, N, K, m0, n0, tid, lds, cx, acc);
   store_tile_lds<E, OutT, BM, BN, WM, WN, MI, LDS_BYTES>(
       acc, C, ldc, M, N, m0, n0, alpha_d, beta_d, tid, lds,
       LA::edge_row(M), LA::edge_shift(M), LB::edge_row(N), LB::edge_shift(N));
 }
 
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
-          int WM, int WN, int MI = 16>
+          int WM, int WN, int MI = 16, bool CX = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     GemmParams p) {
   using T = typename ElemT<E>::T;
@@ -969,9 +1116,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     C = static_cast<OutT *>(p.C) + p.cOff + (int64_t)z * p.strideC;
   int tile_m, tile_n;
   tile_coords(pid, p.tiles_m, p.tiles_n, tile_m, tile_n, gridDim.z < 8);
-  gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES>(
+  gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES, true, CX>(
       A, p.lda, B, p.ldb, C, p.ldc, p.M, p.N, p.K, p.alpha, p.beta,
-      tile_m * BM, tile_n * BN, threadIdx.x, lds);
+      tile_m * BM, tile_n * BN, threadIdx.x, lds,
+      CX ? ComplexArgs{p.cx_ar, p.cx_ai, p.conj_a, p.conj_b} : ComplexArgs{});
 }
 
 // Split-K partial tile: the K range [z ks, min(K, (z + 1) ks)) of one
@@ -980,7 +1128,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
 // CUs and a long K, splitting K gives every CU several workgroups to switch
 // between; splitk_reduce_kernel then adds the partials in split order.
 template <Elem E, bool A_K, bool B_K, int BM, int BN, int BK, int WM, int WN,
-          int MI>
+          int MI, bool CX = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_splitk_kernel(
     GemmParams p, int ks, typename ElemT<E>::Acc *W) {
   using T = typename ElemT<E>::T;
@@ -990,15 +1138,17 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_splitk_kernel(
   const int z = blockIdx.z;
   const int k0 = z * ks;
   const int kl = p.K - k0 < ks ? p.K - k0 : ks;
+  // (k0 is even: of a complex operand, k0 / 2 lines of 2 lda reals)
   const T *A = static_cast<const T *>(p.A) + p.aOff +
                (A_K ? (int64_t)k0 : (int64_t)k0 * p.lda);
   const T *B = static_cast<const T *>(p.B) + p.bOff +
                (B_K ? (int64_t)k0 : (int64_t)k0 * p.ldb);
   int tile_m, tile_n;
   tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-  gemm_tile<E, Acc, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES>(
+  gemm_tile<E, Acc, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES, true, CX>(
       A, p.lda, B, p.ldb, W + (int64_t)z * p.M * p.N, p.M, p.M, p.N, kl, 1.0,
-      0.0, tile_m * BM, tile_n * BN, threadIdx.x, lds);
+      0.0, tile_m * BM, tile_n * BN, threadIdx.x, lds,
+      CX ? ComplexArgs{p.cx_ar, p.cx_ai, p.conj_a, p.conj_b} : ComplexArgs{});
 }
 
 // C = alpha * sum_z W[z] + beta * C, the partials added in split order.

@@ -31,7 +31,7 @@ template <>
 struct TileCfg<Elem::BF16> : TileCfg<Elem::F16> {};
 
 template <Elem E, typename OutT, int BM, int BN, int BK, int WM, int WN,
-          int MI = 16>
+          int MI = 16, bool CX = false>
 hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
                             bool b_k, int64_t batch) {
   p.tiles_m = (int)cdiv(p.M, BM);
@@ -52,7 +52,7 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
     dim3 grid(tiles, 1, (unsigned)nb);
 #define HCB_GEMM_CASE(AK, BKC)                                   \
   if (a_k == AK && b_k == BKC)                                   \
-    gemm_mfma_kernel<E, OutT, AK, BKC, BM, BN, BK, WM, WN, MI>   \
+    gemm_mfma_kernel<E, OutT, AK, BKC, BM, BN, BK, WM, WN, MI, CX> \
         <<<grid, 64 * WM * WN, 0, stream>>>(q);
     HCB_GEMM_CASE(false, false)
     HCB_GEMM_CASE(false, true)
@@ -121,50 +121,51 @@ const MacroTile &pick_tile(int64_t M, int64_t N, int64_t batch, int num_cus,
   return *best;
 }
 
-template <Elem E, typename OutT>
+template <Elem E, typename OutT, bool CX>
 hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
                            bool a_k, bool b_k, int64_t batch) {
   using C = TileCfg<E>;
   const MacroTile &t =
-      pick_tile<E>(p.M, p.N, batch, num_cus, (a_k ? 0 : 1) + (b_k ? 0 : 1));
+      pick_tile<E>(p.M, p.N, batch, num_cus,
+                   CX ? 0 : (a_k ? 0 : 1) + (b_k ? 0 : 1));
   const int64_t tiles = cdiv(p.M, t.bm) * cdiv(p.N, t.bn) * batch;
   if constexpr (E == Elem::F64) {
     if (t.bm == 256)
-      return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 4, 2>(stream, p, a_k,
-                                                              b_k, batch);
+      return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 4, 2, 16, CX>(
+          stream, p, a_k, b_k, batch);
     if (t.bm == 128)
-      return launch_tiles<E, OutT, 128, 64, C::BK_BIG, 2, 4>(stream, p, a_k,
-                                                             b_k, batch);
+      return launch_tiles<E, OutT, 128, 64, C::BK_BIG, 2, 4, 16, CX>(
+          stream, p, a_k, b_k, batch);
   } else {
     if (t.bn == 256)
-      return launch_tiles<E, OutT, 256, 256, C::BK_BIG, 2, 4, 32>(
+      return launch_tiles<E, OutT, 256, 256, C::BK_BIG, 2, 4, 32, CX>(
           stream, p, a_k, b_k, batch);
     if constexpr (E == Elem::F32) {
       if (t.bm == 256)
-        return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 2, 4>(stream, p, a_k,
-                                                                b_k, batch);
+        return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 2, 4, 16, CX>(
+            stream, p, a_k, b_k, batch);
       if (t.bm == 128)
-        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 2>(stream, p, a_k,
-                                                                b_k, batch);
+        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 2, 16, CX>(
+            stream, p, a_k, b_k, batch);
     } else {
       // 8 waves of 64 x 32 (fragment read-ahead, two-vector transposed loads):
       // 2048^3 HGEMM NN 38.6 against 44.4 us with 4 waves of 64 x 64.
       if (t.bm == 128)
-        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 4, 32>(
+        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 4, 32, CX>(
             stream, p, a_k, b_k, batch);
     }
   }
   if (t.bm == 32) {
     if (p.K >= C::LONG_K && tiles <= num_cus)
-      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2>(
+      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2, 16, CX>(
           stream, p, a_k, b_k, batch);
     // (16-bit r-contiguous tiles of 128-deep steps are transposed in
     // registers: 8192 x 8192 x 1024 HGEMM NN 564 us against 743)
     if (sizeof(typename ElemT<E>::T) == 2 && !(a_k && b_k))
-      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2>(
+      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2, 16, CX>(
           stream, p, a_k, b_k, batch);
-    return launch_tiles<E, OutT, 32, 32, C::BK_32, 2, 2>(stream, p, a_k, b_k,
-                                                         batch);
+    return launch_tiles<E, OutT, 32, 32, C::BK_32, 2, 2, 16, CX>(
+        stream, p, a_k, b_k, batch);
   }
   // 64x64 tiles. At most one tile per CU leaves nothing else to cover a tile's
   // load latency: FP32 then runs 8 waves and long K steps (1024^3 NN 22.8 us
@@ -174,25 +175,25 @@ hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
   // waves and 92 with 64-deep steps).
   if constexpr (E == Elem::F32) {
     if (p.K >= 512 && tiles <= num_cus)
-      return launch_tiles<E, OutT, 64, 64, 128, 2, 4>(stream, p, a_k, b_k,
-                                                      batch);
+      return launch_tiles<E, OutT, 64, 64, 128, 2, 4, 16, CX>(
+          stream, p, a_k, b_k, batch);
     if (tiles <= num_cus)
-      return launch_tiles<E, OutT, 64, 64, 64, 2, 4>(stream, p, a_k, b_k,
-                                                     batch);
+      return launch_tiles<E, OutT, 64, 64, 64, 2, 4, 16, CX>(
+          stream, p, a_k, b_k, batch);
   }
   if constexpr (E == Elem::F64) {
     if (tiles <= num_cus)
-      return launch_tiles<E, OutT, 64, 64, 32, 2, 4>(stream, p, a_k, b_k,
-                                                     batch);
-    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 4>(stream, p, a_k, b_k,
-                                                         batch);
+      return launch_tiles<E, OutT, 64, 64, 32, 2, 4, 16, CX>(
+          stream, p, a_k, b_k, batch);
+    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 4, 16, CX>(
+        stream, p, a_k, b_k, batch);
   } else {
-    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 2>(stream, p, a_k, b_k,
-                                                         batch);
+    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 2, 16, CX>(
+        stream, p, a_k, b_k, batch);
   }
 }
 
-template <Elem E, int T, int BK, int WM, int WN>
+template <Elem E, int T, int BK, int WM, int WN, bool CX>
 void launch_splitk_tiles(hipStream_t stream, GemmParams p, bool a_k, bool b_k,
                          const SplitK &sk, typename ElemT<E>::Acc *W) {
   p.tiles_m = (int)cdiv(p.M, T);
@@ -200,7 +201,7 @@ void launch_splitk_tiles(hipStream_t stream, GemmParams p, bool a_k, bool b_k,
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)sk.splits);
 #define HCB_SPLITK_CASE(AK, BKC)                          \
   if (a_k == AK && b_k == BKC)                            \
-    gemm_splitk_kernel<E, AK, BKC, T, T, BK, WM, WN, 16>  \
+    gemm_splitk_kernel<E, AK, BKC, T, T, BK, WM, WN, 16, CX> \
         <<<grid, 64 * WM * WN, 0, stream>>>(p, sk.ks, W);
   HCB_SPLITK_CASE(false, false)
   HCB_SPLITK_CASE(false, true)
@@ -209,7 +210,7 @@ void launch_splitk_tiles(hipStream_t stream, GemmParams p, bool a_k, bool b_k,
 #undef HCB_SPLITK_CASE
 }
 
-template <Elem E, typename OutT>
+template <Elem E, typename OutT, bool CX>
 hcblasStatus_t launch_gemm_splitk(hipStream_t stream, int num_cus,
                                   GemmParams p, bool a_k, bool b_k,
                                   const SplitK &sk,
@@ -218,11 +219,11 @@ hcblasStatus_t launch_gemm_splitk(hipStream_t stream, int num_cus,
   // (64x64 FP64 256 x 128 x 16384 96 us with 8 waves of 32 x 16 against 123 with
   // 4 of 32 x 32)
   if (sk.tile == 32)
-    launch_splitk_tiles<E, 32, TileCfg<E>::BK_32_LONG, 2, 2>(stream, p, a_k,
+    launch_splitk_tiles<E, 32, TileCfg<E>::BK_32_LONG, 2, 2, CX>(stream, p, a_k,
                                                              b_k, sk, W);
   else
     launch_splitk_tiles<E, 64, TileCfg<E>::BK_64, 2,
-                        sizeof(typename ElemT<E>::T) == 2 ? 2 : 4>(
+                        sizeof(typename ElemT<E>::T) == 2 ? 2 : 4, CX>(
         stream, p, a_k, b_k, sk, W);
   hcblasStatus_t st = launch_status();
   if (st != HCBLAS_STATUS_SUCCESS) return st;

@@ -91,3 +91,52 @@ def test_large_tiles_at_odd_sizes(hc, handle, p, M, N, K, ta, tb):
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_few_tiles(hc, handle, p, M, N, K, ta, tb):
     _check(hc, handle, p, COL, ta, tb, M, N, K, 1, M + N + K)
+
+
+# Complex products (embedded by the tile loaders): operands of one element and
+# one vector, odd sizes on both sides of a vector and a tile edge, K tails of
+# every step length, split-K (twice K reaches 2048), 64x64 to the largest tiles.
+COMPLEX = [(1, 1, 1), (1, 5, 3), (3, 1, 2), (7, 2, 1), (33, 31, 17),
+           (65, 63, 33), (127, 130, 5), (70, 41, 1100), (520, 1100, 40),
+           (2050, 2049, 9)]
+
+
+@pytest.mark.parametrize("p", ["c", "z"])
+@pytest.mark.parametrize("tb", [0, 1, 2])
+@pytest.mark.parametrize("ta", [0, 1, 2])
+def test_complex_edges(hc, handle, p, ta, tb):
+    """Each part of an output is a sum of 2K real products of alpha * a (three
+    roundings) and b in some order: within (2K + 6) eps of |alpha||A||B|."""
+    dt, rt = (np.complex64, np.float32) if p == "c" else (np.complex128,
+                                                          np.float64)
+    eps = np.finfo(rt).eps
+    for M, N, K in COMPLEX:
+        rng = np.random.default_rng(M + N + K)
+
+        def rand(r, c):
+            v = rng.uniform(-1, 1, (r, c)) + 1j * rng.uniform(-1, 1, (r, c))
+            return v.astype(dt)
+
+        A = rand(K, M) if ta == 0 else rand(M, K)  # column-major storage
+        B = rand(N, K) if tb == 0 else rand(K, N)
+        C = rand(N, M + 1)
+        alpha, beta = 1.25 - 0.5j, 0.75 + 0j
+        dC = to_dev(C)
+        st = getattr(hc.api, f"hcblas_{p}gemm")(
+            handle, 1, ta, tb, M, N, K, alpha,
+            to_dev(np.concatenate([np.zeros(1, dt), A.ravel()])), 1,
+            A.shape[1], to_dev(np.concatenate([np.zeros(3, dt), B.ravel()])),
+            3, B.shape[1], beta, dC, 0, M + 1)
+        assert st == 0
+        got = to_host(dC)
+
+        def op(X, t):  # storage rows are the matrix's columns
+            X = X.astype(np.complex128)
+            return X.T if t == 0 else X if t == 1 else X.conj()
+
+        a, b = op(A, ta), op(B, tb)
+        ref = alpha * (a @ b) + beta * C.T[:M].astype(np.complex128)
+        mag = abs(alpha) * (abs(a) @ abs(b)) + abs(beta * C.T[:M])
+        assert np.array_equal(got.T[M], C.T[M])
+        assert np.all(abs(got.T[:M] - ref) <= 2 * (2 * K + 6) * eps * mag), \
+            (M, N, K)
