@@ -12,28 +12,27 @@
 // those of an FP32 GEMM of the exact products, at three BF16 MFMAs per 16 k
 // instead of eight FP32 MFMAs (v_mfma_f32_32x32x2f32 takes 2 k).
 //
-// Tile: 256 x 256 x 32 over 8 waves of 64 x 128, or 128 x 128 x 32 over 4 waves
-// of 64 x 64, LDS double-buffered like the plain kernel (the FP32 operand's
-// tile is three planes), epilogue through LDS with the plain kernels'
-// arithmetic; the result is rounded once to BF16.
+// Tile: 256 x 256 x 32 over 8 waves of 64 x 128, 128 x 128 x 32 over 4 waves of
+// 64 x 64 or 64 x 64 x 32 over 2 waves of 32 x 64, LDS double-buffered like the
+// plain kernel (the FP32 operand's tile is three planes), epilogue through LDS
+// with the plain kernels' arithmetic; the result is rounded once to BF16.
 //
 // What bounds it: the MFMAs, and beside them the split's VALU work on the same
-// SIMDs. v_cvt_pk_bf16_f32 rounds two values at once, about 8 operations per
-// element where integer rounding took 18. An operand stored with the inner
-// index as its row index (both operands of dB = op(A)^T dC) is transposed in
-// registers by the tile loader: a thread holds a 4 x 4 block of FP32 or two
-// k-lines of 8 BF16 rows and writes along k, as many LDS writes as the
-// k-contiguous form. (Transposed copies of dC and A in a workspace took 115 us
-// of the 256 x 256x1024x512 backward's 700.)
+// SIMDs and the LDS. (256 x 256x1024x512: with the planes' writes two to a bank,
+// 43-58% of the LDS cycles were conflicts, and with integer rounding in the
+// epilogue, 8 operations per output, the MFMAs were busy 52% of dA and 33% of
+// dB; dA 223 -> 204 us, dB 293 -> 246 without either.) v_cvt_pk_bf16_f32 rounds
+// two values at once, about 8 operations per element where integer rounding
+// took 18. An operand stored with the inner index as its row index (both
+// operands of dB = op(A)^T dC) is transposed in registers by the tile loader: a
+// thread holds a 4 x 4 block of FP32 or two k-lines of 8 BF16 rows and writes
+// along k, as many LDS writes as the k-contiguous form. (Transposed copies of dC
+// and A in a workspace took 115 us of the 256 x 256x1024x512 backward's 700.)
 #include "gemm_common.hpp"
 
 namespace hcb {
 namespace {
 
-__device__ __forceinline__ uint16_t bf16_rne(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
 __device__ __forceinline__ float bf16_val(uint16_t b) {
   return __uint_as_float((uint32_t)b << 16);
 }
@@ -65,7 +64,18 @@ __device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t &h,
 template <int ROWS, int BK, bool KCONT, int NTH>
 struct SplitPlaneLoader : TileLoader<float, ROWS, BK, KCONT, NTH> {
   using L = TileLoader<float, ROWS, BK, KCONT, NTH>;
-  using L::L;
+  // The loader's vectors in an order in which the 8-byte LDS writes of 16 and of
+  // 32 consecutive lanes fall on distinct banks (rows are 80 bytes apart):
+  // k-contiguous, 32 lanes take rows 0, 4, 8, 12 (64 bytes each at offsets 0,
+  // 64, 128, 192 of 256) instead of 0 .. 3; 4 x 4 blocks, 4 r-vectors (64 bytes
+  // apart) by all 8 k-quads instead of twice 4.
+  __device__ __forceinline__ static int order(int t) {
+    static_assert(BK == 32, "eight vectors along k");
+    if (KCONT) return (t & ~0x78) | ((t >> 2) & 0x18) | ((t << 2) & 0x60);
+    return ((t >> 3) & 3) | ((t & 3) << 2) | ((t >> 5) << 4) |
+           (((t >> 2) & 1) * ROWS);  // 16 threads per group, ROWS / 16 groups
+  }
+  __device__ __forceinline__ explicit SplitPlaneLoader(int t) : L(order(t)) {}
   static_assert(KCONT || L::TRANS4, "4 x 4 blocks");
   static_assert(L::NV % NTH == 0, "whole vectors per thread");
   static constexpr int ROWB = BK * 2 + 16;
@@ -110,10 +120,7 @@ struct Bf16Out {
 }  // namespace
 template <>
 __device__ __forceinline__ Bf16Out to_out<Bf16Out, float>(float v) {
-  const uint32_t u = __float_as_uint(v);
-  if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x7FFFFFu))
-    return Bf16Out{(uint16_t)((u >> 16) | 0x40u)};
-  return Bf16Out{bf16_rne(v)};
+  return Bf16Out{(uint16_t)cvt_pk_bf16(v, v)};
 }
 template <>
 __device__ __forceinline__ float from_out<float, Bf16Out>(Bf16Out v) {
@@ -247,10 +254,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
       LB::edge_shift(p.N));
 }
 
-// Tiles: 256 x 256 over 8 waves of 64 x 128 (FP32 operand along the wave
-// tile's short side: 10 fragment reads per 24 MFMAs of a 16-k chunk, against
-// 8 per 12 for 64 x 64 wave tiles) when both output sides reach 256, else
-// 128 x 128 over 4 waves of 64 x 64.
 template <bool AF, int BM, int BN, int WM, int WN>
 hcblasStatus_t launch_mixed_cfg(hipStream_t s, MixedParams p, bool a_k,
                                 bool b_k, int64_t batch) {
@@ -280,16 +283,38 @@ hcblasStatus_t launch_mixed_cfg(hipStream_t s, MixedParams p, bool a_k,
   }
   return HCBLAS_STATUS_SUCCESS;
 }
+// Tiles: 256 x 256 over 8 waves of 64 x 128 (FP32 operand along the wave
+// tile's short side: 10 fragment reads per 24 MFMAs of a 16-k chunk, against
+// 8 per 12 for 64 x 64 wave tiles), 128 x 128 over 4 waves of 64 x 64, 64 x 64
+// over 2 waves of 32 x 64. Taken by the time on the CU with the most tiles,
+// ceil(tiles / CUs) * area / rate (rates relative, from the times below; with
+// 256 x 256 wherever both sides reach it a few large tiles ran on a few CUs):
+//   dB of                          256   128   64 (us, tile edge)
+//   256x 256 x 1024 x 512          245   313   464
+//   100x 300 x 300 x 300            64    42    44
+//   1x 1024 x 1024 x 1024           67    41    30
+//   7x 900 x 900 x 900              66    51    71
+//   16x 1000 x 700 x 900            76    89   110
+//   33x 200 x 130 x 600             24    16    13
 template <bool AF>
-hcblasStatus_t launch_mixed(hipStream_t s, MixedParams p, bool a_k, bool b_k,
-                            int64_t batch) {
-  if (p.M >= 256 && p.N >= 256) {
+hcblasStatus_t launch_mixed(hipStream_t s, int num_cus, MixedParams p,
+                            bool a_k, bool b_k, int64_t batch) {
+  auto time = [&](int64_t t, int rate) {
+    return cdiv(cdiv(p.M, t) * cdiv(p.N, t) * batch, num_cus) * t * t / rate;
+  };
+  const int64_t t256 = time(256, 125), t128 = time(128, 90), t64 = time(64, 48);
+  if (t256 <= t128 && t256 <= t64) {
     if constexpr (AF)
       return launch_mixed_cfg<AF, 256, 256, 4, 2>(s, p, a_k, b_k, batch);
     else
       return launch_mixed_cfg<AF, 256, 256, 2, 4>(s, p, a_k, b_k, batch);
   }
-  return launch_mixed_cfg<AF, 128, 128, 2, 2>(s, p, a_k, b_k, batch);
+  if (t128 <= t64)
+    return launch_mixed_cfg<AF, 128, 128, 2, 2>(s, p, a_k, b_k, batch);
+  if constexpr (AF)
+    return launch_mixed_cfg<AF, 64, 64, 2, 1>(s, p, a_k, b_k, batch);
+  else
+    return launch_mixed_cfg<AF, 64, 64, 1, 2>(s, p, a_k, b_k, batch);
 }
 
 }  // namespace
@@ -314,8 +339,10 @@ hcblasStatus_t gemm_mixed_bf16(hcblasHandle_t h, const Canon &c, bool a_f32,
   p.ldc = ldc;
   p.strideC = strideC;
   p.alpha = alpha;
-  return a_f32 ? launch_mixed<true>(h->stream, p, c.a_k, c.b_k, batch)
-               : launch_mixed<false>(h->stream, p, c.a_k, c.b_k, batch);
+  return a_f32 ? launch_mixed<true>(h->stream, h->num_cus, p, c.a_k, c.b_k,
+                                    batch)
+               : launch_mixed<false>(h->stream, h->num_cus, p, c.a_k, c.b_k,
+                                     batch);
 }
 
 }  // namespace hcb

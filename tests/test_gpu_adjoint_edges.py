@@ -55,6 +55,17 @@ def test_every_orientation(torch_cuda, ta, tb, batch, M, N, K):
         assert bool(((d - r).abs() <= bound + UB * r.abs()).all())
 
 
+# Batches that fill the GPU: dA and dB on 128 and 128, 256 and 128, 128 and 256
+# tiles (those above run on 64 x 64 ones).
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("batch,M,N,K", [(60, 130, 259, 200),
+                                         (64, 509, 515, 261),
+                                         (128, 261, 250, 257)])
+def test_every_tile(torch_cuda, ta, tb, batch, M, N, K):
+    test_every_orientation(torch_cuda, ta, tb, batch, M, N, K)
+
+
 def test_special_cotangents(torch_cuda):
     M, N, K = 40, 48, 24
     g = torch.Generator(device="cuda").manual_seed(1)
