@@ -105,11 +105,14 @@ __device__ __forceinline__ void run_tile(const ProbDev &p, int m0, int n0,
 // OCC: workgroups per CU the launch is sized for (the register budget
 // follows from it: 4 waves per workgroup, one per SIMD).
 constexpr int kXcd = 8;
+constexpr int kHead = (kXcd + 2) / 2;  // entries that hold the part offsets
 
 template <int TM, bool NARROW, int OCC>
 __global__ __launch_bounds__(256, OCC) void grouped_gemm_kernel(
-    const ProbDev *__restrict__ probs, const int2 *__restrict__ work,
-    const int *__restrict__ parts, unsigned int *counters, int dynamic) {
+    const ProbDev *__restrict__ probs, const int2 *__restrict__ table,
+    unsigned int *counters, int dynamic) {
+  const int *__restrict__ parts = reinterpret_cast<const int *>(table);
+  const int2 *__restrict__ work = table + kHead;
   __shared__ __attribute__((aligned(16))) char lds[GroupCfg<TM>::LDS];
   __shared__ int next;
   int part = blockIdx.x % kXcd, left = kXcd;
@@ -175,13 +178,13 @@ struct hcblasGroupedPlan {
   bool narrow = false;  // an operand is shorter than one 16-byte vector
   std::vector<ProbDev> probs;  // host copy (canonical)
   ProbDev *d_probs = nullptr;
-  int2 *d_work = nullptr;
+  int2 *d_work = nullptr;  // kHead: the kXcd + 1 part offsets; the work list
   size_t work_cap = 0;
-  int *d_parts = nullptr;              // kXcd + 1 offsets into d_work
   unsigned int *d_counters = nullptr;  // kXcd queues, finished workgroups
   int total = 0;
   int grid = 0;
   int shape = 0;   // index into kTileShapes
+  int probs_shape = -1;  // the one d_probs' tile counts are for
   int order = 0;   // 0: longest first, 1: table order
   int occ = 0;     // index into kOccupancies
   int sched = 0;   // 0: atomic queue, 1: static stride
@@ -204,15 +207,15 @@ void launch_occ(hcblasGroupedPlan *p, hipStream_t s) {
   switch (kOccupancies[p->occ]) {
     case 2:
       grouped_gemm_kernel<TM, NARROW, 2><<<g, 256, 0, s>>>(
-          p->d_probs, p->d_work, p->d_parts, p->d_counters, p->sched == 0);
+          p->d_probs, p->d_work, p->d_counters, p->sched == 0);
       break;
     case 3:
       grouped_gemm_kernel<TM, NARROW, 3><<<g, 256, 0, s>>>(
-          p->d_probs, p->d_work, p->d_parts, p->d_counters, p->sched == 0);
+          p->d_probs, p->d_work, p->d_counters, p->sched == 0);
       break;
     default:
       grouped_gemm_kernel<TM, NARROW, 4><<<g, 256, 0, s>>>(
-          p->d_probs, p->d_work, p->d_parts, p->d_counters, p->sched == 0);
+          p->d_probs, p->d_work, p->d_counters, p->sched == 0);
       break;
   }
 }
@@ -242,39 +245,53 @@ hcblasStatus_t build(hcblasHandle_t h, hcblasGroupedPlan *p, int shape,
   if (order == 0)
     std::stable_sort(idx.begin(), idx.end(),
                      [&](int a, int b) { return cost[a] > cost[b]; });
+  auto tiles = [&](int i) {
+    const ProbDev &q = p->probs[i];
+    return (int64_t)((q.M + tm - 1) / tm) * q.tiles_n;
+  };
+  int64_t total = 0;
+  for (int i : idx) total += tiles(i);
+  // Up to two 64x64 tiles per CU (or as much work in 32x32 ones), whole problems
+  // would leave one XCD with a second round while others have free CUs: the tiles
+  // go to the XCDs in turn (64 problems of 32 .. 256, 223 tiles: 17.9 us against
+  // 19.1; 369 tiles 21.5 against 23.1; with more, 585 tiles 34.5 against 31.4).
+  const bool whole = total * tm * tm > 2 * (int64_t)h->num_cus * 64 * 64;
   std::vector<int2> list[kXcd];
   int64_t load[kXcd] = {};
+  int turn = 0;
   for (int i : idx) {
-    const ProbDev &q = p->probs[i];
-    const int nt = (q.M + tm - 1) / tm * q.tiles_n;
+    const int64_t nt = tiles(i);
     const int x = (int)(std::min_element(load, load + kXcd) - load);
-    for (int t = 0; t < nt; ++t) list[x].push_back(make_int2(i, t));
+    for (int t = 0; t < nt; ++t)
+      list[whole ? x : turn++ % kXcd].push_back(make_int2(i, t));
     load[x] += cost[i] * nt;
   }
-  std::vector<int2> work;
-  int parts[kXcd + 1] = {};
+  // One upload for a candidate of the same tile shape.
+  std::vector<int2> work(kHead);
+  int parts[2 * kHead] = {};
   for (int x = 0; x < kXcd; ++x) {
     work.insert(work.end(), list[x].begin(), list[x].end());
-    parts[x + 1] = (int)work.size();
+    parts[x + 1] = (int)work.size() - kHead;
   }
-  p->total = (int)work.size();
+  std::memcpy(work.data(), parts, sizeof(parts));
+  p->total = parts[kXcd];
   if (work.size() > p->work_cap) {
     if (p->d_work) (void)hipFree(p->d_work);
     p->d_work = nullptr;
-    if (hipMalloc(&p->d_work, sizeof(int2) * std::max<size_t>(1, work.size())) !=
-        hipSuccess)
+    p->work_cap = 0;
+    if (hipMalloc(&p->d_work, sizeof(int2) * work.size()) != hipSuccess)
       return HCBLAS_STATUS_ALLOC_FAILED;
     p->work_cap = work.size();
   }
-  if (!work.empty() &&
-      hipMemcpy(p->d_work, work.data(), sizeof(int2) * work.size(),
+  if (hipMemcpy(p->d_work, work.data(), sizeof(int2) * work.size(),
                 hipMemcpyHostToDevice) != hipSuccess)
     return HCBLAS_STATUS_EXECUTION_FAILED;
-  if (hipMemcpy(p->d_probs, p->probs.data(), sizeof(ProbDev) * p->count,
-                hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(p->d_parts, parts, sizeof(parts), hipMemcpyHostToDevice) !=
-          hipSuccess)
-    return HCBLAS_STATUS_EXECUTION_FAILED;
+  if (p->probs_shape != shape) {
+    if (hipMemcpy(p->d_probs, p->probs.data(), sizeof(ProbDev) * p->count,
+                  hipMemcpyHostToDevice) != hipSuccess)
+      return HCBLAS_STATUS_EXECUTION_FAILED;
+    p->probs_shape = shape;
+  }
   p->shape = shape;
   p->order = order;
   p->occ = occ;
@@ -373,7 +390,6 @@ hcblasStatus_t hcblasGroupedPlanCreate(hcblasHandle_t handle,
   }
   if (hipMalloc(&p->d_probs, sizeof(ProbDev) * std::max(1, count)) !=
           hipSuccess ||
-      hipMalloc(&p->d_parts, (kXcd + 1) * sizeof(int)) != hipSuccess ||
       hipMalloc(&p->d_counters, (kXcd + 1) * sizeof(unsigned int)) !=
           hipSuccess ||
       hipMemset(p->d_counters, 0, (kXcd + 1) * sizeof(unsigned int)) !=
@@ -463,7 +479,6 @@ hcblasStatus_t hcblasGroupedPlanDestroy(hcblasGroupedPlan_t plan) {
   free_graph(plan);
   if (plan->d_probs) (void)hipFree(plan->d_probs);
   if (plan->d_work) (void)hipFree(plan->d_work);
-  if (plan->d_parts) (void)hipFree(plan->d_parts);
   if (plan->d_counters) (void)hipFree(plan->d_counters);
   delete plan;
   return HCBLAS_STATUS_SUCCESS;
