@@ -82,9 +82,10 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
 // 128 k together; of the others two or more share a CU. (BF16 12x 807x775x189
 // 30 us on 256x256 tiles, 21 on 128x128; HGEMM 64x 446x732x224 36 and 31; but 64x
 // 512^3 30 and 35, 120x 913x750x666 236 and 303.) An FP32 / FP64 32x32 tile pays
-// twice as much for its area as the larger ones (SGEMM 120x 203x698x84 79 us on
-// 32x32, 54 on 64x64, 120x 277x347x69 57 and 41; DGEMM 827x5055x167 45 and 38; but
-// SGEMM 8x 255x257x517 16.3 and 17.1).
+// three times as much for its area as the larger ones (SGEMM 120x 203x698x84 79 us
+// on 32x32, 54 on 64x64, 120x 277x347x69 57 and 41; DGEMM 827x5055x167 45 and 38;
+// CGEMM 120x 130x130x40 28 and 24, ZGEMM 10x 500x400x100 46.6 and 44.9; but SGEMM
+// 8x 255x257x517 16.3 and 17.1, CGEMM 64x 96^3 11.2 and 13.1).
 struct MacroTile {
   int bm, bn;
   int rate[3];
@@ -101,13 +102,13 @@ inline constexpr MacroTile kTiles<Elem::F32>[] = {
     {256, 128, {128, 128, 129}, 20},
     {128, 128, {133, 129, 127}, 20},
     {64, 64, {120, 117, 114}, 20},
-    {32, 32, {105, 97, 80}, 40}};
+    {32, 32, {105, 97, 80}, 60}};
 template <>
 inline constexpr MacroTile kTiles<Elem::F64>[] = {
     {256, 128, {68, 68, 68}, 10},
     {128, 64, {68, 68, 67}, 10},
     {64, 64, {66, 65, 65}, 10},
-    {32, 32, {57, 54, 52}, 20}};
+    {32, 32, {57, 54, 52}, 35}};
 
 // The tile with the least time on the CU that gets the most tiles,
 // ceil(tiles / CUs) * area * (K + lead) / rate: tiles past the edge of C and a
