@@ -13,6 +13,7 @@
 #include <cstdint>
 
 #include "../../include/hcblas.h"
+#include "partial_blocks.hpp"
 
 namespace hcb {
 
@@ -38,6 +39,11 @@ constexpr int kMaxDevices = 64;
 // per device); nullptr if the lookup failed.
 void *scratch_address(int dev);
 
+// Device memory for PartialBlocks. Allocated and freed also while this thread
+// or another captures a graph.
+void *alloc_partials(size_t bytes);
+void free_partials(void *p);
+
 }  // namespace hcb
 
 struct hcblasContext {
@@ -61,20 +67,15 @@ struct hcblasContext {
   double *h_result_dev = nullptr;
   uint64_t result_seq = 0;
 
-  // gemv split-reduction partials and per-row-block tickets (grow-only; the
-  // ticket region is zeroed when it is (re)allocated and every launch leaves
-  // it zero again).
-  hcb::Workspace gemv_partials;
-  hcb::Workspace gemv_tickets;
+  // Partial sums of split reductions (see partials()).
+  hcb::PartialBlocks partials{hcb::alloc_partials, hcb::free_partials};
 
-  // Real embedding of complex GEMM operands.
+  // Real embedding of complex GEMM operands (split precision modes).
   hcb::Workspace gemm_ws;
   // BF16 planes / INT8 slices and exponents of the split GEMM paths (kept
   // apart from gemm_ws: a split complex GEMM reads the embedding while it
   // writes the planes).
   hcb::Workspace split_ws;
-  // Split-K partial tiles of the plain GEMM.
-  hcb::Workspace kpart_ws;
   // This device's address of the fixed scratch of hcblas_gemv_noalloc.
   void *noalloc_scratch = nullptr;
 };
@@ -90,8 +91,10 @@ inline bool handle_ok(hcblasHandle_t h) {
 // on the old block is complete before it is released.
 hipError_t ensure_workspace(Workspace &ws, size_t bytes);
 
-// Makes the gemv ticket region at least `count` counters and zero.
-hipError_t ensure_tickets(hcblasHandle_t h, size_t count);
+// `bytes` of device memory for the partial sums of a call on the handle's
+// stream, free for the call's launches on that stream; nullptr if there is none,
+// and the call then runs unsplit.
+void *partials(hcblasHandle_t h, size_t bytes);
 
 inline hcblasStatus_t launch_status() {
   hipError_t e = hipGetLastError();

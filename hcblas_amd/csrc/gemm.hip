@@ -322,11 +322,9 @@ hcblasStatus_t run_gemm(hcblasHandle_t h, const Canon &c, double alpha,
                     E == Elem::F64 ? 16 : E == Elem::F32 ? 32 : 64);
     if (sk.splits > 1) {
       const size_t bytes = sizeof(Acc) * (size_t)sk.splits * c.M * c.N;
-      if (ensure_workspace(h->kpart_ws, bytes) != hipSuccess)
-        return HCBLAS_STATUS_ALLOC_FAILED;
-      return launch_gemm_splitk<E, OutT, CX>(
-          h->stream, h->num_cus, p, c.a_k, c.b_k, sk,
-          static_cast<Acc *>(h->kpart_ws.ptr));
+      if (Acc *W = static_cast<Acc *>(partials(h, bytes)))
+        return launch_gemm_splitk<E, OutT, CX>(h->stream, h->num_cus, p, c.a_k,
+                                               c.b_k, sk, W);
     }
   }
   return launch_gemm<E, OutT, CX>(h->stream, h->num_cus, p, c.a_k, c.b_k,

@@ -37,8 +37,11 @@ inline int64_t plan_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // lacks on a small or narrow matrix is loads in flight, not their width) but
 // not at a few workgroups more than the GPU holds side by side: 258 bands of
 // a 12000^2 SGEMV-N took 120 us, 255 took 91.
+// split = false: the same without split reductions (there is no memory for the
+// partials).
 inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
-                          bool vec, int vn, size_t esize, int64_t batch) {
+                          bool vec, int vn, size_t esize, int64_t batch,
+                          bool split = true) {
   const int64_t len_y = panel ? R : Cc;
   const int64_t target = (int64_t)num_cus * 4;  // workgroups to aim for
   GemvPlan p{GemvKernel::kColumn, 0, 4, 1, 1, 0};
@@ -59,12 +62,12 @@ inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
   // where the column blocks are few: up to one workgroup per CU, bands of at
   // least 2 steps.
   int64_t bands = plan_cdiv(steps, 16);
-  if (!panel && band) {
+  if (!panel && band && split) {
     const int64_t blocks = plan_cdiv(Cc, kBandCols) * batch;
     bands = std::max(bands,
                      std::min((int64_t)num_cus / blocks, (steps + 1) / 2));
   }
-  if (!panel && band && bands <= 65535) {
+  if (!panel && band && bands <= (split ? 65535 : 1)) {
     int64_t xr = plan_cdiv(steps, bands);
     if (xr > 4) xr = (xr + 1) / 2 * 2;  // instances: 1..4, 6, 8, .. 16
     p.kernel = xr == 16 ? GemvKernel::kBand16 : GemvKernel::kBand8;
@@ -112,6 +115,7 @@ inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
         std::max<int64_t>(1, plan_cdiv(target, p.oblocks * batch)),
         std::min<int64_t>(256, max_split));
   }
+  if (!split) p.splits = 1;
   if (p.splits > 1)
     p.partial_bytes = esize * (size_t)p.splits * (size_t)len_y *
                       (size_t)std::min<int64_t>(batch, 65535);

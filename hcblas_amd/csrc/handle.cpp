@@ -57,15 +57,42 @@ hipError_t ensure_workspace(Workspace &ws, size_t bytes) {
   return hipSuccess;
 }
 
-hipError_t ensure_tickets(hcblasHandle_t h, size_t count) {
-  size_t bytes = count * sizeof(unsigned int);
-  if (h->gemv_tickets.bytes >= bytes) return hipSuccess;
-  hipError_t e = ensure_workspace(h->gemv_tickets, bytes);
-  if (e != hipSuccess) return e;
-  // Zeroed once at allocation; every kernel that takes a ticket leaves it 0.
-  e = hipMemset(h->gemv_tickets.ptr, 0, h->gemv_tickets.bytes);
-  if (e != hipSuccess) return e;
-  return hipDeviceSynchronize();
+namespace {
+// Lets this thread allocate and free memory during captures.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+}  // namespace
+
+void *alloc_partials(size_t bytes) {
+  const RelaxedCapture relaxed;
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+void free_partials(void *p) {
+  const RelaxedCapture relaxed;
+  (void)hipFree(p);
+}
+
+void *partials(hcblasHandle_t h, size_t bytes) {
+  // hipStreamPerThread stands for another stream in each thread.
+  static thread_local const char this_thread = 0;
+  const void *queue = h->stream == hipStreamPerThread
+                          ? static_cast<const void *>(&this_thread)
+                          : static_cast<const void *>(h->stream);
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  // (the default stream cannot be captured)
+  if (h->stream != nullptr &&
+      hipStreamGetCaptureInfo(h->stream, &status, &id) != hipSuccess)
+    (void)hipGetLastError();
+  return h->partials.get(queue, status == hipStreamCaptureStatusActive, id,
+                         bytes);
 }
 
 }  // namespace hcb
@@ -124,11 +151,8 @@ hcblasStatus_t hcblasDestroy(hcblasHandle_t *handle) {
   h->magic = 0;
   (void)hipFree(h->d_partials);
   (void)hipHostFree(h->h_result);
-  if (h->gemv_partials.ptr) (void)hipFree(h->gemv_partials.ptr);
-  if (h->gemv_tickets.ptr) (void)hipFree(h->gemv_tickets.ptr);
   if (h->gemm_ws.ptr) (void)hipFree(h->gemm_ws.ptr);
   if (h->split_ws.ptr) (void)hipFree(h->split_ws.ptr);
-  if (h->kpart_ws.ptr) (void)hipFree(h->kpart_ws.ptr);
   delete h;
   *handle = nullptr;
   return HCBLAS_STATUS_SUCCESS;

@@ -14,7 +14,7 @@
 // column of its row band as one contiguous run; x or the band's sums stay in
 // registers). All stream S once with 16-byte loads and split the reduction
 // across workgroups when the output alone cannot fill 256 CUs; split partials
-// go to a per-handle workspace and a small finish kernel on the same stream
+// go to a block of the handle's and a small finish kernel on the same stream
 // sums them in a fixed order, so results are deterministic.
 //
 // GER updates S[r,c] = fma(v[r], alpha*w[c], S[r,c]) where w is the vector
@@ -22,6 +22,7 @@
 // v = y, w = x for row-major this is bit-identical to CBLAS (netlib
 // "temp = alpha*y(j); a(i,j) += x(i)*temp", row-major by argument swap).
 #include <type_traits>
+#include <utility>
 
 #include "common.hpp"
 #include "gemv_plan.hpp"
@@ -837,8 +838,6 @@ hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
     plan = plan_gemv(h->num_cus, panel, R, Cc, vec, VN, sizeof(T), batch);
   }
   s.splits = plan.splits;
-  const int64_t oblocks = plan.oblocks;
-  const bool bandn = plan.kernel == GemvKernel::kBandN;
   T *part = nullptr;
   if (s.splits > 1) {
     if (fixed_part) {
@@ -847,15 +846,18 @@ hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
       if (plan.partial_bytes > fixed_bytes) return HCBLAS_STATUS_INVALID_VALUE;
       part = static_cast<T *>(fixed_part);
     } else {
-      if (ensure_workspace(h->gemv_partials, plan.partial_bytes) != hipSuccess)
-        return HCBLAS_STATUS_ALLOC_FAILED;
-      part = static_cast<T *>(h->gemv_partials.ptr);
+      part = static_cast<T *>(partials(h, plan.partial_bytes));
+      if (part == nullptr) {
+        plan = plan_gemv(h->num_cus, panel, R, Cc, vec, VN, sizeof(T), batch,
+                         false);
+        s.splits = 1;
+      }
     }
   }
   for (int64_t b0 = 0; b0 < batch; b0 += 65535) {
     int64_t nb = std::min<int64_t>(65535, batch - b0);
-    dim3 grid((unsigned)oblocks, (unsigned)s.splits, (unsigned)nb);
-    if (bandn) grid = dim3((unsigned)s.splits, (unsigned)oblocks, (unsigned)nb);
+    dim3 grid((unsigned)plan.oblocks, (unsigned)s.splits, (unsigned)nb);
+    if (plan.kernel == GemvKernel::kBandN) std::swap(grid.x, grid.y);
     const T *Ab = A + b0 * sA;
     const T *xb = x + b0 * sx;
     T *yb = y + b0 * sy;
@@ -1033,21 +1035,6 @@ hcblasStatus_t ger_entry(hcblasHandle_t h, hcblasOrder_t order, int M, int N,
   return HCBLAS_STATUS_SUCCESS;
 }
 
-// Workspace of the pair kernel. False where it would have to grow while the
-// stream is being captured, or cannot: the two GEMVs then run instead.
-bool pair_workspace(hcblasHandle_t h, size_t bytes) {
-  if (h->gemv_partials.bytes >= bytes) return true;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(h->stream, &cs) != hipSuccess ||
-      cs != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return false;
-  }
-  if (ensure_workspace(h->gemv_partials, bytes) == hipSuccess) return true;
-  (void)hipGetLastError();
-  return false;
-}
-
 // GER from one matrix into another, D = alpha * x * y^T + A.
 template <typename T>
 hcblasStatus_t ger_out_entry(hcblasHandle_t h, hcblasOrder_t order, int M,
@@ -1086,11 +1073,13 @@ hcblasStatus_t ger_backward_entry(hcblasHandle_t h, hcblasOrder_t order,
       (col || order == HCBLAS_ROW_MAJOR)) {
     const PairPlan plan =
         plan_gemv_pair(h->num_cus, R, Cc, VecT<T>::n, sizeof(T));
-    if (plan.xr && pair_workspace(h, plan.partial_bytes)) {
+    // (the two GEMVs where there is no memory for the partials)
+    T *row_part =
+        plan.xr ? static_cast<T *>(partials(h, plan.partial_bytes)) : nullptr;
+    if (row_part != nullptr) {
       const T *p = col ? x : y, *q = col ? y : x;
       const int64_t incp = col ? incx : incy, incq = col ? incy : incx;
       T *yr = col ? dx : dy, *yc = col ? dy : dx;
-      T *row_part = static_cast<T *>(h->gemv_partials.ptr);
       T *col_part = row_part + plan.blocks * R;
       const dim3 grid((unsigned)plan.blocks, (unsigned)plan.bands);
       const bool nt = (int64_t)sizeof(T) * R * Cc >= kStreamBytes;
