@@ -37,6 +37,8 @@ constexpr int kReduceGrid = kReducePartials;
 // a trip takes about 1 us, the finish launch that it saves 2 us on the GPU and
 // 3 us on the host (SDOT and SASUM of 4099 among three updates: the five calls
 // took 51 us with a finish launch each and a launch per vector tail, now 38).
+// Of several trips it adds in FP64 throughout, as the partials of a workgroup
+// for each were added: 0.2 to 0.5 us of the 9 to 10 against FP32 sums.
 constexpr int kAloneTrips = 4;
 constexpr int kMaxGridY = 65535;
 
@@ -276,8 +278,10 @@ struct ReduceOut {
 
 // Vector-path reduction: grid-stride over 16-byte vectors of x (and y) with
 // U vectors in flight per thread; the scalar tail (< one vector) is added by
-// block 0.
-template <typename T, typename Red, bool NT, int U, int TH = kThreads>
+// block 0. Acc: what a thread adds its elements in: T, but FP64 where a workgroup
+// makes several trips alone (a workgroup for each would add their sums in FP64).
+template <typename T, typename Acc, typename Red, bool NT, int U,
+          int TH = kThreads>
 __global__ __launch_bounds__(TH) void reduce_vec_kernel(
     int64_t n, const T *__restrict__ x, const T *__restrict__ y,
     ReduceOut<T> out, Red red) {
@@ -286,11 +290,11 @@ __global__ __launch_bounds__(TH) void reduce_vec_kernel(
   __shared__ double lds[TH / 64];
   const int64_t nvec = n / VN;
   const int64_t stride = (int64_t)gridDim.x * TH;
-  T acc[U][VN];
+  Acc acc[U][VN];
 #pragma unroll
   for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int e = 0; e < VN; ++e) acc[u][e] = T(0);
+    for (int e = 0; e < VN; ++e) acc[u][e] = Acc(0);
   int64_t i = (int64_t)blockIdx.x * TH + threadIdx.x;
   for (; i + (U - 1) * stride < nvec; i += U * stride) {
     V a[U], b[U];
@@ -332,16 +336,16 @@ __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(
   __shared__ double lds[kThreads / 64];
   const int64_t total = n * batch;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  T acc = T(0);
+  double acc = 0.0;
   for (int64_t f = (int64_t)blockIdx.x * kThreads + threadIdx.x; f < total;
        f += stride) {
     // (no 64-bit division for a single vector)
     const int64_t b = batch == 1 ? 0 : f / n, i = f - b * n;
     T xv = x[b * bsx + blas_index(i, n, incx)];
     T yv = Red::two ? y[b * bsy + blas_index(i, n, incy)] : T(0);
-    acc += red(xv, yv);
+    acc += (double)red(xv, yv);
   }
-  out(block_sum((double)acc, lds));
+  out(block_sum(acc, lds));
 }
 
 // ---------------------------------------------------------------------------
@@ -427,6 +431,9 @@ hcblasStatus_t run_reduce(hcblasHandle_t h, int64_t n, int64_t batch,
     constexpr int U = Red::two ? kReduceUnroll
                       : wide   ? kReduceUnroll
                                : 4 * kReduceUnroll;
+    // A dot of several trips alone: all their loads and FP64 additions in one
+    // trip of as many more waves (SDOT of 16384 10.0 us against 10.4).
+    constexpr int ALONE = Red::two ? kAloneTrips * TH : TH;
     const int64_t nvec = flat / VN;
     const int64_t trips = cdiv(nvec, TH * U);
     nparts = trips <= kAloneTrips
@@ -434,11 +441,14 @@ hcblasStatus_t run_reduce(hcblasHandle_t h, int64_t n, int64_t batch,
                  : (int)std::min<int64_t>(trips, kReduceGrid);
     const int64_t bytes = flat * (int64_t)sizeof(T) * (Red::two ? 2 : 1);
     if (bytes >= kStreamBytes)
-      reduce_vec_kernel<T, Red, true, U, TH>
+      reduce_vec_kernel<T, T, Red, true, U, TH>
+          <<<nparts, TH, 0, h->stream>>>(flat, x, yy, out, red);
+    else if (nparts > 1 || trips <= 1)
+      reduce_vec_kernel<T, T, Red, false, U, TH>
           <<<nparts, TH, 0, h->stream>>>(flat, x, yy, out, red);
     else
-      reduce_vec_kernel<T, Red, false, U, TH>
-          <<<nparts, TH, 0, h->stream>>>(flat, x, yy, out, red);
+      reduce_vec_kernel<T, double, Red, false, U, ALONE>
+          <<<1, ALONE, 0, h->stream>>>(flat, x, yy, out, red);
   } else {
     if (flat > kAloneTrips * kThreads)
       nparts = (int)std::min<int64_t>(full_grid(flat), kReduceGrid);

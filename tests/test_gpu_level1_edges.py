@@ -81,3 +81,28 @@ def test_strided_batches(hc, handle, p, n, batch):
     assert getattr(api, f"hcblas{p}copyBatched")(handle, n, dx, inc, dy, inc,
                                                  batch) == 0
     assert bitwise_equal(to_host(dy), exp)
+
+
+@pytest.mark.parametrize("inc", [1, 2])
+def test_short_float_sums_are_exact(hc, handle, inc):
+    """Up to four trips of one workgroup, FP32 sums are held in FP64: of values
+    that are multiples of 2^-24, whose sums FP64 holds exactly, the result is the
+    exact sum rounded once (FP32 partial sums of two such values already round)."""
+    api = hc.api
+    trip_dot, trip_asum = (4096, 16384) if inc == 1 else (256, 256)
+    for trip, name in ((trip_dot, "dot"), (trip_asum, "asum")):
+        for n in (trip, trip + 1, trip + 4, 2 * trip, 3 * trip - 5, 4 * trip):
+            rng = np.random.default_rng(n)
+            x = rng.integers(1 << 23, 1 << 24, n * inc).astype(np.float64)
+            x = (x * 2.0 ** -24).astype(np.float32)
+            y = rng.choice([-1, 1], n * inc).astype(np.float32)
+            dx, dy = to_dev(x), to_dev(y)
+            xs, ys = x[::inc].astype(np.float64), y[::inc].astype(np.float64)
+            if name == "dot":
+                st, got = api.hcblasSdot(handle, n, dx, inc, dy, inc, None)
+                want = np.float32(np.dot(xs, ys))
+            else:
+                st, got = api.hcblasSasum(handle, n, dx, inc, None)
+                want = np.float32(xs.sum())
+            assert st == 0
+            assert np.float32(got) == want, (name, n, got, want)
