@@ -19,8 +19,6 @@ namespace hcb {
 
 constexpr uint32_t kHandleMagic = 0x48434d49u;  // "HCMI"
 
-// Largest grid of the level-1 elementwise kernels (they grid-stride beyond).
-constexpr int kMaxReduceBlocks = 1 << 21;
 // Reduction scratch (dot / asum): one FP64 partial per workgroup of the
 // bounded reduction grid.
 constexpr int kReducePartials = 256;

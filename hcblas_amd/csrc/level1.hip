@@ -18,11 +18,12 @@
 // host block, whose sequence word the host polls; a short vector's only
 // workgroup publishes its sum itself.
 #include "common.hpp"
+#include "level1_plan.hpp"
 
 namespace hcb {
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = kLevel1Threads;
 // Operands larger than this (bytes) bypass the caches (non-temporal).
 constexpr int64_t kStreamBytes = 64ll << 20;
 // Vector-path reductions: loads in flight per thread and maximum grid. A
@@ -40,7 +41,6 @@ constexpr int kReduceGrid = kReducePartials;
 // Of several trips it adds in FP64 throughout, as the partials of a workgroup
 // for each were added: 0.2 to 0.5 us of the 9 to 10 against FP32 sums.
 constexpr int kAloneTrips = 4;
-constexpr int kMaxGridY = 65535;
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef double d2v __attribute__((ext_vector_type(2)));
@@ -145,20 +145,29 @@ __global__ __launch_bounds__(kThreads) void elementwise_vec_kernel(
 }
 
 // Scalar path: any increments. Element (b, i) of the batch lives at
-// base + b*bstride + blas_index(i, n, inc); blockIdx.y walks the batch.
-template <typename T, typename Op>
+// base + b*bstride + blas_index(i, n, inc). ROWS: see plan_strided.
+template <typename T, typename Op, bool ROWS>
 __global__ __launch_bounds__(kThreads) void elementwise_strided_kernel(
     int64_t n, int64_t batch, const T *__restrict__ x, int64_t incx,
     int64_t bsx, T *__restrict__ y, int64_t incy, int64_t bsy, Op op) {
+  const int64_t first = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t b = blockIdx.y; b < batch; b += gridDim.y)
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-         i += stride) {
-      const int64_t ix = b * bsx + blas_index(i, n, incx);
-      const int64_t iy = b * bsy + blas_index(i, n, incy);
-      const T yv = Op::reads_y ? y[iy] : T(0);
-      y[iy] = op(x[ix], yv);
+  auto update = [&](int64_t b, int64_t i) {
+    const int64_t ix = b * bsx + blas_index(i, n, incx);
+    const int64_t iy = b * bsy + blas_index(i, n, incy);
+    const T yv = Op::reads_y ? y[iy] : T(0);
+    y[iy] = op(x[ix], yv);
+  };
+  if constexpr (ROWS) {
+    for (int64_t b = blockIdx.y; b < batch; b += gridDim.y)
+      for (int64_t i = first; i < n; i += stride) update(b, i);
+  } else {
+    const int64_t total = n * batch;
+    for (int64_t f = first; f < total; f += stride) {
+      const int64_t b = f / n;
+      update(b, f - b * n);
     }
+  }
 }
 
 // Complex scal. Products are rounded separately (contraction is switched
@@ -351,12 +360,6 @@ __global__ __launch_bounds__(kThreads) void reduce_strided_kernel(
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
-int full_grid(int64_t work_items) {
-  int64_t g = cdiv(work_items, kThreads);
-  if (g < 1) g = 1;
-  return (int)(g < kMaxReduceBlocks ? g : kMaxReduceBlocks);
-}
-
 template <typename T, typename Op>
 hcblasStatus_t run_elementwise(hcblasHandle_t h, int64_t n, int64_t batch,
                                const T *x, int64_t incx, int64_t bsx, T *y,
@@ -378,10 +381,11 @@ hcblasStatus_t run_elementwise(hcblasHandle_t h, int64_t n, int64_t batch,
           <<<grid, kThreads, 0, h->stream>>>(flat, x, y, op);
     return launch_status();
   }
-  dim3 grid((unsigned)full_grid(n),
-            (unsigned)std::min<int64_t>(batch, kMaxGridY));
-  elementwise_strided_kernel<T, Op><<<grid, kThreads, 0, h->stream>>>(
-      n, batch, x, incx, bsx, y, incy, bsy, op);
+  const StridedGrid g = plan_strided(n, batch);
+  (g.rows ? elementwise_strided_kernel<T, Op, true>
+          : elementwise_strided_kernel<T, Op, false>)
+      <<<dim3(g.x, g.y), kThreads, 0, h->stream>>>(n, batch, x, incx, bsx, y,
+                                                   incy, bsy, op);
   return launch_status();
 }
 

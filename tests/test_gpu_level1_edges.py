@@ -106,3 +106,36 @@ def test_short_float_sums_are_exact(hc, handle, inc):
                 want = np.float32(xs.sum())
             assert st == 0
             assert np.float32(got) == want, (name, n, got, want)
+
+
+@pytest.mark.parametrize("p", ["S", "D"])
+@pytest.mark.parametrize("n,batch", [(1, 1000), (5, 300), (191, 9), (192, 9),
+                                     (255, 70), (257, 70), (383, 5), (384, 5),
+                                     (16, 70000), (250, 70000)])
+@pytest.mark.parametrize("inc", [1, -2])
+def test_strided_update_grids(hc, handle, p, n, batch, inc):
+    """Batches of short vectors at a batch stride of their own: the flat grid, and
+    the one by rows, with more vectors than it has rows. Gaps keep their bits."""
+    dt = DT[p]
+    step = n * abs(inc) + 3
+    rng = np.random.default_rng(n + batch)
+    x = rng.uniform(-1, 1, (batch, step)).astype(dt)
+    y = rng.uniform(-1, 1, (batch, step)).astype(dt)
+    dy = to_dev(y)
+    assert getattr(hc.api, f"hcblas_{p.lower()}axpy_batched")(
+        handle, n, -1.5, to_dev(x), inc, step, dy, abs(inc), step, 0, 0,
+        batch) == 0
+    xs = x[:, :n * abs(inc):abs(inc)]
+    exp = y.copy()
+    # one fused operation: the exact product and sum of these values rounds once
+    wide = np.longdouble if p == "D" else np.float64
+    s = xs[:, ::-1] if inc < 0 else xs
+    exp[:, :n * abs(inc):abs(inc)] = (
+        wide(-1.5) * s.astype(wide) + y[:, :n * abs(inc):abs(inc)].astype(wide)
+    ).astype(dt)
+    got = to_host(dy)
+    gaps = np.ones(step, bool)
+    gaps[:n * abs(inc):abs(inc)] = False
+    assert bitwise_equal(got[:, gaps], y[:, gaps])
+    # (a double rounding of the wide form differs by at most one ulp)
+    assert np.all(abs(got - exp) <= np.finfo(dt).eps * abs(exp))
