@@ -69,8 +69,8 @@ __device__ __forceinline__ void tile_body(const ProbDev &p, int m0, int n0,
                                           int tid, char *lds) {
   using T = typename ElemT<E>::T;
   constexpr int BK = E == Elem::F32 ? kF32BK : kF16BK;
-  gemm_tile<E, OutT, A_K, B_K, TM, TM, BK, 2, 2, 16, GroupCfg<TM>::LDS,
-            NARROW>(
+  gemm_tile<E, OutT, A_K, B_K, TM, TM, BK, 2, 2, 16, GroupCfg<TM>::LDS, NARROW,
+            false, false>(
       static_cast<const T *>(p.A), p.lda, static_cast<const T *>(p.B), p.ldb,
       static_cast<OutT *>(p.C), p.ldc, p.M, p.N, p.K, p.alpha, p.beta, m0, n0,
       tid, lds);

@@ -361,7 +361,11 @@ struct TileLoader {
     return w;
   }
 
-  // An operand shorter than one vector, element by element.
+  // An operand shorter than one vector, element by element. EACH: only the
+  // elements inside it (most vectors of a narrow tile lie outside); otherwise
+  // clamped loads, one vector's addresses at a time, for kernels whose registers
+  // this path must not cost.
+  template <bool EACH = false>
   __device__ __forceinline__ void load_narrow(const T *__restrict__ P,
                                               int64_t ld, int r0, int k0,
                                               int R, int K) {
@@ -375,13 +379,18 @@ struct TileLoader {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const int gr = r0 + r + (KCONT ? 0 : e), gk = k0 + k + (KCONT ? e : 0);
-        const int64_t rr = gr < R ? gr : R - 1, kk = gk < K ? gk : K - 1;
-        const T x = KCONT ? P[rr * ld + kk] : P[kk * ld + rr];
-        t[e] = gk < K ? x : T(0);
+        if constexpr (EACH) {
+          t[e] = T{};
+          if (gr < R && gk < K)
+            t[e] = P[KCONT ? gr * ld + gk : gk * ld + gr];
+        } else {
+          const int64_t rr = gr < R ? gr : R - 1, kk = gk < K ? gk : K - 1;
+          const T x = KCONT ? P[rr * ld + kk] : P[kk * ld + rr];
+          t[e] = gk < K ? x : T(0);
+        }
       }
       __builtin_memcpy(&reg[i], t, 16);
-      // One vector's addresses at a time: this path must not cost registers.
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!EACH) __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -516,10 +525,11 @@ struct ComplexLoader
     L::template load_wide<FULL>(reinterpret_cast<const CT *>(P), ld, r0 / RD,
                                 k0 / 2, R / RD, K / 2);
   }
+  template <bool EACH = false>
   __device__ __forceinline__ void load_narrow(const T *P, int64_t ld, int r0,
                                               int k0, int R, int K) {
     kv = (K - k0) / 2;
-    L::load_narrow(reinterpret_cast<const CT *>(P), ld, r0 / RD, k0 / 2,
+    L::template load_narrow<EACH>(reinterpret_cast<const CT *>(P), ld, r0 / RD, k0 / 2,
                    R / RD, K / 2);
   }
   __device__ __forceinline__ void mask(int k0, int K) { L::mask(k0 / 2, K / 2); }
@@ -898,11 +908,11 @@ __device__ __forceinline__ void gemm_mainloop(
     if (wide_a)
       la.template load_wide<false>(A, lda, m0, k * BK, M, K);
     else
-      la.load_narrow(A, lda, m0, k * BK, M, K);
+      la.template load_narrow<true>(A, lda, m0, k * BK, M, K);
     if (wide_b)
       lb.template load_wide<false>(B, ldb, n0, k * BK, N, K);
     else
-      lb.load_narrow(B, ldb, n0, k * BK, N, K);
+      lb.template load_narrow<true>(B, ldb, n0, k * BK, N, K);
   };
   auto store = [&](int k) {
     if ((k + 1) * BK > K) {
@@ -966,12 +976,13 @@ __device__ __forceinline__ void gemm_mainloop(
 //   16x16 FP64: row l / 16 + 4 r, column l % 16.
 // edge_m / shift_m, edge_n / shift_n: the loaders' edge_row and edge_shift of
 // either operand. Output row m >= edge_m lies in tile row m + shift_m (and
-// columns alike); those few rows leave one by one. C is accessed 16 bytes at
-// a time at any alignment.
+// columns alike). C is accessed 16 bytes at a time at any alignment; one by one
+// leave the rows of a vector that reaches past M, or over edge_m (16-bit outputs
+// of an FP32 operand, whose vectors are shorter). BOTH: below.
 // Expects the LDS free on entry (the main loop ends with a barrier) and ends
 // with a barrier.
 template <Elem E, typename OutT, int BM, int BN, int WM, int WN, int MI,
-          int LDS_BYTES, typename AccArr>
+          int LDS_BYTES, bool BOTH = true, typename AccArr>
 __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
                                                int64_t ldc, int M, int N,
                                                int m0, int n0, double alpha_d,
@@ -1030,39 +1041,55 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
       }
     }
     __syncthreads();
+    // Two loops, one for tiles with moved rows: there a moved vector is read
+    // from LDS by elements and stored whole (BF16 156 x 128x92x28 8.7 -> 6.3 us).
+    // Without BOTH, one loop in which moved rows also leave one by one, for a
+    // kernel of many tile bodies, whose code size counts.
+    auto columns = [&](auto moved) {
 #pragma unroll
-    for (int cc = 0; cc < NC; cc += NTH / TPC) {
-      const int nl = cc + tid / TPC;
-      const int ml = (tid % TPC) * VE;
-      const int n = n0 + c0 + nl, m = m0 + ml;
-      if (nl < NC && n < N && m < M) {
-        OutT *dst = C + (int64_t)n * ldc + m;
-        const Acc *src = t + (n < edge_n ? nl : nl + shift_n) * LROW + ml;
-        if (m + VE <= edge_m) {
-          OutT cin[VE], o[VE];
-          if (beta != Acc(0)) {
-            const vec4u w = *reinterpret_cast<const GV *>(dst);
-            __builtin_memcpy(cin, &w, 16);
-          }
+      for (int cc = 0; cc < NC; cc += NTH / TPC) {
+        const int nl = cc + tid / TPC;
+        const int ml = (tid % TPC) * VE;
+        const int n = n0 + c0 + nl, m = m0 + ml;
+        if (nl < NC && n < N && m < M) {
+          OutT *dst = C + (int64_t)n * ldc + m;
+          const Acc *src = t + (n < edge_n ? nl : nl + shift_n) * LROW + ml;
+          const bool below = !decltype(moved)::value || m < edge_m;
+          const int up = below || !BOTH ? 0 : shift_m;
+          if (m + VE <= (decltype(moved)::value && (below || !BOTH) ? edge_m
+                                                                    : M)) {
+            OutT cin[VE], o[VE];
+            if (beta != Acc(0)) {
+              const vec4u w = *reinterpret_cast<const GV *>(dst);
+              __builtin_memcpy(cin, &w, 16);
+            }
 #pragma unroll
-          for (int e = 0; e < VE; ++e) {
-            Acc v = alpha * src[e];
-            if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(cin[e]), v);
-            o[e] = to_out<OutT>(v);
-          }
-          vec4u w;
-          __builtin_memcpy(&w, o, 16);
-          *reinterpret_cast<GV *>(dst) = w;
-        } else {
-          const int ne = M - m < VE ? M - m : VE;
-          for (int e = 0; e < ne; ++e) {
-            Acc v = alpha * src[m + e < edge_m ? e : e + shift_m];
-            if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(dst[e]), v);
-            dst[e] = to_out<OutT>(v);
+            for (int e = 0; e < VE; ++e) {
+              Acc v = alpha * src[e + up];
+              if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(cin[e]), v);
+              o[e] = to_out<OutT>(v);
+            }
+            vec4u w;
+            __builtin_memcpy(&w, o, 16);
+            *reinterpret_cast<GV *>(dst) = w;
+          } else {
+            const int ne = M - m < VE ? M - m : VE;
+#pragma unroll 1
+            for (int e = 0; e < ne; ++e) {
+              const int s =
+                  decltype(moved)::value && m + e >= edge_m ? e + shift_m : e;
+              Acc v = alpha * src[s];
+              if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(dst[e]), v);
+              dst[e] = to_out<OutT>(v);
+            }
           }
         }
       }
-    }
+    };
+    if (BOTH && (shift_m == 0 || m0 + BM <= edge_m))
+      columns(std::false_type{});
+    else
+      columns(std::true_type{});
     __syncthreads();
   }
 }
@@ -1070,8 +1097,8 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
 // One BM x BN output tile at (m0, n0) of C = alpha*A'*B' + beta*C, the whole
 // K range; beta == 0 never reads C. LDS_BYTES: the LDS at `lds`.
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
-          int WM, int WN, int MI, int LDS_BYTES, bool NARROW = true,
-          bool CX = false>
+          int WM, int WN, int MI, int LDS_BYTES, bool NARROW, bool CX = false,
+          bool BOTH = true>
 __device__ __forceinline__ void gemm_tile(
     const typename ElemT<E>::T *__restrict__ A, int64_t lda,
     const typename ElemT<E>::T *__restrict__ B, int64_t ldb, OutT *C,
@@ -1085,13 +1112,17 @@ __device__ __forceinline__ void gemm_tile(
   typename WT::AccV acc[WT::FM][WT::FN];
   gemm_mainloop<E, A_K, B_K, BM, BN, BK, WM, WN, MI, NARROW, CX>(
       A, lda, B, ldb, M, N, K, m0, n0, tid, lds, cx, acc);
-  store_tile_lds<E, OutT, BM, BN, WM, WN, MI, LDS_BYTES>(
+  store_tile_lds<E, OutT, BM, BN, WM, WN, MI, LDS_BYTES, BOTH>(
       acc, C, ldc, M, N, m0, n0, alpha_d, beta_d, tid, lds,
       LA::edge_row(M), LA::edge_shift(M), LB::edge_row(N), LB::edge_shift(N));
 }
 
+// NARROW: an operand may be shorter than one vector along its contiguous
+// dimension (the host knows; carrying the element-wise loads in every kernel cost
+// 1-5%: SGEMM 1024^3 NN row-major 22.95 us against 22.55, HGEMM 1024^3 NN 9.24
+// against 8.82, sixty-four 96^3 CGEMMs 10.7 against 10.3).
 template <Elem E, typename OutT, bool A_K, bool B_K, int BM, int BN, int BK,
-          int WM, int WN, int MI = 16, bool CX = false>
+          int WM, int WN, int MI = 16, bool CX = false, bool NARROW = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     GemmParams p) {
   using T = typename ElemT<E>::T;
@@ -1116,7 +1147,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     C = static_cast<OutT *>(p.C) + p.cOff + (int64_t)z * p.strideC;
   int tile_m, tile_n;
   tile_coords(pid, p.tiles_m, p.tiles_n, tile_m, tile_n, gridDim.z < 8);
-  gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES, true, CX>(
+  gemm_tile<E, OutT, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES, NARROW, CX>(
       A, p.lda, B, p.ldb, C, p.ldc, p.M, p.N, p.K, p.alpha, p.beta,
       tile_m * BM, tile_n * BN, threadIdx.x, lds,
       CX ? ComplexArgs{p.cx_ar, p.cx_ai, p.conj_a, p.conj_b} : ComplexArgs{});
@@ -1127,8 +1158,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
 // W + z M N (column-major, ld M). For problems with about as many tiles as
 // CUs and a long K, splitting K gives every CU several workgroups to switch
 // between; splitk_reduce_kernel then adds the partials in split order.
+// (The last slice of K may be shorter than a vector: of a k-contiguous operand
+// that is as wide as one, the vector then begins in the slice before.)
 template <Elem E, bool A_K, bool B_K, int BM, int BN, int BK, int WM, int WN,
-          int MI, bool CX = false>
+          int MI, bool CX = false, bool NARROW = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_splitk_kernel(
     GemmParams p, int ks, typename ElemT<E>::Acc *W) {
   using T = typename ElemT<E>::T;
@@ -1145,7 +1178,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_splitk_kernel(
                (B_K ? (int64_t)k0 : (int64_t)k0 * p.ldb);
   int tile_m, tile_n;
   tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-  gemm_tile<E, Acc, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES, true, CX>(
+  gemm_tile<E, Acc, A_K, B_K, BM, BN, BK, WM, WN, MI, LDS_BYTES, NARROW, CX>(
       A, p.lda, B, p.ldb, W + (int64_t)z * p.M * p.N, p.M, p.M, p.N, kl, 1.0,
       0.0, tile_m * BM, tile_n * BN, threadIdx.x, lds,
       CX ? ComplexArgs{p.cx_ar, p.cx_ai, p.conj_a, p.conj_b} : ComplexArgs{});

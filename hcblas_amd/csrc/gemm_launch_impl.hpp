@@ -31,7 +31,7 @@ template <>
 struct TileCfg<Elem::BF16> : TileCfg<Elem::F16> {};
 
 template <Elem E, typename OutT, int BM, int BN, int BK, int WM, int WN,
-          int MI = 16, bool CX = false>
+          int MI = 16, bool CX = false, bool NARROW = false>
 hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
                             bool b_k, int64_t batch) {
   p.tiles_m = (int)cdiv(p.M, BM);
@@ -50,9 +50,9 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
       else q.C = (char *)q.C + b0 * q.strideC * sizeof(OutT);
     }
     dim3 grid(tiles, 1, (unsigned)nb);
-#define HCB_GEMM_CASE(AK, BKC)                                   \
-  if (a_k == AK && b_k == BKC)                                   \
-    gemm_mfma_kernel<E, OutT, AK, BKC, BM, BN, BK, WM, WN, MI, CX> \
+#define HCB_GEMM_CASE(AK, BKC)                                             \
+  if (a_k == AK && b_k == BKC)                                             \
+    gemm_mfma_kernel<E, OutT, AK, BKC, BM, BN, BK, WM, WN, MI, CX, NARROW> \
         <<<grid, 64 * WM * WN, 0, stream>>>(q);
     HCB_GEMM_CASE(false, false)
     HCB_GEMM_CASE(false, true)
@@ -134,6 +134,68 @@ const MacroTile &pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch,
   return *best;
 }
 
+// An operand shorter than one vector along its contiguous dimension (see
+// TileLoader).
+template <Elem E, bool CX>
+bool is_narrow(const GemmParams &p, bool a_k, bool b_k) {
+  constexpr int CE = CX ? 2 : 1;  // reals per element
+  constexpr int VEC = 16 / (CE * (int)sizeof(typename ElemT<E>::T));
+  return (a_k ? p.K : p.M) / CE < VEC || (b_k ? p.K / CE : p.N) < VEC;
+}
+
+// 64x64 (or, with `t32`, 32x32) tiles, `tiles` of them.
+template <Elem E, typename OutT, bool CX, bool NARROW>
+hcblasStatus_t launch_small(hipStream_t stream, int num_cus, GemmParams p,
+                            bool a_k, bool b_k, int64_t batch, bool t32,
+                            int64_t tiles) {
+  using C = TileCfg<E>;
+  if (t32) {
+    if (p.K >= C::LONG_K && tiles <= num_cus)
+      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2, 16, CX, NARROW>(
+          stream, p, a_k, b_k, batch);
+    // (16-bit r-contiguous tiles of 128-deep steps are transposed in
+    // registers: 8192 x 8192 x 1024 HGEMM NN 564 us against 743)
+    if (sizeof(typename ElemT<E>::T) == 2 && !(a_k && b_k))
+      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2, 16, CX, NARROW>(
+          stream, p, a_k, b_k, batch);
+    return launch_tiles<E, OutT, 32, 32, C::BK_32, 2, 2, 16, CX, NARROW>(
+        stream, p, a_k, b_k, batch);
+  }
+  // 64x64 tiles. At most one tile per CU leaves nothing else to cover a tile's
+  // load latency: FP32 then runs 8 waves and long K steps (1024^3 NN 22.8 us
+  // with 128, 23.7 with 64, 27.5 with 4 waves and 32), FP64 32-deep ones
+  // (1024^3 42.3 against 44.1). With more tiles than CUs, 4 waves and short
+  // steps are ahead for FP32 (4096 x 4096 x 256 NN 84 us against 89 with 8
+  // waves and 92 with 64-deep steps), and so they are where one step is all.
+  // FP32 tiles of a single 32-deep step, and narrow 16-bit ones, take 8 waves,
+  // which share its loads and the epilogue: SGEMM 3025 x 96 x 1 4.6 -> 3.8 us,
+  // 3200 x 256 x 23 5.0 -> 4.1, HGEMM 1000 x 1000 x 4 4.1 -> 3.8 (but HGEMM 2000 x
+  // 1000 x 48 4.6 -> 5.5, CGEMM 500 x 300 x 16 4.4 -> 5.8).
+  if constexpr (!CX && (E == Elem::F32 || (NARROW && E != Elem::F64))) {
+    if (p.K <= C::BK_64)
+      return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 4, 16, CX, NARROW>(
+          stream, p, a_k, b_k, batch);
+  }
+  if constexpr (E == Elem::F32) {
+    if (p.K >= 512 && tiles <= num_cus)
+      return launch_tiles<E, OutT, 64, 64, 128, 2, 4, 16, CX, NARROW>(
+          stream, p, a_k, b_k, batch);
+    if (tiles <= num_cus)
+      return launch_tiles<E, OutT, 64, 64, 64, 2, 4, 16, CX, NARROW>(
+          stream, p, a_k, b_k, batch);
+  }
+  if constexpr (E == Elem::F64) {
+    if (tiles <= num_cus && p.K > C::BK_64)
+      return launch_tiles<E, OutT, 64, 64, 32, 2, 4, 16, CX, NARROW>(
+          stream, p, a_k, b_k, batch);
+    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 4, 16, CX, NARROW>(
+        stream, p, a_k, b_k, batch);
+  } else {
+    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 2, 16, CX, NARROW>(
+        stream, p, a_k, b_k, batch);
+  }
+}
+
 template <Elem E, typename OutT, bool CX>
 hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
                            bool a_k, bool b_k, int64_t batch) {
@@ -141,7 +203,23 @@ hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
   const MacroTile &t =
       pick_tile<E>(p.M, p.N, p.K, batch, num_cus,
                    CX ? 0 : (a_k ? 0 : 1) + (b_k ? 0 : 1));
-  const int64_t tiles = cdiv(p.M, t.bm) * cdiv(p.N, t.bn) * batch;
+  auto tiles = [&](int bm, int bn) {
+    return cdiv(p.M, bm) * cdiv(p.N, bn) * batch;
+  };
+  // Narrow operands are a few rows or a K below one vector: the small tiles do
+  // for them, and for 16-bit ones those of 128x128 (8192 x 8192 x 4 HGEMM 42 us,
+  // on 64x64 tiles 58; SGEMM 72 on 64x64).
+  if (is_narrow<E, CX>(p, a_k, b_k)) {
+    if constexpr (sizeof(typename ElemT<E>::T) == 2) {
+      if (t.bm >= 128)
+        return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 4, 32, CX, true>(
+            stream, p, a_k, b_k, batch);
+    }
+    const bool t32 = t.bm == 32;
+    return launch_small<E, OutT, CX, true>(
+        stream, num_cus, p, a_k, b_k, batch, t32,
+        t32 ? tiles(32, 32) : tiles(64, 64));
+  }
   if constexpr (E == Elem::F64) {
     if (t.bm == 256)
       return launch_tiles<E, OutT, 256, 128, C::BK_BIG, 4, 2, 16, CX>(
@@ -168,42 +246,8 @@ hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
             stream, p, a_k, b_k, batch);
     }
   }
-  if (t.bm == 32) {
-    if (p.K >= C::LONG_K && tiles <= num_cus)
-      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2, 16, CX>(
-          stream, p, a_k, b_k, batch);
-    // (16-bit r-contiguous tiles of 128-deep steps are transposed in
-    // registers: 8192 x 8192 x 1024 HGEMM NN 564 us against 743)
-    if (sizeof(typename ElemT<E>::T) == 2 && !(a_k && b_k))
-      return launch_tiles<E, OutT, 32, 32, C::BK_32_LONG, 2, 2, 16, CX>(
-          stream, p, a_k, b_k, batch);
-    return launch_tiles<E, OutT, 32, 32, C::BK_32, 2, 2, 16, CX>(
-        stream, p, a_k, b_k, batch);
-  }
-  // 64x64 tiles. At most one tile per CU leaves nothing else to cover a tile's
-  // load latency: FP32 then runs 8 waves and long K steps (1024^3 NN 22.8 us
-  // with 128, 23.7 with 64, 27.5 with 4 waves and 32), FP64 32-deep ones
-  // (1024^3 42.3 against 44.1). With more tiles than CUs, 4 waves and short
-  // steps are ahead for FP32 (4096 x 4096 x 256 NN 84 us against 89 with 8
-  // waves and 92 with 64-deep steps).
-  if constexpr (E == Elem::F32) {
-    if (p.K >= 512 && tiles <= num_cus)
-      return launch_tiles<E, OutT, 64, 64, 128, 2, 4, 16, CX>(
-          stream, p, a_k, b_k, batch);
-    if (tiles <= num_cus)
-      return launch_tiles<E, OutT, 64, 64, 64, 2, 4, 16, CX>(
-          stream, p, a_k, b_k, batch);
-  }
-  if constexpr (E == Elem::F64) {
-    if (tiles <= num_cus)
-      return launch_tiles<E, OutT, 64, 64, 32, 2, 4, 16, CX>(
-          stream, p, a_k, b_k, batch);
-    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 4, 16, CX>(
-        stream, p, a_k, b_k, batch);
-  } else {
-    return launch_tiles<E, OutT, 64, 64, C::BK_64, 2, 2, 16, CX>(
-        stream, p, a_k, b_k, batch);
-  }
+  return launch_small<E, OutT, CX, false>(stream, num_cus, p, a_k, b_k, batch,
+                                          t.bm == 32, tiles(t.bm, t.bn));
 }
 
 template <Elem E, int T, int BK, int WM, int WN, bool CX>
@@ -212,9 +256,11 @@ void launch_splitk_tiles(hipStream_t stream, GemmParams p, bool a_k, bool b_k,
   p.tiles_m = (int)cdiv(p.M, T);
   p.tiles_n = (int)cdiv(p.N, T);
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)sk.splits);
-#define HCB_SPLITK_CASE(AK, BKC)                          \
-  if (a_k == AK && b_k == BKC)                            \
-    gemm_splitk_kernel<E, AK, BKC, T, T, BK, WM, WN, 16, CX> \
+  const bool narrow = is_narrow<E, CX>(p, a_k, b_k);
+#define HCB_SPLITK_CASE(AK, BKC)                                           \
+  if (a_k == AK && b_k == BKC)                                             \
+    (narrow ? gemm_splitk_kernel<E, AK, BKC, T, T, BK, WM, WN, 16, CX, true>   \
+            : gemm_splitk_kernel<E, AK, BKC, T, T, BK, WM, WN, 16, CX, false>) \
         <<<grid, 64 * WM * WN, 0, stream>>>(p, sk.ks, W);
   HCB_SPLITK_CASE(false, false)
   HCB_SPLITK_CASE(false, true)

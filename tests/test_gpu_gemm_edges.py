@@ -140,3 +140,56 @@ def test_complex_edges(hc, handle, p, ta, tb):
         assert np.array_equal(got.T[M], C.T[M])
         assert np.all(abs(got.T[:M] - ref) <= 2 * (2 * K + 6) * eps * mag), \
             (M, N, K)
+
+
+# Operands shorter than one vector (K or rows), beside whole ones, on small and
+# large outputs; K slices of a split product whose last one is a single element
+# (the k-contiguous vector then begins in the slice before).
+NARROW = [("s", 300, 517, 1), ("s", 300, 517, 3), ("s", 3, 517, 300),
+          ("s", 517, 2, 300), ("s", 3, 65, 2305), ("s", 35, 66, 2305),
+          ("s", 1100, 1030, 2), ("d", 300, 517, 1), ("d", 1, 517, 300),
+          ("d", 517, 1, 130), ("d", 1, 65, 2241), ("d", 35, 66, 2241),
+          ("h", 300, 517, 1), ("h", 300, 517, 7), ("h", 5, 517, 300),
+          ("h", 517, 7, 300), ("h", 7, 65, 2305), ("h", 35, 66, 2305),
+          ("h", 2100, 2050, 5), ("h", 2100, 7, 70)]
+
+
+@pytest.mark.parametrize("p,M,N,K", NARROW)
+@pytest.mark.parametrize("order", [ROW, COL])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_narrow_operands(hc, handle, p, M, N, K, order, ta, tb):
+    for skew in (0, 1):
+        _check(hc, handle, p, order, ta, tb, M, N, K, skew, M + N + K)
+
+
+@pytest.mark.parametrize("p,K", [("c", 1), ("c", 1153), ("z", 1), ("z", 1121)])
+@pytest.mark.parametrize("M,N", [(1, 40), (37, 1), (35, 66), (300, 130)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (2, 2)])
+def test_narrow_complex(hc, handle, p, K, M, N, ta, tb):
+    """The same for complex products, within test_complex_edges' bound."""
+    dt, rt = (np.complex64, np.float32) if p == "c" else (np.complex128,
+                                                          np.float64)
+    rng = np.random.default_rng(M + N + K)
+
+    def rand(r, c):
+        return (rng.uniform(-1, 1, (r, c))
+                + 1j * rng.uniform(-1, 1, (r, c))).astype(dt)
+
+    A = rand(K, M) if ta == 0 else rand(M, K)  # column-major storage
+    B = rand(N, K) if tb == 0 else rand(K, N)
+    C = rand(N, M)
+    dC = to_dev(C)
+    alpha, beta = 1.25 - 0.5j, 0.75 + 0j
+    assert getattr(hc.api, f"hcblas_{p}gemm")(
+        handle, 1, ta, tb, M, N, K, alpha, to_dev(A), 0, A.shape[1], to_dev(B),
+        0, B.shape[1], beta, dC, 0, M) == 0
+    got = to_host(dC).T
+
+    def op(X, t):
+        X = X.astype(np.complex128)
+        return X.T if t == 0 else X if t == 1 else X.conj()
+
+    a, b = op(A, ta), op(B, tb)
+    ref = alpha * (a @ b) + beta * C.T.astype(np.complex128)
+    mag = abs(alpha) * (abs(a) @ abs(b)) + abs(beta * C.T)
+    assert np.all(abs(got - ref) <= 2 * (2 * K + 6) * np.finfo(rt).eps * mag)
