@@ -791,9 +791,13 @@ __device__ __forceinline__ void gemm_mainloop(
   // workgroups per CU) gains the same way (2048^3 SGEMM 166 against 187 us),
   // and so does the 8-wave 128 x 64 FP64 tile (2048^3 DGEMM 294 against
   // 344 us); the 4-wave 128 x 128 16-bit tile, with 4 MFMAs per chunk, was
-  // 5-18% slower with it.
-  constexpr bool ILV = !PIPE && ((WM * WN == 8 && FM * FN >= 4) ||
-                                 (WM * WN == 4 && MI == 16 && FM * FN >= 8));
+  // 5-18% slower with it. The complex 64 x 64 FP32 tile of 4 waves, whose LDS
+  // writes wait for the embedding's arithmetic, gains most: 1024^3 CGEMM NN 94.9
+  // us with the writes before the MFMAs, 77.4 among them (and 93.4 for the
+  // embedding written to memory first); 6144 x 160 x 3208 289, 232 (254).
+  constexpr bool ILV =
+      !PIPE && ((WM * WN == 8 && FM * FN >= 4) ||
+                (WM * WN == 4 && MI == 16 && FM * FN >= (CX ? 4 : 8)));
   // 16-bit tiles have 8 MFMAs per chunk, too few to carry a whole step's
   // writes and loads: their four chunks take A's LDS writes, B's, A's loads
   // and B's loads in turn (8192^3 HGEMM 2-4% faster than all in chunk 0).
