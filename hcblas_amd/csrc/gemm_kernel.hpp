@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemm_tiles.hpp"
 
 namespace hcb {
 
@@ -42,8 +43,6 @@ typedef double doublex4 __attribute__((ext_vector_type(4)));
 typedef int intx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-enum class Elem { F32, F64, F16, BF16, I8 };
 
 template <Elem E>
 struct ElemT;

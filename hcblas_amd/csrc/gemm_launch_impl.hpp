@@ -65,84 +65,6 @@ hcblasStatus_t launch_tiles(hipStream_t stream, GemmParams p, bool a_k,
   return HCBLAS_STATUS_SUCCESS;
 }
 
-// Macro tiles, largest first, and the rate of each in TF/s over a grid of many
-// tiles (8192 x 8192 x 1024 on MI355X), with 0, 1 or 2 operands r-contiguous
-// (transposed on their way into LDS):
-//   FP32  256x256x32, 8 waves of 128x64 on 32x32 MFMA blocks (146-148 TF/s at
-//         8192^3, 93-94% of peak), 256x128 8 waves, 128x128, 64x64 and 32x32 4
-//         waves;
-//   FP64  256x128x16, 8 waves of 64x64 (71.6 TF/s at 8192^3, 91%), 128x64, 64x64
-//         8 waves, 32x32 4 waves;
-//   F16 / BF16 256x256x64, 8 waves on 32x32 blocks, 128x128 8 waves of 64x32,
-//         64x64 4 waves (8192 x 8192 x 1024 HGEMM NN 292 us against 655 with 8,
-//         whose r-contiguous tiles go to LDS by elements), 32x32 4 waves.
-//
-// `lead`: time of a tile beside its K loop, in k. One 16-bit 256x256 tile fills a
-// CU's LDS, so nothing runs beside its first loads and its epilogue, as long as
-// 128 k together; of the others two or more share a CU. (BF16 12x 807x775x189
-// 30 us on 256x256 tiles, 21 on 128x128; HGEMM 64x 446x732x224 36 and 31; but 64x
-// 512^3 30 and 35, 120x 913x750x666 236 and 303.) An FP32 / FP64 32x32 tile pays
-// three times as much for its area as the larger ones (SGEMM 120x 203x698x84 79 us
-// on 32x32, 54 on 64x64, 120x 277x347x69 57 and 41; DGEMM 827x5055x167 45 and 38;
-// CGEMM 120x 130x130x40 28 and 24, ZGEMM 10x 500x400x100 46.6 and 44.9; but SGEMM
-// 8x 255x257x517 16.3 and 17.1, CGEMM 64x 96^3 11.2 and 13.1).
-struct MacroTile {
-  int bm, bn;
-  int rate[3];
-  int lead = 0;
-};
-template <Elem E>
-inline constexpr MacroTile kTiles[] = {{256, 256, {1180, 1110, 916}, 128},
-                                       {128, 128, {1017, 820, 589}},
-                                       {64, 64, {610, 465, 304}},
-                                       {32, 32, {330, 238, 152}}};
-template <>
-inline constexpr MacroTile kTiles<Elem::F32>[] = {
-    {256, 256, {140, 140, 133}, 20},
-    {256, 128, {128, 128, 129}, 20},
-    {128, 128, {133, 129, 127}, 20},
-    {64, 64, {120, 117, 114}, 20},
-    {32, 32, {105, 97, 80}, 60}};
-template <>
-inline constexpr MacroTile kTiles<Elem::F64>[] = {
-    {256, 128, {68, 68, 68}, 10},
-    {128, 64, {68, 68, 67}, 10},
-    {64, 64, {66, 65, 65}, 10},
-    {32, 32, {57, 54, 52}, 35}};
-
-// The tile with the least time on the CU that gets the most tiles,
-// ceil(tiles / CUs) * area * (K + lead) / rate: tiles past the edge of C and a
-// last round that leaves most CUs idle count in full. (Taking the largest tile
-// whose grid covers every CU instead: 3072 x 3072 x 1024 SGEMM NN 267 us on 288
-// tiles of 256x128, 180 on 2304 of 64x64; 5512 x 6720 x 1024 738 on 256x256, 658
-// on 128x128; a batch of 212 512 x 37 x 32 DGEMMs 36 us on 256x128, 21 on 64x64;
-// 529 x 192 x 1152 28.8 on 27 tiles of 64x64, 12.1 on 32x32.)
-template <Elem E>
-const MacroTile &pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch,
-                           int num_cus, int r_contiguous) {
-  const MacroTile *best = nullptr;
-  double least = 0;
-  for (const MacroTile &t : kTiles<E>) {
-    const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
-    const double time = (double)cdiv(tiles, num_cus) * t.bm * t.bn *
-                        (double)(K + t.lead) / t.rate[r_contiguous];
-    if (best == nullptr || time < least) {
-      best = &t;
-      least = time;
-    }
-  }
-  return *best;
-}
-
-// An operand shorter than one vector along its contiguous dimension (see
-// TileLoader).
-template <Elem E, bool CX>
-bool is_narrow(const GemmParams &p, bool a_k, bool b_k) {
-  constexpr int CE = CX ? 2 : 1;  // reals per element
-  constexpr int VEC = 16 / (CE * (int)sizeof(typename ElemT<E>::T));
-  return (a_k ? p.K : p.M) / CE < VEC || (b_k ? p.K / CE : p.N) < VEC;
-}
-
 // 64x64 (or, with `t32`, 32x32) tiles, `tiles` of them.
 template <Elem E, typename OutT, bool CX, bool NARROW>
 hcblasStatus_t launch_small(hipStream_t stream, int num_cus, GemmParams p,
@@ -209,7 +131,8 @@ hcblasStatus_t launch_gemm(hipStream_t stream, int num_cus, GemmParams p,
   // Narrow operands are a few rows or a K below one vector: the small tiles do
   // for them, and for 16-bit ones those of 128x128 (8192 x 8192 x 4 HGEMM 42 us,
   // on 64x64 tiles 58; SGEMM 72 on 64x64).
-  if (is_narrow<E, CX>(p, a_k, b_k)) {
+  if (is_narrow(p.M, p.N, p.K, a_k, b_k, CX ? 2 : 1,
+                (int)sizeof(typename ElemT<E>::T))) {
     if constexpr (sizeof(typename ElemT<E>::T) == 2) {
       if (t.bm >= 128)
         return launch_tiles<E, OutT, 128, 128, C::BK_BIG, 2, 4, 32, CX, true>(
@@ -256,7 +179,8 @@ void launch_splitk_tiles(hipStream_t stream, GemmParams p, bool a_k, bool b_k,
   p.tiles_m = (int)cdiv(p.M, T);
   p.tiles_n = (int)cdiv(p.N, T);
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)sk.splits);
-  const bool narrow = is_narrow<E, CX>(p, a_k, b_k);
+  const bool narrow = is_narrow(p.M, p.N, p.K, a_k, b_k, CX ? 2 : 1,
+                                (int)sizeof(typename ElemT<E>::T));
 #define HCB_SPLITK_CASE(AK, BKC)                                           \
   if (a_k == AK && b_k == BKC)                                             \
     (narrow ? gemm_splitk_kernel<E, AK, BKC, T, T, BK, WM, WN, 16, CX, true>   \
