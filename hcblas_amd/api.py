@@ -206,42 +206,45 @@ def _bind(name, proto, fn):
     usual case of each first. Interpreting the prototype on every call (a loop
     of string and type tests, on a callable made anew) took 8-15 us of host
     time, several times a small kernel's launch."""
-    body, call, after = [], [], "return st"
+    body, params, call, after = [], [], [], "return st"
     box_by_type = {"f": "c_float", "d": "c_double"}
+    # (The C arguments take names of their own: the parameters keep the caller's
+    # objects, and with them the memory that is passed, alive during the call.)
     for ctype, p in proto.args:
         base = _base_type(ctype)
+        c = f"c_{p}"
         if p in ("alpha", "beta") and "*" in ctype:
             if base == "void":
-                body.append(f"{p} = scalar_of(dtype, {p})")
+                body.append(f"{c} = scalar_of(dtype, {p})")
             else:
                 kind = _SCALAR_BY_TYPE[base]
-                slow = f"{p} = scalar({kind!r}, {p})"
+                slow = f"scalar({kind!r}, {p})"
                 if kind in box_by_type:
-                    body += [f"if {p}.__class__ is float:",
-                             f"    {p} = byref({box_by_type[kind]}({p}))",
-                             "else:", f"    {slow}"]
-                else:
-                    body.append(slow)
+                    slow = (f"byref({box_by_type[kind]}({p})) "
+                            f"if {p}.__class__ is float else {slow}")
+                body.append(f"{c} = {slow}")
         elif p == "result":
             kind = _SCALAR_BY_TYPE[base]
             body += [f"box = {p} is None and new_box({kind!r}, 0)",
-                     f"{p} = byref(box) if {p} is None else to_c({p})"]
+                     f"{c} = byref(box) if {p} is None else to_c({p})"]
             after = (f"return st if box is False else "
                      f"(st, unbox({kind!r}, box))")
         elif base == "hcblasHandle_t" and "*" not in ctype:
-            body.append(f"{p} = {p}._h if {p}.__class__ is Handle "
+            body.append(f"{c} = {p}._h if {p}.__class__ is Handle "
                         f"else to_c({p})")
-        elif p != "dtype":
-            body += [f"if {p}.__class__ is not int:",
-                     f"    {p} = to_c({p})"]
-        call.append(p)
+        elif p == "dtype":
+            c = p
+        else:
+            body.append(f"{c} = {p} if {p}.__class__ is int else to_c({p})")
+        params.append(p)
+        call.append(c)
     src = "".join(f"    {line}\n" for line in
                   body + [f"st = fn({', '.join(call)})", after])
     scope = {"fn": fn, "Handle": Handle, "to_c": _pass, "scalar": _scalar,
              "scalar_of": _scalar_of, "new_box": _box, "unbox": _unbox,
              "byref": ctypes.byref, "c_float": ctypes.c_float,
              "c_double": ctypes.c_double}
-    exec(f"def {name}({', '.join(call)}):\n{src}", scope)
+    exec(f"def {name}({', '.join(params)}):\n{src}", scope)
     return scope[name]
 
 
