@@ -84,3 +84,41 @@ def test_special_cotangents(torch_cuda):
     ref = _refs(A, B, torch.nan_to_num(W, 0.0, 0.0, 0.0), False, False)[0]
     assert bool(((dA[0, rest] - ref[0, rest]).abs() <=
                  2 * UB * ref[0, rest].abs() + 2.0 ** -130).all())
+
+
+@pytest.mark.parametrize("e", [-112, -124, -128, -131])
+def test_subnormal_cotangents_count(torch_cuda, e):
+    """Cotangents around 2^e under operands large enough for normal gradients. The
+    planes hold a value to within half of BF16's smallest subnormal, 2^-134; beside
+    that only the result's rounding is allowed (2^-8, and 2^-15 for the sums)."""
+    M, N, K = 40, 48, 24
+    g = torch.Generator(device="cuda").manual_seed(1 - e)
+
+    def rand(*s):
+        return torch.rand(*s, generator=g, device="cuda") + 0.5
+
+    A, B = (rand(1, M, K) * 2 ** 20).bfloat16(), (rand(1, K, N) * 2 ** 20).bfloat16()
+    W = (rand(1, M, N).double() * 2.0 ** e).float()
+    dA, dB = (d.double() for d in _adjoints(A, B, W, False, False))
+    w, a, b = W.double(), A.double(), B.double()
+    rA, rB = w @ b.mT.contiguous(), a.mT.contiguous() @ w
+    lost = 2.0 ** -134
+    for d, r, few in ((dA, rA, b.sum(2)[:, None, :]), (dB, rB, a.sum(1)[:, :, None])):
+        bound = (2.0 ** -8 + 2.0 ** -15) * r + lost * few
+        assert bool((bound < 0.5 * r).all())  # a flushed input fails
+        assert bool(((d - r).abs() <= bound).all())
+
+
+def test_special_cotangents_leave_other_columns(torch_cuda):
+    """dB's columns without an Inf or NaN above them, beside those that have one."""
+    M, N, K = 40, 48, 24
+    g = torch.Generator(device="cuda").manual_seed(2)
+    A = (torch.rand(1, M, K, generator=g, device="cuda") + 0.5).bfloat16()
+    B = (torch.rand(1, K, N, generator=g, device="cuda") + 0.5).bfloat16()
+    W = torch.rand(1, M, N, generator=g, device="cuda")
+    W[0, 3, 5], W[0, 7, 9], W[0, 8, 47] = float("inf"), float("nan"), -float("inf")
+    dB = _adjoints(A, B, W, False, False)[1]
+    rest = [n for n in range(N) if n not in (5, 9, 47)]
+    W[0, :, [5, 9, 47]] = 0
+    ref = _refs(A, B, W, False, False)[1]
+    assert bool(((dB - ref)[0][:, rest].abs() <= 2 * UB * ref[0][:, rest]).all())
