@@ -185,3 +185,40 @@ def test_pair_edge_rows_do_not_leak(hc, handle, p):
         exp = np.full(R, Cc, dt)
         exp[R - 2] = np.inf
         assert np.array_equal(to_host(dx), exp), (R, Cc)
+
+
+@pytest.mark.parametrize("p", ["s", "d"])
+@pytest.mark.parametrize("R,Cc", [(1, 1), (3, 17), (5, 16), (7, 33), (23, 46),
+                                  (179, 125), (1022, 31), (1025, 15), (2051, 48)])
+@pytest.mark.parametrize("src", [False, True])
+def test_ger_edge_rows_and_columns(hc, handle, p, R, Cc, src):
+    """Rows that are no whole vector beside columns that are no whole block, in
+    place and into another matrix: each element is one fused operation, and
+    the padding between columns keeps its bits."""
+    dt = np.float32 if p == "s" else np.float64
+    rng = np.random.default_rng(R + Cc)
+    ld, ldd = R + 2, R + 3
+    A = rng.uniform(-1, 1, (Cc, ld)).astype(dt)
+    D = rng.uniform(-1, 1, (Cc, ldd)).astype(dt)
+    x, y = rng.uniform(-1, 1, R).astype(dt), rng.uniform(-1, 1, Cc).astype(dt)
+    dA, dD = to_dev(A), to_dev(D)
+    dx, dy = to_dev(x), to_dev(y)
+    if src:
+        st = getattr(hc.api, f"hcblas_{p}ger_out")(
+            handle, 1, R, Cc, 0.75, dx, 1, dy, 1, dA, ld, dD, ldd)
+        out, pad = to_host(dD), D
+        assert np.array_equal(to_host(dA), A)
+    else:
+        st = getattr(hc.api, f"hcblas_{p}ger")(
+            handle, 1, R, Cc, 0.75, dx, 0, 1, dy, 0, 1, dA, 0, ld)
+        out, pad = to_host(dA), A
+    assert st == 0
+    wide = np.longdouble
+    # alpha * y rounds once, the fused multiply-add once (through an
+    # extended type, at most one more unit)
+    t = (dt(0.75) * y).astype(dt)
+    want = (t.astype(wide)[:, None] * x.astype(wide) + A[:, :R].astype(wide)).astype(dt)
+    assert st == 0
+    eps = np.finfo(dt).eps
+    assert np.all(abs(out[:, :R] - want) <= eps * abs(want))
+    assert np.array_equal(out[:, R:], pad[:, R:])
