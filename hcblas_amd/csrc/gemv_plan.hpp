@@ -49,36 +49,47 @@ inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
   const int64_t steps = plan_cdiv(R, step);
   // Below three quarters of a step a band would leave a whole wave idle.
   const bool band = vec && 4 * R >= 3 * step;
-  // Row-contiguous case of at most 512 columns and 32 MB: sixteen waves per 64
-  // vectors of rows, a wave's columns in at most two trips, one launch. (Each
+  // Row-contiguous case of 129 to 512 columns and at most 32 MB: sixteen waves per
+  // 64 vectors of rows, a wave's columns in at most two trips, one launch. (Each
   // workgroup reads 1 KiB of every column; the split form's second launch
-  // costs more than the CUs that stay idle.)
+  // costs more than the CUs that stay idle. Up to 128 columns four waves do: 3.6
+  // us in the mean against 4.0.)
   const int64_t pblocks = plan_cdiv(R, 64 * (int64_t)(vec ? vn : 1));
-  const bool short_sums = panel && Cc > 32 && Cc <= 512 &&
+  const bool short_sums = panel && Cc > 128 && Cc <= 512 &&
                           pblocks * batch < 2 * (int64_t)num_cus &&
                           R * Cc * (int64_t)esize * batch <= (32ll << 20);
   // Column case. A band of up to 16 steps, all bands alike (R = 20011, 20
   // steps: two bands of 10 instead of 16 and 4), and more, shorter bands
   // where the column blocks are few: up to one workgroup per CU, bands of at
-  // least 2 steps.
+  // least 2 steps, from 5 steps on (below, the second launch costs more than they
+  // save: 3 steps 5.5 us in one band, 6.8 in two).
+  // Up to 128 MB the column kernel is ahead where a band's lanes idle: more than a
+  // quarter of them (0.86 to 0.9 of the band's time, 1 to 3 steps; with few idle
+  // ones up to 1.1), and of rows that are whole vectors up to 1.8 steps (0.86 to
+  // 0.93; above 1.0). Larger matrices stream faster in bands at any row count
+  // (1024 x 100000 fp32 61 us, 77).
+  const bool columns = R * Cc * (int64_t)esize * batch < (128ll << 20) &&
+                       (4 * R < 3 * steps * step ||
+                        (R % vn == 0 && 5 * R < 9 * step));
   int64_t bands = plan_cdiv(steps, 16);
-  if (!panel && band && split) {
+  if (split && steps >= 5) {
     const int64_t blocks = plan_cdiv(Cc, kBandCols) * batch;
     bands = std::max(bands,
                      std::min((int64_t)num_cus / blocks, (steps + 1) / 2));
   }
-  if (!panel && band && bands <= (split ? 65535 : 1)) {
+  if (!panel && band && !columns && bands <= (split ? 65535 : 1)) {
     int64_t xr = plan_cdiv(steps, bands);
     if (xr > 4) xr = (xr + 1) / 2 * 2;  // instances: 1..4, 6, 8, .. 16
     p.kernel = xr == 16 ? GemvKernel::kBand16 : GemvKernel::kBand8;
     p.xr = (int)xr;
     p.oblocks = plan_cdiv(Cc, kBandCols);
     p.splits = (int)plan_cdiv(steps, xr);
-  } else if (panel && band && !short_sums && Cc >= 64 && steps <= 65535) {
-    // Row-contiguous case: bands of 4 steps (16 KiB of each column in one
-    // run) where they waste at most an eighth of their lanes and, with at
-    // least 64 columns per block, still give every CU a workgroup; else 2
-    // or 1. Column blocks: about one workgroup per CU (at 16384^2 fp32 256
+  } else if (panel && band && Cc > 512 && steps <= 65535) {
+    // Row-contiguous case (up to 512 columns the panel kernel is as fast or
+    // faster: 1024 x 225 fp64 in a batch of 43 13.7 us, here 20.1): bands of 4
+    // steps (16 KiB of each column in one run) where they waste at most an
+    // eighth of their lanes and, with at least 64 columns per block, still give
+    // every CU a workgroup; else 2 or 1. Column blocks: about one workgroup per CU (at 16384^2 fp32 256
     // workgroups took 152 us, 128 178 us, 512 159 us), at least 32 columns.
     // (4096^2 fp32 used one band of 4 steps in 16 blocks: 16 workgroups,
     // 75 us.)
@@ -99,13 +110,14 @@ inline GemvPlan plan_gemv(int num_cus, bool panel, int64_t R, int64_t Cc,
   } else if (panel) {
     p.kernel = GemvKernel::kPanel;
     p.oblocks = pblocks;
-    // Otherwise splits of at least 8 columns for each of four waves.
+    // Otherwise, above 128 columns, splits of at least 8 columns for each of
+    // four waves, or of 32 where the row blocks give every CU a workgroup.
     if (short_sums)
       p.waves = 16;
-    else
+    else if (Cc > 128)
       p.splits = (int)std::min<int64_t>(
           plan_cdiv(target, p.oblocks * batch),
-          std::min<int64_t>(256, std::max<int64_t>(1, Cc / 32)));
+          std::min<int64_t>(256, Cc / (p.oblocks * batch < num_cus ? 32 : 128)));
   } else {
     p.kernel = GemvKernel::kColumn;
     p.oblocks = plan_cdiv(Cc, kColsPerBlock);

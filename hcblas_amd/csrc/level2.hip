@@ -424,25 +424,28 @@ __global__ __launch_bounds__(kThreads) void gemv_column_kernel(
       // belong to another lane and count as zeros here.
       const int64_t rr = r + VN <= s.R ? r : s.R - VN;
       T xv[VN];
+      V a[kCPW];
 #pragma unroll
-      for (int e = 0; e < VN; ++e)
-        xv[e] = rr + e >= r ? x[bidx(rr + e, s.R, s.incx)] : T(0);
+      for (int j = 0; j < kCPW; ++j) a[j] = vld<NT>(cols[j] + rr);
 #pragma unroll
-      for (int j = 0; j < kCPW; ++j) {
-        if (!colok[j]) continue;
-        const V a = vld<NT>(cols[j] + rr);
+      for (int e = 0; e < VN; ++e) xv[e] = x[bidx(rr + e, s.R, s.incx)];
+#pragma unroll
+      for (int e = 0; e < VN; ++e) xv[e] = rr + e >= r ? xv[e] : T(0);
+#pragma unroll
+      for (int j = 0; j < kCPW; ++j)
 #pragma unroll
         for (int e = 0; e < VN; ++e)
-          acc[j][e] = fma_t(rr + e >= r ? vlane<T>(a, e) : T(0), xv[e],
+          acc[j][e] = fma_t(rr + e >= r ? vlane<T>(a[j], e) : T(0), xv[e],
                             acc[j][e]);
-      }
     }
   } else {
     for (int64_t r = r_begin + lane_id; r < r_end; r += step) {
-      T xv = x[bidx(r, s.R, s.incx)];
+      const T xv = x[bidx(r, s.R, s.incx)];
+      T a[kCPW];
 #pragma unroll
-      for (int j = 0; j < kCPW; ++j)
-        if (colok[j]) acc[j][0] = fma_t(cols[j][r], xv, acc[j][0]);
+      for (int j = 0; j < kCPW; ++j) a[j] = cols[j][r];
+#pragma unroll
+      for (int j = 0; j < kCPW; ++j) acc[j][0] = fma_t(a[j], xv, acc[j][0]);
     }
   }
 
@@ -854,8 +857,10 @@ hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
     return launch_status();
   }
   constexpr int VN = VecT<T>::n;
-  // Rows are read 16 bytes at a time unless there is not even one vector.
-  bool vec = R >= VN;
+  // Rows are read 16 bytes at a time unless there is not even one vector, or, in
+  // the column kernel, one element for each lane of a wave reaches them all
+  // (SGEMV-T 37 x 576 3.9 us by vectors, 3.0).
+  bool vec = panel ? R >= VN : R > 64;
   const bool nt = (int64_t)sizeof(T) * R * Cc * batch >= kStreamBytes;
   GemvShape s{R, Cc, ld, incx, incy, sA, sx, sy, 1};
   GemvPlan plan =
