@@ -1044,11 +1044,30 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
       }
     }
     __syncthreads();
-    // Two loops, one for tiles with moved rows: there a moved vector is read
+    // BOTH: two loops, one for tiles with moved rows, where a moved vector is read
     // from LDS by elements and stored whole (BF16 156 x 128x92x28 8.7 -> 6.3 us).
-    // Without BOTH, one loop in which moved rows also leave one by one, for a
-    // kernel of many tile bodies, whose code size counts.
-    auto columns = [&](auto moved) {
+    // Without it one loop, in which moved rows leave one by one, for kernels of
+    // many tile bodies (4096^3 among the grouped problems 371 -> 374 us in two
+    // loops) or with no registers to spare (the adjoints, whose 256 x 256 tile
+    // with an FP32 A spills one in two: 177 BF16 backward products of 31 x 214 x
+    // 931 87 -> 99 us, one of 79 x 31 x 128 11.9 -> 12.6).
+    const auto whole = [&](OutT *dst, const Acc *src) {
+      OutT cin[VE], o[VE];
+      if (beta != Acc(0)) {
+        const vec4u w = *reinterpret_cast<const GV *>(dst);
+        __builtin_memcpy(cin, &w, 16);
+      }
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+        Acc v = alpha * src[e];
+        if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(cin[e]), v);
+        o[e] = to_out<OutT>(v);
+      }
+      vec4u w;
+      __builtin_memcpy(&w, o, 16);
+      *reinterpret_cast<GV *>(dst) = w;
+    };
+    const auto columns = [&](auto moved) {
 #pragma unroll
       for (int cc = 0; cc < NC; cc += NTH / TPC) {
         const int nl = cc + tid / TPC;
@@ -1058,23 +1077,8 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
           OutT *dst = C + (int64_t)n * ldc + m;
           const Acc *src = t + (n < edge_n ? nl : nl + shift_n) * LROW + ml;
           const bool below = !decltype(moved)::value || m < edge_m;
-          const int up = below || !BOTH ? 0 : shift_m;
-          if (m + VE <= (decltype(moved)::value && (below || !BOTH) ? edge_m
-                                                                    : M)) {
-            OutT cin[VE], o[VE];
-            if (beta != Acc(0)) {
-              const vec4u w = *reinterpret_cast<const GV *>(dst);
-              __builtin_memcpy(cin, &w, 16);
-            }
-#pragma unroll
-            for (int e = 0; e < VE; ++e) {
-              Acc v = alpha * src[e + up];
-              if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(cin[e]), v);
-              o[e] = to_out<OutT>(v);
-            }
-            vec4u w;
-            __builtin_memcpy(&w, o, 16);
-            *reinterpret_cast<GV *>(dst) = w;
+          if (m + VE <= (decltype(moved)::value && below ? edge_m : M)) {
+            whole(dst, below ? src : src + shift_m);
           } else {
             const int ne = M - m < VE ? M - m : VE;
 #pragma unroll 1
@@ -1089,10 +1093,33 @@ __device__ __forceinline__ void store_tile_lds(const AccArr &acc, OutT *C,
         }
       }
     };
-    if (BOTH && (shift_m == 0 || m0 + BM <= edge_m))
-      columns(std::false_type{});
-    else
-      columns(std::true_type{});
+    if constexpr (BOTH) {
+      if (shift_m == 0 || m0 + BM <= edge_m)
+        columns(std::false_type{});
+      else
+        columns(std::true_type{});
+    } else {
+#pragma unroll
+      for (int cc = 0; cc < NC; cc += NTH / TPC) {
+        const int nl = cc + tid / TPC;
+        const int ml = (tid % TPC) * VE;
+        const int n = n0 + c0 + nl, m = m0 + ml;
+        if (nl < NC && n < N && m < M) {
+          OutT *dst = C + (int64_t)n * ldc + m;
+          const Acc *src = t + (n < edge_n ? nl : nl + shift_n) * LROW + ml;
+          if (m + VE <= edge_m) {
+            whole(dst, src);
+          } else {
+            const int ne = M - m < VE ? M - m : VE;
+            for (int e = 0; e < ne; ++e) {
+              Acc v = alpha * src[m + e < edge_m ? e : e + shift_m];
+              if (beta != Acc(0)) v = fma_acc(beta, from_out<Acc>(dst[e]), v);
+              dst[e] = to_out<OutT>(v);
+            }
+          }
+        }
+      }
+    }
     __syncthreads();
   }
 }

@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mixed_kernel(
       __syncthreads();
     }
   }
-  store_tile_lds<Elem::BF16, Bf16Out, BM, BN, WM, WN, MI, LDS>(
+  store_tile_lds<Elem::BF16, Bf16Out, BM, BN, WM, WN, MI, LDS, false>(
       acc, C, p.ldc, p.M, p.N, m0, n0, (double)p.alpha, 0.0, threadIdx.x, lds,
       LA::edge_row(p.M), LA::edge_shift(p.M), LB::edge_row(p.N),
       LB::edge_shift(p.N));
