@@ -22,8 +22,11 @@
 // Each tile runs the plain GEMM's main loop with the same K step and an
 // epilogue with the same arithmetic (staged through LDS so that C is written
 // with 16-byte column runs), so a grouped result is bit-identical to
-// per-problem hcblas_sgemm / hcblas_hgemm launches (of K < 2048: beyond, those
-// may split K, which the grouped kernel never does).
+// per-problem hcblas_sgemm / hcblas_hgemm launches for problems that those run on
+// 16x16 MFMA blocks without splitting K. The grouped kernel never splits K and
+// uses 16x16 blocks throughout; the plain launcher may split K from 2048 on and
+// takes 32x32 blocks, which add the same products in another order, on its 256x256
+// tiles and its 16-bit 128x128 ones.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -62,8 +65,8 @@ struct GroupCfg {
           : tile_lds_bytes<Elem::F16, TM, TM, kF16BK>();
 };
 
-// One tile: the plain kernels' main loop (same K step, so the sums are
-// bit-identical to per-problem launches), then the LDS-staged epilogue.
+// One tile: the plain kernels' main loop (same K step, so the sums are those of
+// per-problem launches on 16x16 MFMA blocks), then the LDS-staged epilogue.
 template <Elem E, typename OutT, int TM, bool NARROW, bool A_K, bool B_K>
 __device__ __forceinline__ void tile_body(const ProbDev &p, int m0, int n0,
                                           int tid, char *lds) {

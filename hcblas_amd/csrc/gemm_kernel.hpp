@@ -726,7 +726,9 @@ struct WaveTile {
 // Main loop of one BM x BN tile at (m0, n0): acc = A'(m0.., :) * B'(:, n0..)
 // over the whole K range. Shared by the plain / batched kernel, the grouped
 // kernel and the residue kernel, so all of them produce bit-identical sums
-// for the same K step. CX: a complex product's operands (cx).
+// on MFMA blocks of the same size MI (a block's lane groups hold different k of a
+// chunk, so 16x16 and 32x32 blocks add in another order, and a size's last bits can
+// change with its tile). CX: a complex product's operands (cx).
 template <Elem E, bool A_K, bool B_K, int BM, int BN, int BK, int WM, int WN,
           int MI, bool NARROW, bool CX>
 __device__ __forceinline__ void gemm_mainloop(
@@ -972,7 +974,7 @@ __device__ __forceinline__ void gemm_mainloop(
 // the main loop's LDS holds), and each thread then blends and stores VE
 // consecutive rows of one column with one 16-byte access, a column's BM rows
 // by BM / VE consecutive lanes. The arithmetic is the direct form's
-// (alpha * acc, then fma(beta, C, .)), so results are bit-identical.
+// (alpha * acc, then fma(beta, C, .)), so results are bit-identical to it.
 // Accumulator layouts (value r of lane l, block row / column):
 //   32x32 FP32/INT32: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32;
 //   16x16 FP32: row 4 (l / 16) + r, column l % 16;

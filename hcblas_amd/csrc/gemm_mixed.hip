@@ -18,12 +18,13 @@
 // with the plain kernels' arithmetic; the result is rounded once to BF16.
 //
 // What bounds it: the MFMAs, and beside them the split's VALU work on the same
-// SIMDs and the LDS. (256 x 256x1024x512: with the planes' writes two to a bank,
-// 43-58% of the LDS cycles were conflicts, and with integer rounding in the
-// epilogue, 8 operations per output, the MFMAs were busy 52% of dA and 33% of
-// dB; dA 223 -> 204 us, dB 293 -> 246 without either.) v_cvt_pk_bf16_f32 rounds
-// two values at once, about 8 operations per element where integer rounding
-// took 18. An operand stored with the inner index as its row index (both
+// SIMDs, the LDS, and the prologue and epilogue of a tile that fills a CU.
+// (Counters of 256 x 256x1024x512: MFMAs busy 53% of dA, 189 us, and 38% of dB, 268
+// us of 8 K steps a tile; 43-46% of wave time in s_waitcnt; 11-14% of the LDS
+// cycles are conflicts. With the planes' writes two to a bank and integer
+// rounding in the epilogue, 8 operations per output, dA took 223 us where it then
+// took 204, dB 293 and 246.) v_cvt_pk_bf16_f32 rounds two values at once, about 8
+// operations per element where integer rounding took 18. An operand stored with the inner index as its row index (both
 // operands of dB = op(A)^T dC) is transposed in registers by the tile loader: a
 // thread holds a 4 x 4 block of FP32 or two k-lines of 8 BF16 rows and writes
 // along k, as many LDS writes as the k-contiguous form. (Transposed copies of dC

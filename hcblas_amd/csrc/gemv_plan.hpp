@@ -16,6 +16,7 @@ constexpr int kCPW = 4;           // columns per wave of the column kernel
 constexpr int kColsPerBlock = 4 * kCPW;
 constexpr int kBandCols = 8;      // columns per workgroup of the band kernel
 
+// kBand16: the band kernel with 16 row steps; kBand8: with 1 to 14.
 enum class GemvKernel { kBandN, kPanel, kBand16, kBand8, kColumn };
 
 struct GemvPlan {

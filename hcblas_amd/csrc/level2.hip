@@ -865,8 +865,9 @@ hcblasStatus_t run_gemv(hcblasHandle_t h, bool panel, int64_t R, int64_t Cc,
   GemvShape s{R, Cc, ld, incx, incy, sA, sx, sy, 1};
   GemvPlan plan =
       plan_gemv(h->num_cus, panel, R, Cc, vec, VN, sizeof(T), batch);
-  // Bands of a matrix of more than about 80 GB can need more partials than
-  // the allocation-free entry's scratch holds. Where the operands are not
+  // Bands of a column-contiguous matrix can need more partials than the
+  // allocation-free entry's scratch holds from about 68 GB on (FP64 8193 x
+  // 1048577: 16 bytes more; FP32 from twice that). Where the operands are not
   // 16-byte aligned both entries then read by elements, whose splits fit.
   if (batch == 1 && plan.partial_bytes > kNoAllocScratchBytes &&
       (!aligned16(A) || ld % VN || R % VN ||

@@ -36,10 +36,8 @@ void check(hcblasStatus_t st, const char *what) {
               static_cast<int>(st));
 }
 
-// One handle per (thread, device, stream): a handle's workspaces (split-K
-// partials, the transposed operand copies of a BF16 backward) are used by the
-// work it enqueues, so two streams never share one handle, and work on one
-// stream cannot overwrite a workspace that another stream is still reading.
+// One handle per (thread, device, stream): a handle is not thread-safe, and the
+// work that it enqueues uses its device memory, so two streams never share one.
 struct StreamKey {
   int device;
   hipStream_t stream;

@@ -151,7 +151,11 @@ hcblasStatus_t hcblasDestroy(hcblasHandle_t *handle);
 
 /* Selects the stream for all later calls; NULL is the default stream.
  * Replaces hcblasSetAcclView (hcblas.h:140, hcblas.cpp:95-103) with the
- * hipblasSetStream semantics of lib/src/hcc_detail/hipblas.cpp:51-62. */
+ * hipblasSetStream semantics of lib/src/hcc_detail/hipblas.cpp:51-62.
+ *   Work enqueued before the change may still run: the partial sums of split
+ * reductions (GEMM, GEMV, the adjoint of GER) are kept per stream. The workspace
+ * of the split-precision modes is not: between two calls in those modes on
+ * different streams the caller orders the streams, or uses a handle for each. */
 hcblasStatus_t hcblasSetStream(hcblasHandle_t handle, hipStream_t stream);
 
 /* Returns the stream set on the handle. Replaces hcblasGetAcclView
